@@ -83,6 +83,11 @@ int32_t launch_prefill_plan(const AttnArgs& args, void* workspace, hipStream_t s
 int32_t launch_prefill_mfma_planned(AttnArgs args, int32_t dtype, void* workspace,
                                     bool plan_ready, hipStream_t stream);
 
+// float32 MFMA varlen kernel (paged_prefill_f32.hip): float32 with head_dim
+// 128, contiguous K/V or a block size of at least 16.
+bool prefill_f32_supported(const AttnArgs& args, int32_t dtype);
+int32_t launch_prefill_f32(const AttnArgs& args, hipStream_t stream);
+
 // MFMA decode kernel (paged_decode_mfma.hip): 16-bit caches, head_dim 128,
 // up to 16 query heads per KV head, block size >= 16, paged.
 bool decode_mfma_supported(const AttnArgs& args, int32_t dtype);
