@@ -28,10 +28,9 @@
 //    scores have used the registers: each half hides the other's loads.
 //
 // Chunks of 118 / 325 / 210 rows on contexts of 155 / 325 / 359 (16 / 8
-// heads), graph-replayed: 27.6 us a launch, 76.3 on the vector kernel; 1000
-// rows on 1700 keys: 131.7 us, 74.7 TFLOP/s. Error against 64 bits 1.8e-7
-// (1.4e-7): each wave sums a quarter of the keys in one chain, where the
-// vector kernel had sixteen.
+// heads), graph-replayed: 27.5 us a launch, 76.3 on the vector kernel; 1000
+// rows on 1700 keys: 127 us, 77 TFLOP/s. Error against 64 bits 1.5e-7, as
+// the vector kernel's (1.4e-7), through short summation chains.
 #include "paged_attention.h"
 
 namespace mi {
@@ -180,27 +179,34 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
     }
     // The compiler would sink these loads below the products that hide them.
     __builtin_amdgcn_sched_barrier(0);
-    f32x4_t s[4];  // four sums: shorter chains, added as a tree
+    // Eight chains of 16 terms, added as a tree: a score's rounding error is
+    // that of short sums (one chain of 128 had 1.6 times the error).
+    f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < 2; ++h) {
+      f32x4_t c[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+      for (int e = 0; e < 4; ++e) c[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        s[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[j][e], s[e], 0, 0, 0);
+      for (int j = 4 * h; j < 4 * h + 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          c[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[j][e], c[e], 0, 0, 0);
+      s += (c[0] + c[1]) + (c[2] + c[3]);
+    }
     // Unconditional (the last round repeats the last tile): the waits below
     // then count these loads as in flight on every path.
     bool next_ok;
     const int64_t next_base = tile_base(next, next_blk, next_ok);
     load_k(kf, next, next_base);
     __builtin_amdgcn_sched_barrier(0);
-    // s[.][i]: key p0 + 4 quad + i, query row `col`.
+    // s[i]: key p0 + 4 quad + i, query row `col`.
     const bool masked = !ok || p0 + kRows > keys_all;  // uniform
     const int lim = masked ? (ok ? limit : 0) : INT32_MAX;
     float sc[4], tmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float v = ((s[0][i] + s[1][i]) + (s[2][i] + s[3][i])) * a.scale_log2;
+      const float v = s[i] * a.scale_log2;
       sc[i] = p0 + 4 * quad + i < lim ? v : -INFINITY;
       tmax = fmaxf(tmax, sc[i]);
     }
@@ -243,14 +249,20 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
         break;
       }
     }
+    // The tile's own sums, then added to the running ones (short chains again).
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 2; ++j) {
+      f32x4_t c[4];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int e = 0; e < 4; ++e) c[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          o[4 * j + e] =
-              __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j][e], pr[i], o[4 * j + e], 0, 0, 0);
+          c[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j][e], pr[i], c[e], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[4 * j + e] += c[e];
+    }
     ok = next_ok;
     base = next_base;
   }
