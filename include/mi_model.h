@@ -30,8 +30,8 @@ extern "C" {
 /*
  * y[m, n] = sum_k x[m, k] * w[n, k] (torch's F.linear without bias), float32
  * accumulation, one rounding to the element type. For m <= 64 (decode
- * batches): each weight row streams through MFMA once; a workgroup's waves
- * split k and add their sums in a fixed order (deterministic).
+ * batches): a workgroup's waves split k and add their sums in a fixed order
+ * (deterministic); one or two rows take a vector kernel, more MFMA.
  * n % 16 == 0, k % 32 == 0, every pointer and row stride 16-byte aligned.
  * m > 64 returns MI_ERR_UNSUPPORTED.
  */
@@ -52,6 +52,25 @@ int32_t mi_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_
 int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
                          int64_t w_row_stride, void* y, int64_t y_row_stride, int32_t m,
                          int32_t inter, int32_t k, int32_t dtype, void* stream);
+
+/*
+ * A projection with what surrounds it in a decoder layer, one launch:
+ *   s = norm_weight ? rms_norm(x) : x
+ *   y = residual + s . w^T            (swiglu = 0; w holds n rows)
+ *   y = silu(gate) * up               (swiglu = 1; w holds n = 2 inter rows,
+ *                                      gate's then up's, y is [m, inter])
+ * The norm (FuseLayerNorm, microinfer/layer/norm.py:26-35, on a sum already
+ * made) is applied as (1 / rms) * ((x * norm_weight rounded once) . w^T), so
+ * it differs from mi_rms_norm_residual + mi_linear by that pair's second
+ * rounding. The projection's sum is rounded to the element type before the
+ * residual is added and the result rounded again, as x + F.linear(...) does;
+ * residual may be NULL and may be y itself. norm_weight may be NULL. Shapes,
+ * alignment and limits are those of mi_linear / mi_linear_swiglu.
+ */
+int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
+                        const void* w, int64_t w_row_stride, const void* residual,
+                        int64_t residual_row_stride, void* y, int64_t y_row_stride, int32_t m,
+                        int32_t n, int32_t k, int32_t swiglu, int32_t dtype, void* stream);
 
 /*
  * FuseLayerNorm's forward (microinfer/layer/norm.py:26-35) on `rows` rows:

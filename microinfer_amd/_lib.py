@@ -91,6 +91,9 @@ SIGNATURES = {
     ),
     "mi_linear": (_I32, [_P, _I64, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _P]),
     "mi_linear_swiglu": (_I32, [_P, _I64, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _P]),
+    "mi_linear_fused": (
+        _I32,
+        [_P, _I64, _P, _F32, _P, _I64, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P]),
     "mi_rms_norm_residual": (
         _I32, [_P, _I64, _P, _I64, _P, _F32, _P, _I64, _P, _I64, _I32, _I32, _I32, _P]),
     "mi_silu_mul": (_I32, [_P, _I64, _P, _I64, _I32, _I32, _I32, _P]),

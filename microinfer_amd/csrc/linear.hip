@@ -1,0 +1,605 @@
+// Dense projections of the decoder layer at decode batch sizes on gfx950:
+// y = x . w^T for m <= 64 rows, with the layer's RMSNorm in front of it, the
+// SwiGLU gate or the residual sum behind it (entry points in
+// include/mi_model.h).
+//
+// What bounds them: w streams once from memory (8.4 MB for a 4096 x 1024
+// projection: 1.7 us at the measured copy rate of 4.9 TB/s), but a launch of
+// that size is mostly latency -- the launch itself, one memory round trip,
+// the sum over the waves -- so the kernels keep everything a wave needs in
+// flight at once, and a step's norm, gate and residual sum ride on the
+// projections instead of being launches of their own (3.1-3.6 us each).
+//
+// Two kernels:
+//  * linear_kernel (MFMA): a workgroup owns 16 or 32 columns and every row;
+//    its waves split k. A operand: 16 weight rows as stored; B operand: 16
+//    rows of x. All waves then add the partial sums, wave by wave in order,
+//    each wave a share of the tiles.
+//  * gemv_kernel (m <= 4): a wave owns whole weight rows, a lane 8 elements
+//    of every 512, so a load instruction takes 1 KiB of one row; narrow
+//    outputs (1024 columns) then still give all CUs work, where 16-column
+//    tiles leave three quarters of them idle.
+//
+// RMSNorm in front: y[m] = (1 / rms(x[m])) * (x[m] * weight) . w^T. The
+// product x * weight is rounded once to the element type (torch's norm rounds
+// twice), 1 / rms scales the float32 sum.
+#include "mi_common.h"
+#include "mi_model.h"
+
+namespace mi {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <typename E>
+struct LinMfma;
+template <>
+struct LinMfma<BF16> {
+  using vec8 = bf16x8_t;
+  using el = __bf16;
+  static __device__ __forceinline__ f32x4_t mma(vec8 a, vec8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct LinMfma<F16> {
+  using vec8 = f16x8_t;
+  using el = _Float16;
+  static __device__ __forceinline__ f32x4_t mma(vec8 a, vec8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+constexpr int kLinMaxRows = 64;
+constexpr int kLinStep = 32;  // k per MFMA
+
+struct LinArgs {
+  const void* x;
+  int64_t xs;
+  const void* w;
+  int64_t ws;
+  void* y;
+  int64_t ys;
+  int32_t m, n, k;
+  int32_t row_groups; // MFMA launches: groups of 16 MT rows
+  int32_t inter;      // GLU: rows [0, inter) of w are the gate, the rest up
+  const void* norm;   // RMSNorm weight of x (null: x as it is)
+  float eps;
+  const void* res;    // added to y (null: none)
+  int64_t rs;
+};
+
+// x[i] * w[i] over an 8-element fragment, rounded once.
+template <typename E>
+__device__ __forceinline__ Pack<uint16_t, 8> scale8(const Pack<uint16_t, 8>& x,
+                                                    const Pack<uint16_t, 8>& w) {
+  Pack<uint16_t, 8> r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    r.v[i] = __builtin_bit_cast(
+        uint16_t, static_cast<typename LinMfma<E>::el>(E::load(x.v[i]) * E::load(w.v[i])));
+  return r;
+}
+
+// acc + sum of x[i] * w[i] over the fragment.
+template <typename E>
+__device__ __forceinline__ float dot8(const Pack<uint16_t, 8>& x, const Pack<uint16_t, 8>& w,
+                                      float acc) {
+  const Pack<uint32_t, 4> a = __builtin_bit_cast(Pack<uint32_t, 4>, x);
+  const Pack<uint32_t, 4> b = __builtin_bit_cast(Pack<uint32_t, 4>, w);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = E::dot2(a.v[i], b.v[i], acc);
+  return acc;
+}
+
+// The residual sum of one element, rounded as a separate launch rounds it.
+template <typename E>
+__device__ __forceinline__ uint16_t add_residual(uint16_t y, uint16_t res) {
+  return E::store(E::load(y) + E::load(res));
+}
+
+// ---------------------------------------------------------------------------
+// MFMA kernel.
+// ---------------------------------------------------------------------------
+constexpr int kChunk = 128;  // k per staged chunk (four MFMA steps)
+constexpr int kChunkSteps = kChunk / kLinStep;
+constexpr int kRowBytes = kChunk * 2;    // one row of a chunk: 256 bytes
+constexpr int kTileBytes = 16 * kRowBytes;
+
+// NW waves split k by chunks (wave w: a contiguous range); NT 16-column tiles
+// per workgroup (GLU: tile 0 is gate columns, tile 1 the matching up columns);
+// MT 16-row tiles of x per workgroup, row groups of one column tile on one XCD.
+// S LDS slots of one chunk per wave.
+//
+// A wave stages its chunks of w and x in its own LDS slots with direct
+// global->LDS loads, four rows of 256 bytes per instruction, and reads the
+// MFMA fragments from there. Loading the fragments straight into registers
+// puts 16 different rows in 16 neighbouring lanes, and the address unit then
+// takes about 64 cycles per instruction instead of 16: at 64 rows that alone
+// was 4.1 of the 7.1 us of a 4096 x 1024 projection.
+// LDS rows are 256 bytes; 16-byte piece c of row r sits at place c ^ (r & 15),
+// which makes the fragment reads free of bank conflicts.
+template <typename E, int NW, int NT, int MT, int S, bool GLU, bool NORM>
+__global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
+  using M = LinMfma<E>;
+  using vec8 = typename M::vec8;
+  using R = uint16_t;
+  static_assert(!GLU || NT == 2, "GLU launches: gate and up tiles");
+  constexpr int kUnits = GLU ? MT : NT * MT;  // result tiles to add up and store
+  constexpr int kSlot = (NT + MT) * kTileBytes;
+  constexpr int kSums = NW * NT * MT * kWave * 16;
+  constexpr int kRing = NW * S * kSlot;
+  // The ring, then (after every wave has read its last chunk) the sums.
+  __shared__ __attribute__((aligned(16))) char s_mem[kRing > kSums ? kRing : kSums];
+  __shared__ float s_ss[NORM ? NW : 1][MT * 16];
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int col = lane % 16;   // weight row (output column) / x row within a tile
+  const int quad = lane / 16;  // 8-element group of the k-step
+  const int xcd = blockIdx.x % 8, rest = blockIdx.x / 8;
+  const int r0 = 16 * MT * (rest % a.row_groups);
+  const int n0 = (rest / a.row_groups * 8 + xcd) * (GLU ? 16 : 16 * NT);
+  if (n0 >= (GLU ? a.inter : a.n)) return;
+  const int chunks = (a.k + kChunk - 1) / kChunk;
+  const int per_wave = (chunks + NW - 1) / NW;
+  const int c_begin = min(wave * per_wave, chunks);
+  const int c_end = min(c_begin + per_wave, chunks);
+
+  f32x4_t acc[NT][MT];
+  float ss[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    ss[t] = 0.f;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) acc[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // Load i of a tile takes its rows 4 i .. 4 i + 3; lane / 16 is the row of
+  // them, lane % 16 the place in it. n % 16 == 0: a tile's columns exist or
+  // none do (then tile 0 is read in its place). Rows of x past m repeat the
+  // last one; their results are not stored.
+  const R* src[(NT + MT) * 4];
+  int piece[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 4 * i + quad;
+    piece[i] = (col ^ row) * 8;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int wr = GLU ? u * a.inter + n0 : (n0 + 16 * u < a.n ? n0 + 16 * u : n0);
+      src[u * 4 + i] = static_cast<const R*>(a.w) + static_cast<int64_t>(wr + row) * a.ws;
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+      src[(NT + t) * 4 + i] = static_cast<const R*>(a.x) +
+                              static_cast<int64_t>(min(r0 + 16 * t + row, a.m - 1)) * a.xs;
+  }
+  char* ring = s_mem + wave * S * kSlot;
+  auto issue = [&](int slot, int c) {
+    char* dst = ring + slot * kSlot;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // A last chunk may end early: pieces past the row read its start.
+      int off = c * kChunk + piece[i];
+      off = off < a.k ? off : 0;
+#pragma unroll
+      for (int t = 0; t < NT + MT; ++t)
+        lds_load16(src[t * 4 + i] + off, dst + t * kTileBytes + i * 4 * kRowBytes);
+    }
+  };
+  auto fragment = [&](const char* tile, int step) {
+    return *reinterpret_cast<const Pack<R, 8>*>(tile + col * kRowBytes +
+                                                (((4 * step + quad) ^ col) * 16));
+  };
+  const R* nrow = static_cast<const R*>(a.norm) + quad * 8;
+  if (c_begin < c_end) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (c_begin + s < c_end) issue(s, c_begin + s);
+    for (int c = c_begin, slot = 0; c < c_end; ++c, slot = slot + 1 == S ? 0 : slot + 1) {
+      Pack<R, 8> g[NORM ? kChunkSteps : 1];
+      if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < kChunkSteps; ++j) {
+          const int off = c * kChunk + j * kLinStep;
+          g[j] = load_pack<R, 8>(nrow + (off < a.k ? off : 0));
+        }
+      }
+      // Chunk c is in its slot once at most the younger one is in flight
+      // (and the norm weights, which were issued last).
+      if (!NORM && S > 1 && c + 1 < c_end)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (4 * (NT + MT) & 15) | ((4 * (NT + MT) >> 4) << 14));
+      else
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      const char* cur = ring + slot * kSlot;
+      const int steps = min(kChunkSteps, (a.k - c * kChunk) / kLinStep);
+#pragma unroll
+      for (int j = 0; j < kChunkSteps; ++j) {
+        if (j >= steps) break;  // uniform
+        vec8 wf[NT];
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+          wf[u] = __builtin_bit_cast(vec8, fragment(cur + u * kTileBytes, j));
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          Pack<R, 8> x = fragment(cur + (NT + t) * kTileBytes, j);
+          if constexpr (NORM) {
+            ss[t] = dot8<E>(x, x, ss[t]);
+            x = scale8<E>(x, g[j]);
+          }
+#pragma unroll
+          for (int u = 0; u < NT; ++u)
+            acc[u][t] = M::mma(wf[u], __builtin_bit_cast(vec8, x), acc[u][t]);
+        }
+      }
+      if (c + S < c_end) {
+        // The fragment reads of this slot have returned.
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        issue(slot, c + S);
+      }
+    }
+  }
+  __syncthreads();  // the ring is free
+
+  // acc[u][t][j] = y^T[n0 + 16 u + 4 quad + j][r0 + 16 t + col], this wave's k.
+  f32x4_t* sums = reinterpret_cast<f32x4_t*>(s_mem);
+  auto sum_at = [&](int w, int tile) -> f32x4_t& {
+    return sums[(w * NT * MT + tile) * kWave + lane];
+  };
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) sum_at(wave, u * MT + t) = acc[u][t];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const float v = xor_sum<16, kWave>(ss[t]);
+      if (lane < 16) s_ss[wave][16 * t + lane] = v;
+    }
+  }
+  __syncthreads();
+  R* y = static_cast<R*>(a.y);
+#pragma unroll
+  for (int i = 0; i < (kUnits + NW - 1) / NW; ++i) {
+    const int unit = wave + i * NW;
+    if (unit >= kUnits) break;
+    const int t = unit % MT, u = unit / MT;  // GLU: u = 0
+    f32x4_t v = sum_at(0, unit), up = {};
+    if constexpr (GLU) up = sum_at(0, MT + unit);
+#pragma unroll
+    for (int wv = 1; wv < NW; ++wv) {
+      v += sum_at(wv, unit);
+      if constexpr (GLU) up += sum_at(wv, MT + unit);
+    }
+    if constexpr (NORM) {
+      float sum = 0.f;
+#pragma unroll
+      for (int wv = 0; wv < NW; ++wv) sum += s_ss[wv][16 * t + col];
+      const float inv = rsqrtf(sum / static_cast<float>(a.k) + a.eps);
+      v *= inv;
+      up *= inv;
+    }
+    const int r = r0 + 16 * t + col;
+    const int c = n0 + 16 * u + 4 * quad;
+    if (r >= a.m || (!GLU && n0 + 16 * u >= a.n)) continue;
+    Pack<R, 4> out;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      out.v[j] = GLU ? silu_mul_round<E>(E::store(v[j]), E::store(up[j])) : E::store(v[j]);
+    if (a.res != nullptr) {
+      const Pack<R, 4> res =
+          load_pack<R, 4>(static_cast<const R*>(a.res) + static_cast<int64_t>(r) * a.rs + c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) out.v[j] = add_residual<E>(out.v[j], res.v[j]);
+    }
+    store_pack<R, 4>(y + static_cast<int64_t>(r) * a.ys + c, out);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows (m <= 4).
+// ---------------------------------------------------------------------------
+constexpr int kGemvWaves = 4;
+constexpr int kGemvChunk = 8 * kWave;  // elements of a row one load takes
+
+// A wave owns RW weight rows (GLU: one gate row and its up row) and all M rows
+// of x; U loads of each row are in flight.
+template <typename E, int M, int RW, int U, bool GLU, bool NORM>
+__global__ __launch_bounds__(kGemvWaves* kWave) void gemv_kernel(const LinArgs a) {
+  using R = uint16_t;
+  static_assert(!GLU || RW == 2, "GLU: a gate row and an up row");
+  const int lane = threadIdx.x % kWave;
+  const int item = __builtin_amdgcn_readfirstlane(blockIdx.x * kGemvWaves + threadIdx.x / kWave);
+  const int n0 = GLU ? item : item * RW;
+  if (n0 >= (GLU ? a.inter : a.n)) return;
+  const R* wrow[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r)
+    wrow[r] = static_cast<const R*>(a.w) +
+              static_cast<int64_t>(GLU ? n0 + r * a.inter : min(n0 + r, a.n - 1)) * a.ws;
+  const R* xrow[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+    xrow[i] = static_cast<const R*>(a.x) + static_cast<int64_t>(min(i, a.m - 1)) * a.xs;
+  const R* nrow = static_cast<const R*>(a.norm);
+
+  float acc[RW][M], ss[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    ss[i] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RW; ++r) acc[r][i] = 0.f;
+  }
+  for (int k0 = 0; k0 < a.k; k0 += U * kGemvChunk) {
+    Pack<R, 8> w[U][RW], x[U][M], g[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int off = k0 + u * kGemvChunk + lane * 8;
+      const bool in = off < a.k;
+      const int at = in ? off : 0;
+#pragma unroll
+      for (int r = 0; r < RW; ++r) w[u][r] = load_pack<R, 8>(wrow[r] + at);
+      if constexpr (NORM) g[u] = load_pack<R, 8>(nrow + at);
+#pragma unroll
+      for (int i = 0; i < M; ++i) x[u][i] = load_pack<R, 8>(xrow[i] + at);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + u * kGemvChunk + lane * 8 < a.k) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+          Pack<R, 8> xv = x[u][i];
+          if constexpr (NORM) {
+            ss[i] = dot8<E>(xv, xv, ss[i]);
+            xv = scale8<E>(xv, g[u]);
+          }
+#pragma unroll
+          for (int r = 0; r < RW; ++r) acc[r][i] = dot8<E>(xv, w[u][r], acc[r][i]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    if constexpr (NORM) {
+      const float inv = rsqrtf(group_sum<kWave>(ss[i]) / static_cast<float>(a.k) + a.eps);
+#pragma unroll
+      for (int r = 0; r < RW; ++r) acc[r][i] = group_sum<kWave>(acc[r][i]) * inv;
+    } else {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) acc[r][i] = group_sum<kWave>(acc[r][i]);
+    }
+  }
+  // Lane i stores row i of x: the wave's columns are neighbours.
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    if (lane != i || i >= a.m) continue;
+    R* y = static_cast<R*>(a.y) + static_cast<int64_t>(i) * a.ys + n0;
+    const R* res = a.res != nullptr
+                       ? static_cast<const R*>(a.res) + static_cast<int64_t>(i) * a.rs + n0
+                       : nullptr;
+    if constexpr (GLU) {
+      const R v = silu_mul_round<E>(E::store(acc[0][i]), E::store(acc[1][i]));
+      y[0] = res != nullptr ? add_residual<E>(v, res[0]) : v;
+    } else {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) {
+        if (n0 + r >= a.n) continue;
+        const R v = E::store(acc[r][i]);
+        y[r] = res != nullptr ? add_residual<E>(v, res[r]) : v;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Dispatch.
+// ---------------------------------------------------------------------------
+template <typename E, int NW, int NT, int MT, int S, bool GLU, bool NORM>
+void launch_mfma(LinArgs a, hipStream_t stream) {
+  a.row_groups = (a.m + 16 * MT - 1) / (16 * MT);
+  const int col_tiles = GLU ? a.inter / 16 : (a.n + 16 * NT - 1) / (16 * NT);
+  const dim3 grid(static_cast<uint32_t>((col_tiles + 7) / 8 * 8 * a.row_groups));
+  linear_kernel<E, NW, NT, MT, S, GLU, NORM><<<grid, NW * kWave, 0, stream>>>(a);
+}
+
+// Two slots per wave while every workgroup has a CU to itself (4096 x 1024 at
+// 64 rows: 4.5 us, 4.9 with one), else one slot and more workgroups per CU
+// (24576 x 4096 at 32 rows: 40.7, 41.6 with two). With the norm, whose weights
+// are waited for with the chunk, one slot.
+template <typename E, int NT, int MT, bool GLU, bool NORM>
+void launch_tile(const LinArgs& a, bool eight, bool alone, hipStream_t stream) {
+  if (eight) {
+    if constexpr (MT <= 2) {
+      if constexpr (NT == 1 && MT == 1 && !NORM) {
+        if (alone) return launch_mfma<E, 8, NT, MT, 2, GLU, NORM>(a, stream);
+      }
+      return launch_mfma<E, 8, NT, MT, 1, GLU, NORM>(a, stream);
+    }
+  } else {
+    if constexpr (MT <= 2 && !NORM) {
+      if (alone) return launch_mfma<E, 4, NT, MT, 2, GLU, NORM>(a, stream);
+    }
+    return launch_mfma<E, 4, NT, MT, 1, GLU, NORM>(a, stream);
+  }
+}
+
+// Tile per workgroup (NT 16-column tiles x MT 16-row tiles): a workgroup's
+// time goes with the rows of w and x it stages, so the tile with the least
+// (workgroups per CU, rounded up) x (NT + MT). Measured against the others
+// (us): 4096 x 1024 at 64 rows 2 x 2 4.5, 1 x 1 6.0, 1 x 2 7.0; 2048 x 6144 at
+// 48 rows 1 x 2 11.2, 1 x 1 14.7, 2 x 2 15.0; 24576 x 4096 at 48 rows 2 x 3 45,
+// 2 x 2 55.
+struct LinTile {
+  int nt, mt;
+  bool alone;  // at most one workgroup per CU
+};
+LinTile pick_tile(const LinArgs& a, bool glu, bool eight) {
+  static constexpr int kTiles[][2] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {2, 3}};
+  const int cus = device_cus(), rows = (a.m + 15) / 16;
+  LinTile best{0, 0, false};
+  int64_t best_cost = 0;
+  for (const auto& t : kTiles) {
+    const int nt = t[0], mt = t[1];
+    if (mt > rows || (glu && nt != 2) || (!glu && nt == 2 && mt == 1) || (eight && mt == 3))
+      continue;
+    const int64_t cols = glu ? a.inter / 16 : (a.n + 16 * nt - 1) / (16 * nt);
+    const int64_t groups = cols * ((rows + mt - 1) / mt);
+    const int64_t cost = (groups + cus - 1) / cus * (nt + mt);
+    if (best.nt == 0 || cost < best_cost) {
+      best = LinTile{nt, mt, groups <= cus};
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+template <typename E, bool GLU, bool NORM>
+void launch_many_rows(const LinArgs& a, hipStream_t stream) {
+  // Narrow outputs: eight waves per tile (1024 x 3072 at 8 rows: 4.35 us, 4.68
+  // with four); wider ones have workgroups enough (4096 x 1024: 3.9, 3.7 with
+  // four). By n alone, so that the fused gate sums as the projection does.
+  const bool eight = a.n < 4096;
+  const LinTile t = pick_tile(a, GLU, eight);
+  if constexpr (!GLU) {
+    if (t.nt == 1 && t.mt == 1) return launch_tile<E, 1, 1, GLU, NORM>(a, eight, t.alone, stream);
+    if (t.nt == 1) return launch_tile<E, 1, 2, GLU, NORM>(a, eight, t.alone, stream);
+  } else if (t.mt == 1) {
+    return launch_tile<E, 2, 1, GLU, NORM>(a, eight, t.alone, stream);
+  }
+  if (t.mt == 2) return launch_tile<E, 2, 2, GLU, NORM>(a, eight, t.alone, stream);
+  return launch_tile<E, 2, 3, GLU, NORM>(a, eight, t.alone, stream);
+}
+
+template <typename E, int M, bool GLU, bool NORM>
+void launch_gemv(const LinArgs& a, hipStream_t stream) {
+  // Rows per wave and loads in flight: one weight row and, past 1024 elements,
+  // up to six loads of it; with the norm two rows share the scaled x.
+  constexpr int RW = GLU || NORM ? 2 : 1;
+  const int items = GLU ? a.inter : (a.n + RW - 1) / RW;
+  const dim3 grid(static_cast<uint32_t>((items + kGemvWaves - 1) / kGemvWaves));
+  const dim3 block(kGemvWaves * kWave);
+  if (GLU || NORM || a.k <= 2 * kGemvChunk)
+    gemv_kernel<E, M, RW, 2, GLU, NORM><<<grid, block, 0, stream>>>(a);
+  else if (a.k <= 4 * kGemvChunk)
+    gemv_kernel<E, M, RW, 4, GLU, NORM><<<grid, block, 0, stream>>>(a);
+  else
+    gemv_kernel<E, M, RW, 6, GLU, NORM><<<grid, block, 0, stream>>>(a);
+}
+
+// One or two rows take the vector kernel (1024 x 2048: 3.1 / 3.2 us, 3.5 / 3.6
+// on MFMA; 4096 x 1024 3.6, 3.8; the gate/up 6144 x 1024 4.7 / 5.1, 5.2 / 5.3);
+// four take MFMA (3.8 against 3.7, 4.1 against 3.7, 6.6 against 5.3).
+template <typename E, bool GLU, bool NORM>
+void launch_typed(const LinArgs& a, hipStream_t stream) {
+  if (a.m == 1)
+    launch_gemv<E, 1, GLU, NORM>(a, stream);
+  else if (a.m == 2)
+    launch_gemv<E, 2, GLU, NORM>(a, stream);
+  else
+    launch_many_rows<E, GLU, NORM>(a, stream);
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+int32_t linear(const char* who, const LinArgs& a, bool swiglu, int32_t dtype, void* stream) {
+  clear_error();
+  const std::string fn(who);
+  if (!valid_dtype(dtype)) return fail(MI_ERR_INVALID_ARGUMENT, fn + ": bad dtype");
+  const int out = swiglu ? a.inter : a.n;
+  if (a.m < 0 || out <= 0 || a.k <= 0 || out % 16 || a.k % kLinStep)
+    return fail(MI_ERR_INVALID_ARGUMENT,
+                fn + ": need m >= 0, the output width a positive multiple of 16, k of 32");
+  if (dtype == MI_DTYPE_F32) return fail(MI_ERR_UNSUPPORTED, fn + ": 16-bit types only");
+  if (a.m > kLinMaxRows) return fail(MI_ERR_UNSUPPORTED, fn + ": m above 64");
+  if (a.m == 0) return MI_OK;
+  if (!a.x || !a.w || !a.y) return fail(MI_ERR_INVALID_ARGUMENT, fn + ": null pointer");
+  if (a.xs < a.k || a.ws < a.k || a.ys < out || (a.res && a.rs < out))
+    return fail(MI_ERR_INVALID_ARGUMENT, fn + ": row strides below the row lengths");
+  if (!aligned16(a.x) || !aligned16(a.w) || !aligned16(a.y) || a.xs % 8 || a.ws % 8 ||
+      a.ys % 8 || (a.norm && !aligned16(a.norm)) || (a.res && (!aligned16(a.res) || a.rs % 8)))
+    return fail(MI_ERR_INVALID_ARGUMENT,
+                fn + ": pointers and row strides must be 16-byte aligned");
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  auto go = [&](auto type) {
+    using E = decltype(type);
+    if (swiglu)
+      a.norm ? launch_typed<E, true, true>(a, s) : launch_typed<E, true, false>(a, s);
+    else
+      a.norm ? launch_typed<E, false, true>(a, s) : launch_typed<E, false, false>(a, s);
+  };
+  if (dtype == MI_DTYPE_BF16)
+    go(BF16{});
+  else
+    go(F16{});
+  return check_launch(who);
+}
+
+}  // namespace
+}  // namespace mi
+
+extern "C" int32_t mi_linear(const void* x, int64_t x_row_stride, const void* w,
+                             int64_t w_row_stride, void* y, int64_t y_row_stride, int32_t m,
+                             int32_t n, int32_t k, int32_t dtype, void* stream) {
+  mi::LinArgs a{};
+  a.x = x;
+  a.xs = x_row_stride;
+  a.w = w;
+  a.ws = w_row_stride;
+  a.y = y;
+  a.ys = y_row_stride;
+  a.m = m;
+  a.n = n;
+  a.k = k;
+  return mi::linear("mi_linear", a, false, dtype, stream);
+}
+
+extern "C" int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
+                                    int64_t w_row_stride, void* y, int64_t y_row_stride,
+                                    int32_t m, int32_t inter, int32_t k, int32_t dtype,
+                                    void* stream) {
+  mi::LinArgs a{};
+  a.x = x;
+  a.xs = x_row_stride;
+  a.w = w;
+  a.ws = w_row_stride;
+  a.y = y;
+  a.ys = y_row_stride;
+  a.m = m;
+  a.n = 2 * inter;
+  a.inter = inter;
+  a.k = k;
+  return mi::linear("mi_linear_swiglu", a, true, dtype, stream);
+}
+
+extern "C" int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const void* norm_weight,
+                                   float eps, const void* w, int64_t w_row_stride,
+                                   const void* residual, int64_t residual_row_stride, void* y,
+                                   int64_t y_row_stride, int32_t m, int32_t n, int32_t k,
+                                   int32_t swiglu, int32_t dtype, void* stream) {
+  mi::LinArgs a{};
+  a.x = x;
+  a.xs = x_row_stride;
+  a.norm = norm_weight;
+  a.eps = eps;
+  a.w = w;
+  a.ws = w_row_stride;
+  a.res = residual;
+  a.rs = residual_row_stride;
+  a.y = y;
+  a.ys = y_row_stride;
+  a.m = m;
+  a.n = n;
+  a.inter = n / 2;
+  a.k = k;
+  if (swiglu && n % 2 != 0) {
+    mi::clear_error();
+    return mi::fail(MI_ERR_INVALID_ARGUMENT, "mi_linear_fused: gate/up needs an even n");
+  }
+  return mi::linear("mi_linear_fused", a, swiglu != 0, dtype, stream);
+}

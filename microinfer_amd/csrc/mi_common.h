@@ -65,6 +65,15 @@ struct F16 {
 // range flush to zero, which only affects weights already < 2^-126).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// round(round(silu(g)) * u) on 16-bit inputs: the rounding steps of torch's
+// F.silu(gate) * up.
+template <typename E>
+__device__ __forceinline__ uint16_t silu_mul_round(uint16_t g, uint16_t u) {
+  const float x = E::load(g);
+  const float act = E::load(E::store(x / (1.f + expf(-x))));
+  return E::store(act * E::load(u));
+}
+
 // N consecutive raw elements moved with one load/store instruction.
 template <typename R, int N>
 struct alignas(sizeof(R) * N) Pack {

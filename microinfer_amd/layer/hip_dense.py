@@ -40,13 +40,32 @@ def prefer_hip_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``hip_linear`` beats torch's product for this request.
 
     Measured on MI355X (hipGraph-replayed, the Qwen3-0.6B projections, us per
-    launch, HIP against hipBLASLt): at 64 rows QKV 8.1 / 8.5, output 6.1 /
-    8.0, gate/up 10.4 / 11.9, down 8.1 / 9.7; at 8 rows 4.1 / 5.9, 5.3 /
-    8.1, 6.2 / 8.0, 7.0 / 9.1. The vocabulary projection (151936 columns)
-    stays on hipBLASLt past 16 rows (64 rows: 138 against 85)."""
-    if not supported_linear(x, weight):
-        return False
-    return x.shape[0] <= 16 or weight.shape[0] <= 32768
+    launch, HIP against hipBLASLt): at 64 rows QKV 4.5 / 8.5, output 4.3 /
+    8.0, gate/up 8.0 / 11.9, down 4.7 / 9.7; at 8 rows 3.7 / 5.9, 3.8 /
+    8.1, 5.3 / 8.0, 4.4 / 9.1. The vocabulary projection (151936 columns)
+    goes to hipBLASLt past 48 rows (1 row 50 / 60, 16 rows 64 / 62, 32 rows
+    70 / 75, 48 rows 77 / 78, 64 rows 104 / 82)."""
+    return supported_linear(x, weight) and _measured_faster(x.shape[0], weight)
+
+
+def _measured_faster(rows: int, weight: torch.Tensor) -> bool:
+    return rows <= 48 or weight.shape[0] <= 32768
+
+
+def prefer_hip_rows(rows: int, weight: torch.Tensor) -> bool:
+    """``prefer_hip_linear`` for aligned x of ``rows`` rows of weight's dtype."""
+    return (0 < rows <= LINEAR_MAX_ROWS and weight.is_cuda and weight.dtype in _HALF
+            and weight.dim() == 2 and weight.shape[0] % 16 == 0 and weight.shape[1] % 32 == 0
+            and _rows_aligned(weight) and _measured_faster(rows, weight))
+
+
+def prefer_fused_norm(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the norm in front of a preferred projection is better done
+    inside it: every workgroup then scales the x rows it reads again, which
+    past 16 rows and 2048 elements costs more than the norm's own launch (3.6
+    us; 24576 x 4096 at 64 rows 67 against 59 + 3.6, 12288 x 2048 22.7
+    against 19.4 + 3.6, 4096 x 1024 6.2 against 4.5 + 3.6)."""
+    return prefer_hip_linear(x, weight) and (x.shape[0] <= 16 or x.shape[1] <= 2048)
 
 
 def hip_linear(x: torch.Tensor, weight: torch.Tensor, *,
@@ -90,6 +109,42 @@ def hip_linear_swiglu(x: torch.Tensor, gate_up: torch.Tensor, *,
         x.data_ptr(), x.stride(0), gate_up.data_ptr(), gate_up.stride(0), out.data_ptr(),
         out.stride(0), m, inter, k, _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)),
         "mi_linear_swiglu")
+    return out
+
+
+def hip_linear_fused(x: torch.Tensor, weight: torch.Tensor, *,
+                     norm_weight: torch.Tensor | None = None, eps: float = 0.0,
+                     residual: torch.Tensor | None = None, swiglu: bool = False) -> torch.Tensor:
+    """``residual + F.linear(rms_norm(x) * norm_weight, weight)`` in one launch,
+    or with ``swiglu`` the gate ``silu(gate) * up`` of a ``[2 I, k]`` weight;
+    ``norm_weight`` and ``residual`` are optional (``FuseLayerNorm.forward``,
+    norm.py:26-35, around the projections of ``TransformerLayer.forward``,
+    transformer.py:245-252). The norm's product is rounded once and its scale
+    applied to the float32 sum; the other roundings are those of the separate
+    calls."""
+    _lib.require_device(x, weight, norm_weight, residual, what="fused projection")
+    if not supported_linear(x, weight) or (swiglu and weight.shape[0] % 32):
+        raise ValueError("hip_linear_fused: x [m <= 64, k] and weight [n % 16 == 0, k % 32 == 0] "
+                         "(gate/up: n % 32 == 0) of one 16-bit dtype with 16-byte aligned rows "
+                         "are required")
+    m, k = x.shape
+    n = weight.shape[0]
+    width = n // 2 if swiglu else n
+    if norm_weight is not None and (norm_weight.shape != (k,) or norm_weight.dtype != x.dtype
+                                    or not norm_weight.is_contiguous()
+                                    or norm_weight.data_ptr() % 16):
+        raise ValueError("hip_linear_fused: norm_weight must be an aligned [k] of x's dtype")
+    if residual is not None and (residual.shape != (m, width) or residual.dtype != x.dtype
+                                 or not _rows_aligned(residual)):
+        raise ValueError("hip_linear_fused: residual must be [m, width] of x's dtype with "
+                         "aligned rows")
+    out = torch.empty((m, width), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.load().mi_linear_fused(
+        x.data_ptr(), x.stride(0), 0 if norm_weight is None else norm_weight.data_ptr(),
+        float(eps), weight.data_ptr(), weight.stride(0),
+        0 if residual is None else residual.data_ptr(),
+        0 if residual is None else residual.stride(0), out.data_ptr(), out.stride(0), m, n, k,
+        int(swiglu), _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)), "mi_linear_fused")
     return out
 
 

@@ -14,8 +14,8 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_swiglu, hip_rms_norm_residual,
-                                            hip_silu_mul)
+from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_fused, hip_linear_swiglu,
+                                            hip_rms_norm_residual, hip_silu_mul)
 from microinfer_amd.runner import capture_graph
 
 pytestmark = pytest.mark.gpu
@@ -195,3 +195,48 @@ def test_linear_swiglu_rejects_and_strides():
     y = hip_linear_swiglu(x, w, out=out)
     assert y.data_ptr() == out.data_ptr()
     assert torch.equal(y, hip_silu_mul(hip_linear(x.contiguous(), w)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 2, 3, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(4096, 1024), (1024, 3072), (6144, 4096), (48, 64), (2048, 160)])
+def test_linear_fused_is_norm_projection_and_sum(dtype, m, n, k):
+    """Every tile shape of the launcher, partial tiles and chunks. Without the
+    norm the launch equals the separate ones bit for bit; with it the float64
+    result within the roundings of the scaled x and of the output (and of
+    gate and up)."""
+    torch.manual_seed(m * 17 + n + k)
+    eps = 1e-6
+    x = torch.randn(m, k, device=DEV).to(dtype)
+    w = (0.05 * torch.randn(n, k, device=DEV)).to(dtype)
+    g = (1 + 0.1 * torch.randn(k, device=DEV)).to(dtype)
+    r = torch.randn(m, n, device=DEV).to(dtype)
+    assert torch.equal(hip_linear_fused(x, w, residual=r), r + hip_linear(x, w))
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    normed = F.rms_norm(x.double(), (k,), g.double(), eps)
+    # One rounding of each scaled x (k of them, independent) and one of y.
+    spread = unit * (normed.square() @ w.double().square().t()).sqrt()
+    y = normed @ w.double().t()
+    got = hip_linear_fused(x, w, norm_weight=g, eps=eps).double()
+    assert bool(((got - y).abs() <= 4 * spread + unit * y.abs() + 1e-6).all())
+    if n % 32 == 0:
+        fused = hip_linear_fused(x, w, swiglu=True)
+        assert torch.equal(fused, hip_linear_swiglu(x, w))
+        gate, up = y.chunk(2, dim=-1)
+        e_gate, e_up = (4 * spread + unit * y.abs() + 1e-6).chunk(2, dim=-1)
+        want = F.silu(gate) * up
+        # |silu'| <= 1.1; two more roundings.
+        bound = 1.1 * e_gate * (up.abs() + e_up) + F.silu(gate).abs() * e_up + 2 * unit * want.abs()
+        got = hip_linear_fused(x, w, norm_weight=g, eps=eps, swiglu=True).double()
+        assert bool(((got - want).abs() <= bound + 1e-6).all())
+
+
+def test_linear_fused_rejects():
+    x = torch.randn(8, 1024, device=DEV).to(torch.bfloat16)
+    w = torch.randn(64, 1024, device=DEV).to(torch.bfloat16)
+    with pytest.raises(ValueError):
+        hip_linear_fused(x, w, norm_weight=torch.ones(512, device=DEV, dtype=torch.bfloat16))
+    with pytest.raises(ValueError):
+        hip_linear_fused(x, w, residual=torch.zeros(8, 32, device=DEV, dtype=torch.bfloat16))
+    with pytest.raises(ValueError):
+        hip_linear_fused(x, w[:48], swiglu=True)
