@@ -29,8 +29,10 @@ from dataclasses import dataclass
 import torch
 from torch.nn import functional as F
 
-from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_swiglu, hip_rms_norm_residual,
-                                            hip_silu_mul, prefer_hip_linear, supported_rows)
+from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_fused, hip_linear_swiglu,
+                                            hip_rms_norm_residual, hip_silu_mul,
+                                            prefer_fused_norm, prefer_hip_linear, prefer_hip_rows,
+                                            supported_rows)
 from microinfer_amd.layer.hip_qk_norm_rope import qk_norm_rope_append, rope_tables
 from microinfer_amd.layer.paged_attention import paged_attention_meta, varlen_attention
 
@@ -128,31 +130,61 @@ class Qwen3Model:
             return hip_linear_swiglu(x, gate_up)
         return self._swiglu(self._linear(x, gate_up))
 
+    def _norm_project(self, x, norm_weight, weight, swiglu=False):
+        """A projection (or gate/up with its gate) of the normalised rows."""
+        if prefer_fused_norm(x, weight):
+            return hip_linear_fused(x, weight, norm_weight=norm_weight,
+                                    eps=self.config.norm_eps, swiglu=swiglu)
+        x, _ = self._norm(x, None, norm_weight)
+        return self._ffn_gate(x, weight) if swiglu else self._linear(x, weight)
+
+    def _fuses(self, layer, hidden) -> bool:
+        """Whether this layer's projections take its norms, gate and residual
+        sums along: the HIP projections are preferred for all four."""
+        rows = hidden.shape[0]
+        return (self.hip_dense and supported_rows(hidden) and layer.gate_up.shape[0] % 32 == 0
+                and all(w.dtype == hidden.dtype and prefer_hip_rows(rows, w)
+                        for w in (layer.qkv, layer.out, layer.gate_up, layer.down)))
+
+    def _attend(self, layer, cache, qkv, positions, metadata):
+        """Attention output ``[T, Hq D]`` of one layer's fused QKV rows."""
+        c = self.config
+        tokens = qkv.shape[0]
+        direct = metadata.is_prefill and metadata.direct_prefill
+        rotated = qk_norm_rope_append(
+            qkv, q_weight=layer.q_norm, k_weight=layer.k_norm, eps=c.norm_eps,
+            cos_table=self.cos, sin_table=self.sin, positions=positions,
+            num_q_heads=c.num_q_head, num_kv_heads=c.num_kv_head, head_dim=c.head_dim,
+            interleaved=c.rope_interleaved, slot_mapping=metadata.slot_mapping,
+            key_cache=cache.keys, value_cache=cache.values, return_k=direct)
+        if direct:  # no cached prefix: attend over this step's own K/V
+            q, k = rotated
+            v = qkv[:, (c.num_q_head + c.num_kv_head) * c.head_dim:]
+            v = v.reshape(tokens, c.num_kv_head, c.head_dim)
+            attn = varlen_attention(q, k, v.contiguous(), metadata)
+        else:
+            attn = paged_attention_meta(rotated, cache.keys, cache.values, metadata)
+        return attn.reshape(tokens, c.num_q_head * c.head_dim)
+
     def forward(self, input_ids, positions, metadata):
         """Hidden states ``[T, H]`` of the packed tokens of one step."""
-        c = self.config
         if self.caches is None:
             raise RuntimeError("bind the KV caches before running the model")
-        tokens = input_ids.shape[0]
-        q_width, kv_width = c.num_q_head * c.head_dim, c.num_kv_head * c.head_dim
-        direct = metadata.is_prefill and metadata.direct_prefill
         hidden, residual = F.embedding(input_ids, self.embedding), None
         for layer, cache in zip(self.layers, self.caches):
+            if self._fuses(layer, hidden):
+                # Five launches: each norm in front of its projection, each
+                # residual sum and the gate behind theirs.
+                x = hidden if residual is None else hidden + residual
+                qkv = self._norm_project(x, layer.pre_norm, layer.qkv)
+                attn = self._attend(layer, cache, qkv, positions, metadata)
+                x = hip_linear_fused(attn, layer.out, residual=x)
+                gate = self._norm_project(x, layer.post_norm, layer.gate_up, swiglu=True)
+                hidden, residual = hip_linear_fused(gate, layer.down, residual=x), None
+                continue
             x, residual = self._norm(hidden, residual, layer.pre_norm)
-            qkv = self._linear(x, layer.qkv)
-            rotated = qk_norm_rope_append(
-                qkv, q_weight=layer.q_norm, k_weight=layer.k_norm, eps=c.norm_eps,
-                cos_table=self.cos, sin_table=self.sin, positions=positions,
-                num_q_heads=c.num_q_head, num_kv_heads=c.num_kv_head, head_dim=c.head_dim,
-                interleaved=c.rope_interleaved, slot_mapping=metadata.slot_mapping,
-                key_cache=cache.keys, value_cache=cache.values, return_k=direct)
-            if direct:  # no cached prefix: attend over this step's own K/V
-                q, k = rotated
-                v = qkv[:, q_width + kv_width:].reshape(tokens, c.num_kv_head, c.head_dim)
-                attn = varlen_attention(q, k, v.contiguous(), metadata)
-            else:
-                attn = paged_attention_meta(rotated, cache.keys, cache.values, metadata)
-            hidden = self._linear(attn.reshape(tokens, q_width), layer.out)
+            attn = self._attend(layer, cache, self._linear(x, layer.qkv), positions, metadata)
+            hidden = self._linear(attn, layer.out)
             x, residual = self._norm(hidden, residual, layer.post_norm)
             hidden = self._linear(self._ffn_gate(x, layer.gate_up), layer.down)
         return self._norm(hidden, residual, self.final_norm)[0]
