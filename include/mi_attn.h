@@ -212,6 +212,38 @@ int32_t mi_paged_decode_append_noalloc(
     int32_t num_blocks, int32_t split_k, float scale, int32_t dtype, void* stream);
 
 /*
+ * Decode step of one layer from its fused QKV projection rows: the Q/K norm,
+ * RoPE and append of mi_qk_norm_rope_append, then mi_paged_decode, in one
+ * launch. Row s of qkv ([q heads | k heads | v heads], head_dim elements each)
+ * belongs to sequence s; positions[s] (int64) and slot_mapping[s] are its
+ * position and cache slot. Same result as the two calls -- the query rows
+ * equal theirs up to the summation order of the norm -- where slot_mapping[s]
+ * is the sequence's place context_lens[s] - 1 in its table, as the step
+ * metadata builds it. A row with another slot (a graph pad row) is stored
+ * there and not attended to from this launch; a slot outside the cache or a
+ * position outside the angle table is not stored. As with
+ * mi_paged_decode_append, the block that receives a row must not be read by
+ * another sequence of the call.
+ *
+ * bf16/f16, head_dim 128, at most 16 query heads per KV head, block_size >= 16
+ * (MI_ERR_UNSUPPORTED otherwise: make the two calls). qkv, the caches and out
+ * 16-byte aligned with strides of whole 16-byte vectors. The rest is as for
+ * mi_paged_decode.
+ */
+int32_t mi_paged_decode_qkv(
+    const void* qkv, int64_t qkv_token_stride, const void* q_weight, const void* k_weight,
+    float eps, const float* cos_table, const float* sin_table, int32_t table_len,
+    int32_t interleaved, const int64_t* positions, const int32_t* slot_mapping, void* key_cache,
+    void* value_cache, int64_t cache_block_stride, int64_t cache_token_stride,
+    int64_t cache_head_stride, const int32_t* block_tables, int64_t block_table_stride,
+    int32_t block_table_width, const int32_t* context_lens, void* out,
+    int64_t out_token_stride, int64_t out_head_stride, void* workspace,
+    int64_t workspace_bytes, int32_t* counters, const void* plan, int64_t plan_bytes,
+    int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+    int32_t block_size, int32_t num_blocks, int32_t split_k, float scale, int32_t dtype,
+    void* stream);
+
+/*
  * Paged varlen (prefill / mixed) attention with a bottom-right causal mask:
  * request r owns query rows [cu_seqlens_q[r], cu_seqlens_q[r+1]) and context
  * c_r = cu_seqlens_k[r+1] - cu_seqlens_k[r]; its query row i sits at position

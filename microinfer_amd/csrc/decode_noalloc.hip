@@ -100,5 +100,5 @@ extern "C" int32_t mi_paged_decode_append_noalloc(
                       block_table_stride, block_table_width, context_lens, out,
                       out_token_stride, out_head_stride, workspace, room, counters, nullptr,
                       0, num_seqs, num_q_heads, num_kv_heads, head_dim, block_size,
-                      num_blocks, split_k, scale, dtype, rows, stream);
+                      num_blocks, split_k, scale, dtype, rows, QkvRows{}, stream);
 }

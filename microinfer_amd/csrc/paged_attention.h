@@ -88,10 +88,26 @@ int32_t launch_prefill_mfma_planned(AttnArgs args, int32_t dtype, void* workspac
 bool prefill_f32_supported(const AttnArgs& args, int32_t dtype);
 int32_t launch_prefill_f32(const AttnArgs& args, hipStream_t stream);
 
+// Norm and rotation of the fused QKV rows [q heads | k heads | v heads] that
+// AttnArgs::q then holds (null q_weight: q holds finished query rows), and the
+// cache slots and positions of their K/V.
+struct QkvRows {
+  int64_t ts = 0;
+  const void* q_weight = nullptr;
+  const void* k_weight = nullptr;
+  float eps = 0.f;
+  const float* cos_t = nullptr;  // [table_len, D / 2]
+  const float* sin_t = nullptr;
+  int32_t table_len = 0, interleaved = 0;
+  const int64_t* positions = nullptr;
+  const int32_t* slots = nullptr;
+};
+
 // MFMA decode kernel (paged_decode_mfma.hip): 16-bit caches, head_dim 128,
 // up to 16 query heads per KV head, block size >= 16, paged.
 bool decode_mfma_supported(const AttnArgs& args, int32_t dtype);
-int32_t launch_decode_mfma(const AttnArgs& args, int32_t dtype, hipStream_t stream);
+int32_t launch_decode_mfma(const AttnArgs& args, const QkvRows& qkv, int32_t dtype,
+                           hipStream_t stream);
 
 // Upper bound on decode work items for a launch (grid.x / Hkv).
 int32_t decode_max_items(int32_t num_seqs, int32_t num_kv_heads, int32_t split_k);
@@ -126,6 +142,6 @@ int32_t paged_decode(
     int64_t workspace_bytes, int32_t* counters, const void* plan, int64_t plan_bytes,
     int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
     int32_t block_size, int32_t num_blocks, int32_t split_k, float scale, int32_t dtype,
-    const NewRows& rows, void* stream);
+    const NewRows& rows, const QkvRows& qkv, void* stream);
 
 }  // namespace mi

@@ -81,7 +81,7 @@ int32_t paged_decode(
     int64_t workspace_bytes, int32_t* counters, const void* plan, int64_t plan_bytes,
     int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
     int32_t block_size, int32_t num_blocks, int32_t split_k, float scale, int32_t dtype,
-    const NewRows& rows, void* stream) {
+    const NewRows& rows, const QkvRows& qkv, void* stream) {
   int32_t st = check_common("mi_paged_decode", dtype, num_q_heads, num_kv_heads, head_dim,
                             block_size, num_blocks, block_table_width);
   if (st != MI_OK) return st;
@@ -155,6 +155,10 @@ int32_t paged_decode(
   a.new_v = rows.values;
   a.nv_ts = rows.v_ts;
   a.nv_hs = rows.v_hs;
+  if (qkv.q_weight != nullptr && !decode_mfma_supported(a, dtype))
+    return fail(MI_ERR_UNSUPPORTED,
+                "mi_paged_decode_qkv: bf16/f16 with head_dim 128, at most 16 query heads per KV "
+                "head and blocks of at least 16 only");
   hipStream_t s = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   const int64_t plan_region = round_up(decode_plan_bytes(num_seqs, num_kv_heads, split_k), 256);
@@ -176,7 +180,7 @@ int32_t paged_decode(
     a.ws_ml = a.ws_acc + acc_floats;
     a.counters = counters;
   }
-  if (decode_mfma_supported(a, dtype)) return launch_decode_mfma(a, dtype, s);
+  if (decode_mfma_supported(a, dtype)) return launch_decode_mfma(a, qkv, dtype, s);
   return dispatch_vector(a, dtype, s);
 }
 
@@ -199,7 +203,7 @@ extern "C" int32_t mi_paged_decode(
                           out, out_token_stride, out_head_stride, workspace, workspace_bytes,
                           counters, plan, plan_bytes, num_seqs, num_q_heads, num_kv_heads,
                           head_dim, block_size, num_blocks, split_k, scale, dtype,
-                          mi::NewRows{}, stream);
+                          mi::NewRows{}, mi::QkvRows{}, stream);
 }
 
 extern "C" int32_t mi_paged_decode_append(
@@ -230,7 +234,46 @@ extern "C" int32_t mi_paged_decode_append(
                           out, out_token_stride, out_head_stride, workspace, workspace_bytes,
                           counters, plan, plan_bytes, num_seqs, num_q_heads, num_kv_heads,
                           head_dim, block_size, num_blocks, split_k, scale, dtype, rows,
-                          stream);
+                          mi::QkvRows{}, stream);
+}
+
+extern "C" int32_t mi_paged_decode_qkv(
+    const void* qkv, int64_t qkv_token_stride, const void* q_weight, const void* k_weight,
+    float eps, const float* cos_table, const float* sin_table, int32_t table_len,
+    int32_t interleaved, const int64_t* positions, const int32_t* slot_mapping, void* key_cache,
+    void* value_cache, int64_t cache_block_stride, int64_t cache_token_stride,
+    int64_t cache_head_stride, const int32_t* block_tables, int64_t block_table_stride,
+    int32_t block_table_width, const int32_t* context_lens, void* out,
+    int64_t out_token_stride, int64_t out_head_stride, void* workspace,
+    int64_t workspace_bytes, int32_t* counters, const void* plan, int64_t plan_bytes,
+    int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+    int32_t block_size, int32_t num_blocks, int32_t split_k, float scale, int32_t dtype,
+    void* stream) {
+  using namespace mi;
+  clear_error();
+  if (!q_weight || !k_weight || !cos_table || !sin_table || !positions || !slot_mapping)
+    return fail(MI_ERR_INVALID_ARGUMENT, "mi_paged_decode_qkv: null pointer");
+  if (table_len <= 0 ||
+      qkv_token_stride < (static_cast<int64_t>(num_q_heads) + 2 * num_kv_heads) * head_dim)
+    return fail(MI_ERR_INVALID_ARGUMENT,
+                "mi_paged_decode_qkv: empty angle table or rows shorter than the heads");
+  QkvRows rows;
+  rows.ts = qkv_token_stride;
+  rows.q_weight = q_weight;
+  rows.k_weight = k_weight;
+  rows.eps = eps;
+  rows.cos_t = cos_table;
+  rows.sin_t = sin_table;
+  rows.table_len = table_len;
+  rows.interleaved = interleaved;
+  rows.positions = positions;
+  rows.slots = slot_mapping;
+  return paged_decode(qkv, qkv_token_stride, head_dim, key_cache, value_cache,
+                      cache_block_stride, cache_token_stride, cache_head_stride, block_tables,
+                      block_table_stride, block_table_width, context_lens, out,
+                      out_token_stride, out_head_stride, workspace, workspace_bytes, counters,
+                      plan, plan_bytes, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                      block_size, num_blocks, split_k, scale, dtype, NewRows{}, rows, stream);
 }
 
 namespace {

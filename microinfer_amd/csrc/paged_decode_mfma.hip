@@ -26,6 +26,11 @@
 //  * The fused append: the wave whose tile holds position ctx - 1 writes the
 //    step's new K/V row into its LDS tile (over the stale cache row) before
 //    reading the fragments, and stores the row to the cache after its loop.
+//  * From the fused QKV rows (QKV): wave g norms and rotates query head g (one
+//    rotation pair per lane) into LDS while the first tiles are in flight,
+//    and the wave after the last head does the new K row, which the fused
+//    append then takes. The norm + RoPE launch this saves is 3.5-4.7 us a
+//    layer; here it costs the barrier and about 100 instructions of one wave.
 //  * End of the workgroup: the waves' states are combined through LDS by all
 //    threads; a split sequence's partitions publish (acc, m, l) and the last
 //    arrival merges every partition with all its threads, one load round trip
@@ -125,8 +130,47 @@ __device__ __forceinline__ void merge_step(float& mx, float& ls, float& os, floa
   mx = mnew;
 }
 
-template <typename E, int NW, int NS>
-__global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const AttnArgs a) {
+// The QKV launches' arguments; the others keep the smaller block.
+struct QkvArgs : AttnArgs {
+  QkvRows qkv;
+};
+template <bool QKV>
+using ArgsOf = typename std::conditional<QKV, QkvArgs, AttnArgs>::type;
+
+// One head row of the fused QKV rows, normed and rotated by a wave as
+// qk_norm_rope_kernel does it: x * (1 / rms) * w in float32 rounded to the
+// element type, the rotation in float32 rounded again. Lane i holds rotation
+// pair i: elements (i, i + 64) or, interleaved, (2 i, 2 i + 1). A position
+// outside the angle table gives a zero row.
+template <typename E>
+__device__ __forceinline__ void norm_rope_row(const QkvRows& a, const uint16_t* row,
+                                              const uint16_t* weight, int pos, int64_t pos_true,
+                                              int lane, uint16_t* dst) {
+  using R = uint16_t;
+  const int ia = a.interleaved ? 2 * lane : lane;
+  const int ib = a.interleaved ? 2 * lane + 1 : lane + kD / 2;
+  const float x = E::load(row[ia]), y = E::load(row[ib]);
+  const float wx = E::load(weight[ia]), wy = E::load(weight[ib]);
+  // The angles of the row's place in its context, at once; the position
+  // itself is normally that and only then known.
+  const int safe = min(max(pos, 0), a.table_len - 1);
+  float cs = a.cos_t[static_cast<int64_t>(safe) * (kD / 2) + lane];
+  float sn = a.sin_t[static_cast<int64_t>(safe) * (kD / 2) + lane];
+  if (pos_true != safe) {
+    const bool ok = pos_true >= 0 && pos_true < a.table_len;
+    cs = ok ? a.cos_t[pos_true * (kD / 2) + lane] : 0.f;
+    sn = ok ? a.sin_t[pos_true * (kD / 2) + lane] : 0.f;
+  }
+  const float inv =
+      1.f / sqrtf(group_sum<kWave>(fmaf(x, x, y * y)) / static_cast<float>(kD) + a.eps);
+  const float nx = E::load(E::store(x * inv * wx));
+  const float ny = E::load(E::store(y * inv * wy));
+  dst[ia] = E::store(nx * cs - ny * sn);
+  dst[ib] = E::store(ny * cs + nx * sn);
+}
+
+template <typename E, int NW, int NS, bool QKV>
+__global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const ArgsOf<QKV> a) {
   using M = DecodeMfma<E>;
   using vec8 = typename M::vec8;
   using R = uint16_t;
@@ -137,6 +181,8 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
   __shared__ float s_m[NW][kHeads];
   __shared__ float s_l[NW][kHeads];
   __shared__ int s_arrived;
+  // QKV: the normed and rotated query rows, then the new K row.
+  __shared__ __attribute__((aligned(16))) uint16_t s_q[QKV ? (kHeads + 1) * kD : 8];
 
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
@@ -171,12 +217,17 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
   // wave whose tile holds it writes the row into LDS (and later the cache).
   bool append = false;
   int append_tile = -1;
-  if (a.new_k != nullptr && ctx >= 1 && a.ctx[seq] == ctx) {
+  if ((QKV || a.new_k != nullptr) && ctx >= 1 && a.ctx[seq] == ctx) {
     const int last = (ctx - 1) >> lb;
     append = blk_begin <= last && last < blk_end;
     if (append) append_tile = (ctx - 1 - pos_begin) / kTile;
   }
   const bool owner = append && append_tile % NW == wave;
+  // QKV: the row's slot is its place in the context (then it is attended to
+  // from LDS) or, for graph pad rows, another one of their pad block (then
+  // it is stored only); a negative or foreign slot is skipped.
+  [[maybe_unused]] bool in_slot = false;
+  int64_t row_off = -1;  // element offset of the appended row; -1: none
 
   const R* kc = static_cast<const R*>(a.kc);
   const R* vc = static_cast<const R*>(a.vc);
@@ -221,6 +272,36 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
     for (int ks = 0; ks < kD / 32; ++ks) {
       Pack<R, 8> p = zero_pack<R, 8>();
       if (col < G) p = load_pack<R, 8>(qrow + ks * 32 + quad * 8);
+      qf[ks] = __builtin_bit_cast(vec8, p);
+    }
+  };
+  // QKV: all G query rows and the new K row, one wave each, into LDS.
+  auto prepare_rows = [&](const auto& a) {
+    const R* row = static_cast<const R*>(a.q) + seq * a.qkv.ts;
+    const int64_t pos_true = a.qkv.positions[seq];
+    for (int r = wave; r <= G; r += NW) {
+      const bool is_k = r == G;
+      if (is_k && !append) continue;
+      norm_rope_row<E>(a.qkv, row + (is_k ? a.num_kv_heads * G + head : head * G + r) * kD,
+                       static_cast<const R*>(is_k ? a.qkv.k_weight : a.qkv.q_weight), ctx - 1, pos_true,
+                       lane, s_q + (is_k ? kHeads : r) * kD);
+    }
+    if (owner) {
+      const int slot = pos_true >= 0 && pos_true < a.qkv.table_len ? a.qkv.slots[seq] : -1;
+      const int blk = slot >> lb;
+      const int off = slot & (a.block_size - 1);
+      in_slot = slot >= 0 && blk == ctab[(ctx - 1) >> lb] &&
+                off == ((ctx - 1) & (a.block_size - 1)) && blk < a.num_blocks;
+      if (slot >= 0 && blk < a.num_blocks)
+        row_off = static_cast<int64_t>(blk) * a.c_bs + static_cast<int64_t>(off) * a.c_ts +
+                  head_off;
+    }
+  };
+  auto load_q_lds = [&]() {
+#pragma unroll
+    for (int ks = 0; ks < kD / 32; ++ks) {
+      Pack<R, 8> p = zero_pack<R, 8>();
+      if (col < G) p = load_pack<R, 8>(s_q + col * kD + ks * 32 + quad * 8);
       qf[ks] = __builtin_bit_cast(vec8, p);
     }
   };
@@ -293,13 +374,25 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
   // Static interleave: wave w takes tiles w, w + NW, ...; NS ring slots per
   // wave, so up to NS tiles of a wave are in flight.
   const int k0 = wave;
-  if (k0 < ntiles) {
-    bool ok_slot[NS];
+  bool ok_slot[NS];
 #pragma unroll
-    for (int j = 0; j < NS; ++j) ok_slot[j] = false;
-    ok_slot[0] = issue(0, k0);
-    load_q();
-    if (owner) {
+  for (int j = 0; j < NS; ++j) ok_slot[j] = false;
+  if constexpr (QKV) {
+    if (k0 < ntiles) ok_slot[0] = issue(0, k0);
+    prepare_rows(a);
+    if (owner)
+      new_v = load_pack<R, 8>(static_cast<const R*>(a.q) + seq * a.qkv.ts +
+                              (a.num_kv_heads * (G + 1) + head) * kD + col * 8);
+    __syncthreads();
+    load_q_lds();
+    if (owner) new_k = load_pack<R, 8>(s_q + kHeads * kD + col * 8);
+  }
+  if (k0 < ntiles) {
+    if constexpr (!QKV) {
+      ok_slot[0] = issue(0, k0);
+      load_q();
+    }
+    if (!QKV && owner) {
       const R* nk = static_cast<const R*>(a.new_k) + seq * a.nk_ts + head * a.nk_hs;
       const R* nv = static_cast<const R*>(a.new_v) + seq * a.nv_ts + head * a.nv_hs;
       new_k = load_pack<R, 8>(nk + col * 8);
@@ -363,7 +456,7 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
           }
         }
       }
-      if (owner && k == append_tile) {
+      if ((QKV ? in_slot : owner) && k == append_tile) {
         // The step's new row replaces the (stale) cache row in the tile.
         const int r = (ctx - 1) & (kTile - 1);
         if (lane < 16) {
@@ -387,7 +480,7 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
       k += NW;
       slot = slot + 1 == NS ? 0 : slot + 1;
     }
-  } else {
+  } else if constexpr (!QKV) {
     load_q();  // no tiles: the state stays empty
   }
   __builtin_amdgcn_s_setprio(0);
@@ -411,13 +504,16 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
 
   // The appended row goes to the cache (its block must be valid).
   if (owner && lane < 16) {
-    const int pos = ctx - 1;
-    const int blk = ctab[pos >> lb];
-    if (blk >= 0 && blk < a.num_blocks) {
-      const int64_t row = static_cast<int64_t>(blk) * a.c_bs +
-                          static_cast<int64_t>(pos & (a.block_size - 1)) * a.c_ts + head_off;
-      store_pack<R, 8>(const_cast<R*>(kc) + row + lane * 8, new_k);
-      store_pack<R, 8>(const_cast<R*>(vc) + row + lane * 8, new_v);
+    if constexpr (!QKV) {
+      const int pos = ctx - 1;
+      const int blk = ctab[pos >> lb];
+      if (blk >= 0 && blk < a.num_blocks)
+        row_off = static_cast<int64_t>(blk) * a.c_bs +
+                  static_cast<int64_t>(pos & (a.block_size - 1)) * a.c_ts + head_off;
+    }
+    if (row_off >= 0) {
+      store_pack<R, 8>(const_cast<R*>(kc) + row_off + lane * 8, new_k);
+      store_pack<R, 8>(const_cast<R*>(vc) + row_off + lane * 8, new_v);
     }
   }
 
@@ -574,14 +670,14 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Att
 // CUs run two workgroups per CU: 8 waves with one ring slot each (64 KiB of
 // LDS; 1-3 % faster than 4 waves with two slots on 64-128 short sequences)
 // instead of one 8-wave workgroup with two slots (128 KiB).
-template <typename E>
-int32_t launch_typed(const AttnArgs& a, hipStream_t stream) {
+template <typename E, bool QKV>
+int32_t launch_typed(const ArgsOf<QKV>& a, hipStream_t stream) {
   const dim3 grid(static_cast<uint32_t>(a.max_items) * a.num_kv_heads);
   const bool narrow = static_cast<int64_t>(a.num_seqs) * a.num_kv_heads > device_cus();
   if (narrow)
-    paged_decode_mfma_kernel<E, 8, 1><<<grid, kWave * 8, 0, stream>>>(a);
+    paged_decode_mfma_kernel<E, 8, 1, QKV><<<grid, kWave * 8, 0, stream>>>(a);
   else
-    paged_decode_mfma_kernel<E, 8, 2><<<grid, kWave * 8, 0, stream>>>(a);
+    paged_decode_mfma_kernel<E, 8, 2, QKV><<<grid, kWave * 8, 0, stream>>>(a);
   return check_launch("paged decode (MFMA)");
 }
 
@@ -593,9 +689,18 @@ bool decode_mfma_supported(const AttnArgs& a, int32_t dtype) {
          a.block_size >= kTile && a.c_ts >= 0 && a.c_ts * kTile < (int64_t(1) << 30);
 }
 
-int32_t launch_decode_mfma(const AttnArgs& a, int32_t dtype, hipStream_t stream) {
+int32_t launch_decode_mfma(const AttnArgs& a, const QkvRows& qkv, int32_t dtype,
+                           hipStream_t stream) {
   if (!decode_mfma_supported(a, dtype)) return MI_ERR_UNSUPPORTED;
-  return dtype == MI_DTYPE_BF16 ? launch_typed<BF16>(a, stream) : launch_typed<F16>(a, stream);
+  if (qkv.q_weight != nullptr) {
+    QkvArgs b;
+    static_cast<AttnArgs&>(b) = a;
+    b.qkv = qkv;
+    return dtype == MI_DTYPE_BF16 ? launch_typed<BF16, true>(b, stream)
+                                  : launch_typed<F16, true>(b, stream);
+  }
+  return dtype == MI_DTYPE_BF16 ? launch_typed<BF16, false>(a, stream)
+                                : launch_typed<F16, false>(a, stream);
 }
 
 }  // namespace mi

@@ -10,13 +10,15 @@ GQA attention over the paged KV cache, SwiGLU, a final norm and an untied
 last row on prefill (qwen3.py:57-65).
 
 On this path the per-layer Q/K norm + RoPE + KV append is one HIP launch
-(``mi_qk_norm_rope_append``), attention is the HIP paged decode / varlen
+(``mi_qk_norm_rope_append``; in decode steps part of the attention's,
+``mi_paged_decode_qkv``), attention is the HIP paged decode / varlen
 prefill (``paged_attention_meta`` / ``varlen_attention``), and RMSNorm with
 its residual sum and the SwiGLU gate are HIP launches too (``hip_dense``:
 the counterparts of the reference's compiled ``_compiled_add_rms_norm`` /
 ``_compiled_swiglu``), as are the projections of decode batches (up to 64
 rows) where the HIP product is measured faster than torch's
-(``prefer_hip_linear``); the rest stay on torch (hipBLASLt). Weights are
+(``prefer_hip_linear``), with the norms, residual sums and the gate inside
+them (``mi_linear_fused``); the rest stay on torch (hipBLASLt). Weights are
 random:
 N(0, 0.02) from a seeded generator, norm weights 1, since no checkpoint is
 available to load (``init_std`` sets the spread).
@@ -33,6 +35,7 @@ from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_fused, hip_li
                                             hip_rms_norm_residual, hip_silu_mul,
                                             prefer_fused_norm, prefer_hip_linear, prefer_hip_rows,
                                             supported_rows)
+from microinfer_amd.layer.hip_paged_attention import hip_qkv_decode, supported_qkv_decode
 from microinfer_amd.layer.hip_qk_norm_rope import qk_norm_rope_append, rope_tables
 from microinfer_amd.layer.paged_attention import paged_attention_meta, varlen_attention
 
@@ -150,6 +153,15 @@ class Qwen3Model:
         """Attention output ``[T, Hq D]`` of one layer's fused QKV rows."""
         c = self.config
         tokens = qkv.shape[0]
+        if (metadata.is_decode and metadata.slots_at_end
+                and supported_qkv_decode(qkv, cache.keys, cache.values, c.num_q_head)):
+            attn = hip_qkv_decode(
+                qkv, cache.keys, cache.values, metadata.block_tables, metadata.context_lens,
+                metadata.slot_mapping, positions, q_weight=layer.q_norm, k_weight=layer.k_norm,
+                eps=c.norm_eps, cos_table=self.cos, sin_table=self.sin,
+                num_q_heads=c.num_q_head, interleaved=c.rope_interleaved,
+                plan=metadata.decode_plan(c.num_kv_head, cache.block_size))
+            return attn.reshape(tokens, c.num_q_head * c.head_dim)
         direct = metadata.is_prefill and metadata.direct_prefill
         rotated = qk_norm_rope_append(
             qkv, q_weight=layer.q_norm, k_weight=layer.k_norm, eps=c.norm_eps,
@@ -173,7 +185,7 @@ class Qwen3Model:
         hidden, residual = F.embedding(input_ids, self.embedding), None
         for layer, cache in zip(self.layers, self.caches):
             if self._fuses(layer, hidden):
-                # Five launches: each norm in front of its projection, each
+                # Five launches for a decode step: each norm in front of its projection, each
                 # residual sum and the gate behind theirs.
                 x = hidden if residual is None else hidden + residual
                 qkv = self._norm_project(x, layer.pre_norm, layer.qkv)

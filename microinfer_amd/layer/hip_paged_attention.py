@@ -243,6 +243,93 @@ def hip_paged_decode(
     return output
 
 
+def supported_qkv_decode(qkv: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
+                         num_q_heads: int) -> bool:
+    """Whether ``hip_qkv_decode`` takes these rows and caches."""
+    _, block_size, num_kv_heads, head_dim = key_cache.shape
+    aligned = all(t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1])
+                  for t in (qkv, key_cache, value_cache))
+    return (qkv.is_cuda and qkv.dtype in (torch.float16, torch.bfloat16) and qkv.dim() == 2
+            and head_dim == 128 and block_size >= 16 and _is_pow2(block_size)
+            and num_q_heads % num_kv_heads == 0 and num_q_heads // num_kv_heads <= 16
+            and qkv.stride(1) == 1 and key_cache.dtype == qkv.dtype
+            and value_cache.dtype == qkv.dtype and key_cache.stride() == value_cache.stride()
+            and key_cache.stride(-1) == 1 and 0 < qkv.shape[0] <= 4096 and aligned)
+
+
+def hip_qkv_decode(
+    qkv: torch.Tensor,
+    key_cache: torch.Tensor,
+    value_cache: torch.Tensor,
+    block_tables: torch.Tensor,
+    context_lens: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    positions: torch.Tensor,
+    *,
+    q_weight: torch.Tensor,
+    k_weight: torch.Tensor,
+    eps: float,
+    cos_table: torch.Tensor,
+    sin_table: torch.Tensor,
+    num_q_heads: int,
+    interleaved: bool = False,
+    scale: float | None = None,
+    plan: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """``qk_norm_rope_append`` and ``hip_paged_decode`` of one decode step in
+    one launch: ``qkv [R, (Hq + 2 Hkv) * D]`` -> ``[R, Hq, D]``.
+
+    ``slot_mapping`` holds each row's place ``context_lens - 1`` in its block
+    table, as the step metadata builds it; a row with another slot (a graph
+    pad row) is stored there and not attended to in this launch."""
+    if not supported_qkv_decode(qkv, key_cache, value_cache, num_q_heads):
+        raise ValueError("hip_qkv_decode: bf16/f16 rows and caches with head_dim 128, blocks of "
+                         "at least 16, aligned rows and equal cache strides are required")
+    _lib.require_device(qkv, key_cache, block_tables, context_lens, slot_mapping, positions,
+                        q_weight, k_weight, cos_table, sin_table, plan, what="hip_qkv_decode")
+    num_blocks, block_size, num_kv_heads, head_dim = key_cache.shape
+    rows = qkv.shape[0]
+    if qkv.shape[1] < (num_q_heads + 2 * num_kv_heads) * head_dim:
+        raise ValueError("qkv must be [rows, (Hq + 2 Hkv) * D]")
+    if block_tables.ndim != 2 or block_tables.shape[0] != rows:
+        raise ValueError("block_tables must have one row per request")
+    if any(t.numel() != rows for t in (context_lens, slot_mapping, positions)):
+        raise ValueError("context_lens, slot_mapping and positions need one entry per request")
+    for w in (q_weight, k_weight):
+        if w.shape != (head_dim,) or w.dtype != qkv.dtype:
+            raise ValueError("norm weights must be [head_dim] in the dtype of qkv")
+    for t in (cos_table, sin_table):
+        if t.dtype != torch.float32 or t.ndim != 2 or t.shape != (cos_table.shape[0],
+                                                                 head_dim // 2):
+            raise ValueError("cos/sin tables must be float32 [max_len, head_dim / 2]")
+    if plan is not None and (plan.dtype != torch.uint8 or not plan.is_contiguous()):
+        raise ValueError("plan must come from decode_plan()")
+    block_tables, context_lens = _index32(block_tables), _index32(context_lens)
+    slot_mapping, positions = _index32(slot_mapping), positions.long().contiguous()
+    q_weight, k_weight = q_weight.contiguous(), k_weight.contiguous()
+    cos_table, sin_table = cos_table.contiguous(), sin_table.contiguous()
+    output = torch.empty((rows, num_q_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
+    lib = _lib.load()
+    ws_bytes = decode_workspace_bytes(rows, num_q_heads, num_kv_heads, head_dim, None)
+    stream = _lib.stream_handle(qkv.device)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
+    counters = _decode_counters(qkv.device, stream, rows * num_kv_heads)
+    status = lib.mi_paged_decode_qkv(
+        qkv.data_ptr(), qkv.stride(0), q_weight.data_ptr(), k_weight.data_ptr(), float(eps),
+        cos_table.data_ptr(), sin_table.data_ptr(), cos_table.shape[0], int(bool(interleaved)),
+        positions.data_ptr(), slot_mapping.data_ptr(), key_cache.data_ptr(),
+        value_cache.data_ptr(), key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
+        block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+        context_lens.data_ptr(), output.data_ptr(), output.stride(0), output.stride(1),
+        workspace.data_ptr(), ws_bytes, counters.data_ptr(),
+        None if plan is None else plan.data_ptr(), 0 if plan is None else plan.numel(), rows,
+        num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, 0,
+        float(1.0 / math.sqrt(head_dim) if scale is None else scale),
+        _lib.dtype_code(qkv.dtype), stream)
+    _lib.check(status, "mi_paged_decode_qkv")
+    return output
+
+
 @dataclass(frozen=True)
 class PrefillPlan:
     """Launch plan of planned prefill calls (``prefill_plan``): the workspace

@@ -29,6 +29,11 @@ class AttentionMetadata:
     block_tables: torch.Tensor | None = None
     direct_prefill: bool = False
     validate_cache_write: bool = True
+    # Decode rows as StepMetadataBuilder makes them: each row's position is
+    # context_lens - 1 and its slot that place in its table (pad rows: another
+    # slot of the pad block). Then norm, RoPE, append and attention may share a
+    # launch; other slots need the append to finish first.
+    slots_at_end: bool = False
     _cu_q_cpu: tuple[int, ...] | None = field(default=None, repr=False)
     _context_lens_cpu: tuple[int, ...] | None = field(default=None, repr=False)
     _q_lens_cpu: tuple[int, ...] | None = field(default=None, repr=False)

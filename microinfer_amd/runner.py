@@ -223,13 +223,15 @@ class DecodeBuffers:
     def metadata(self, batch: int) -> AttentionMetadata:
         """Decode metadata over the first ``batch`` rows (``_make_decode_metadata``,
         microinfer/runner.py:190-197)."""
-        return AttentionMetadata.build(
+        metadata = AttentionMetadata.build(
             is_prefill=False,
             slot_mapping=self.slot_mapping[:batch],
             context_lens=self.context_lens[:batch],
             block_tables=self.block_tables[:batch],
             validate_cache_write=False,
         )
+        metadata.slots_at_end = True
+        return metadata
 
 
 class _Upload:
@@ -468,6 +470,7 @@ class StepMetadataBuilder:
             block_tables=buffers.block_tables[:n],
             validate_cache_write=self.debug_mode,
         )
+        metadata.slots_at_end = True
         if self.debug_mode:
             self.validate(seqs, buffers.input_ids[:n], buffers.positions[:n], metadata, False)
         return buffers.input_ids[:n], buffers.positions[:n], metadata
