@@ -1,0 +1,42 @@
+"""The decode plan's items and their order, against a plain restatement: parts
+of one size per sequence in slot order, dispatched largest first. Up to 64
+sequences run on the one-wave kernel, more (and forced splits) on the general
+one; both follow the same rules."""
+
+import numpy as np
+import pytest
+import torch
+
+from microinfer_amd.layer.hip_paged_attention import decode_plan
+
+pytestmark = pytest.mark.gpu
+TARGET, MIN_BLOCKS = 192, 4
+
+
+def _expected(contexts, hkv, block_size):
+    blocks = [-(-c // block_size) for c in contexts]
+    part = max(MIN_BLOCKS, 1, -(-sum(blocks) * hkv // TARGET))
+    items, slot = [], 0
+    for r in sorted(range(len(blocks)), key=lambda r: (-blocks[r], r)):
+        parts = max(1, -(-blocks[r] // part))
+        for p in range(parts):
+            end = min(blocks[r], (p + 1) * part)
+            items.append((end - p * part, slot + p,
+                          [r, p * part, end, parts, slot, contexts[r], p, 0]))
+        slot += parts
+    return [i[2] for i in sorted(items, key=lambda i: (-i[0], i[1]))]
+
+
+@pytest.mark.parametrize("hkv,block_size", [(8, 16), (1, 16), (2, 64)])
+@pytest.mark.parametrize("contexts", [
+    [1], [0, 0], [64, 65, 1], [32768], [5000, 16, 4999, 0, 16], [100] * 64,
+    list(range(1, 2049, 32)), [31 * i % 700 for i in range(65)],
+])
+def test_plan_items_and_order(contexts, hkv, block_size):
+    lens = torch.tensor(contexts, dtype=torch.int32, device="cuda")
+    width = max(-(-max(contexts) // block_size), 1)
+    plan = decode_plan(lens, num_kv_heads=hkv, block_size=block_size, block_table_width=width)
+    got = plan.cpu().numpy().view(np.int32).reshape(-1, 8)
+    want = _expected(contexts, hkv, block_size)
+    assert got[:len(want)].tolist() == want
+    assert (got[len(want):, 0] == -1).all()
