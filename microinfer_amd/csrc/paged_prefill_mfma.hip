@@ -93,14 +93,17 @@ static_assert(kWaves == 4 && kRowsPerWave % 4 == 0, "tile load mapping");
 // LDS tile layouts (LDS serves 256 bytes per clock, so an access is
 // conflict-free when each group of lanes served together covers 256
 // distinct bytes):
-//  * K: [key half][16-byte chunk][16 keys]. A K fragment read (16 lanes x
-//    16 bytes: keys k..k+15 of one half, one chunk) covers 256 contiguous
-//    bytes, and the reads of successive k-steps are 512 bytes apart, so
-//    each is one register plus an immediate offset.
-//  * V: key rows of 256 bytes, row-major, with the 16-byte chunk c of key k
-//    stored at position c ^ swz_v(k). The transposed reads (32 lanes x 8
-//    bytes: 4 consecutive keys x 4 aligned chunks) need the 4 keys' chunk
-//    groups disjoint: swz_v(k) = 4 * (k & 3).
+//  * Both: key rows of 256 bytes, row-major, as the direct loads bring them
+//    (16 neighbouring lanes take one row's 256 bytes; a layout whose loads
+//    took 16 rows at a time cost the address unit four times the cycles, 640
+//    a tile for a workgroup against 256, next to 512 of MFMA). The 16-byte
+//    chunk c of key k is stored at position c ^ swz(k).
+//  * K: a fragment read (16 lanes x 16 bytes: keys k..k+15 of one half, one
+//    chunk) needs 16 different positions: swz_k(k) = k & 15.
+//  * V: the transposed reads (32 lanes x 8 bytes: 4 consecutive keys x 4
+//    aligned chunks) need the 4 keys' chunk groups disjoint: swz_v(k) =
+//    4 * (k & 3).
+__device__ __forceinline__ int swz_k(int key) { return key & 15; }
 __device__ __forceinline__ int swz_v(int key) { return 4 * (key & 3); }
 
 // A (row block, KV head) split along its keys has at most kMaxParts
@@ -135,19 +138,6 @@ __device__ __forceinline__ BufRsrc make_buf_rsrc(const void* base) {
   r.z = -1;           // num_records
   r.w = 0x00020000;   // 32-bit data format, no swizzle
   return r;
-}
-
-// One direct buffer->LDS load of 16 bytes per lane: lane i writes LDS bytes
-// lds_dst + 16 i from rsrc + soff + voff (one wait state after the M0
-// write). Untracked by the compiler, like lds_load16.
-__device__ __forceinline__ void lds_load16_buf(BufRsrc rsrc, uint32_t soff, uint32_t voff,
-                                               const void* lds_dst) {
-  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (const __attribute__((address_space(3))) void*)(lds_dst)));
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds)
-               : "memory", "m0");
 }
 
 // Two direct buffer->LDS loads of 16 bytes per lane sharing one M0 (one
@@ -519,11 +509,9 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
   // base, 1 KiB per instruction). Waves 0-1 move the tile's first 16-key
   // half, waves 2-3 the second; each half lies in one cache block (block
   // size >= 16), so a wave's loads share one scalar base and each lane adds
-  // a constant offset. Per wave and tile, two K and two V instructions:
-  //  * K instruction j: chunks 8 (w % 2) + 4j .. +3 of the half's 16 keys
-  //    (lane i: key i % 16, chunk 8 (w % 2) + 4j + i / 16);
-  //  * V instruction j: key rows 8w + 4j .. +3 (lane i: row 8w + 4j + i / 16,
-  //    LDS chunk position i % 16, i.e. logical chunk (i % 16) ^ swz_v(row)).
+  // a constant offset. Per wave and tile, two K and two V instructions;
+  // instruction j takes key rows 8w + 4j .. +3 (lane i: row 8w + 4j + i / 16,
+  // LDS chunk position i % 16, i.e. logical chunk (i % 16) ^ swz(row)).
   const R* kc = static_cast<const R*>(a.kc);
   const R* vc = static_cast<const R*>(a.vc);
   const int32_t* trow = paged ? a.tables + req * a.t_stride : nullptr;
@@ -532,29 +520,27 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
   const int c_bs32 = static_cast<int>(a.c_bs);  // used when A32
   const bool wave_half = wave >= 2;  // which 16-key half of a tile this wave moves
   const int wrow = wave_half ? 16 : 0;
-  const int kkey = lane % 16;  // key within the half (K loads)
-  int k_ch[2], v_key[2], v_ch[2];
+  int key[2], k_ch[2], v_ch[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    k_ch[j] = 8 * (wave % 2) + 4 * j + lane / 16;
-    v_key[j] = wave * kRowsPerWave + 4 * j + lane / 16;
-    v_ch[j] = (lane % 16) ^ swz_v(v_key[j]);
+    key[j] = wave * kRowsPerWave + 4 * j + lane / 16;
+    k_ch[j] = (lane % 16) ^ swz_k(key[j]);
+    v_ch[j] = (lane % 16) ^ swz_v(key[j]);
   }
-  // LDS element offsets of the wave's instructions within a tile buffer.
-  const int k_lds = (wave_half ? 16 * kD : 0) + (8 * (wave % 2)) * 16 * 8;
-  const int v_lds = wave * kRowsPerWave * kD;
+  // LDS element offset of the wave's rows within a tile buffer.
+  const int lds_row = wave * kRowsPerWave * kD;
   // Byte offsets from the wave's half-tile base (row within the half, then
   // chunk), constant over the whole loop, so a tile's loads need no per-lane
   // address arithmetic.
   uint32_t off_k[2], off_v[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    off_k[j] = static_cast<uint32_t>((kkey * c_ts + k_ch[j] * 8) * 2);
-    off_v[j] = static_cast<uint32_t>(((v_key[j] % 16) * c_ts + v_ch[j] * 8) * 2);
+    off_k[j] = static_cast<uint32_t>(((key[j] % 16) * c_ts + k_ch[j] * 8) * 2);
+    off_v[j] = static_cast<uint32_t>(((key[j] % 16) * c_ts + v_ch[j] * 8) * 2);
   }
   // A32 paged loads are buffer loads: the head's K and V bases sit in two
   // buffer resources and a tile's block offset is the scalar soffset. The
-  // two V loads share one M0 (the second adds 1024 to both its LDS and
+  // two loads of K, and of V, share one M0 (the second adds 1024 to both its LDS and
   // memory addresses, so its lane offset is taken 1024 lower: rows 4-7 of a
   // wave's eight lie at least 4 * c_ts * 2 >= 1024 bytes into the block,
   // c_ts >= 128 being checked on the host).
@@ -602,16 +588,15 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
       if constexpr (A32) {
         const uint32_t soff = static_cast<uint32_t>(widc) * bs_bytes +
                               static_cast<uint32_t>(wt0 & (a.block_size - 1)) * ts_bytes;
-        lds_load16_buf(rsrc_k, soff, off_k[0], kbuf + k_lds);
-        lds_load16_buf(rsrc_k, soff, off_k[1], kbuf + k_lds + 4 * 16 * 8);
-        lds_load16x2_buf(rsrc_v, soff, off_v[0], off_v[1] - 1024u, vbuf + v_lds);
+        lds_load16x2_buf(rsrc_k, soff, off_k[0], off_k[1] - 1024u, kbuf + lds_row);
+        lds_load16x2_buf(rsrc_v, soff, off_v[0], off_v[1] - 1024u, vbuf + lds_row);
       } else {
         const int64_t wbase = static_cast<int64_t>(widc) * a.c_bs +
                               (wt0 & (a.block_size - 1)) * a.c_ts + head_off;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          lds_load16_sbase(kc + wbase, off_k[j], kbuf + k_lds + j * 4 * 16 * 8);
-          lds_load16_sbase(vc + wbase, off_v[j], vbuf + v_lds + j * 4 * kD);
+          lds_load16_sbase(kc + wbase, off_k[j], kbuf + lds_row + j * 4 * kD);
+          lds_load16_sbase(vc + wbase, off_v[j], vbuf + lds_row + j * 4 * kD);
         }
       }
       return mask;
@@ -620,37 +605,34 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     // instead (their scores are masked).
     if constexpr (A32) {
       // Lane offsets from the head's base.
-      const int rk = min(wt0 + kkey, kv_end - 1) + static_cast<int>(krow0);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int rv = min(t0 + v_key[j], kv_end - 1) + static_cast<int>(krow0);
-        lds_load16_sbase(kc + head_off, static_cast<uint32_t>(rk * c_ts + k_ch[j] * 8) * 2u,
-                         kbuf + k_lds + j * 4 * 16 * 8);
-        lds_load16_sbase(vc + head_off, static_cast<uint32_t>(rv * c_ts + v_ch[j] * 8) * 2u,
-                         vbuf + v_lds + j * 4 * kD);
+        const int row = min(t0 + key[j], kv_end - 1) + static_cast<int>(krow0);
+        lds_load16_sbase(kc + head_off, static_cast<uint32_t>(row * c_ts + k_ch[j] * 8) * 2u,
+                         kbuf + lds_row + j * 4 * kD);
+        lds_load16_sbase(vc + head_off, static_cast<uint32_t>(row * c_ts + v_ch[j] * 8) * 2u,
+                         vbuf + lds_row + j * 4 * kD);
       }
     } else {
       // The same from the tile's first row (64-bit scalar base; a row within
       // the tile times c_ts < 2^26 stays below 2^32 bytes).
       const int64_t tbase = (krow0 + t0) * a.c_ts + head_off;
-      const int rk = min(wt0 + kkey, kv_end - 1) - t0;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int rv = min(t0 + v_key[j], kv_end - 1) - t0;
-        lds_load16_sbase(kc + tbase, static_cast<uint32_t>(rk * c_ts + k_ch[j] * 8) * 2u,
-                         kbuf + k_lds + j * 4 * 16 * 8);
-        lds_load16_sbase(vc + tbase, static_cast<uint32_t>(rv * c_ts + v_ch[j] * 8) * 2u,
-                         vbuf + v_lds + j * 4 * kD);
+        const int row = min(t0 + key[j], kv_end - 1) - t0;
+        lds_load16_sbase(kc + tbase, static_cast<uint32_t>(row * c_ts + k_ch[j] * 8) * 2u,
+                         kbuf + lds_row + j * 4 * kD);
+        lds_load16_sbase(vc + tbase, static_cast<uint32_t>(row * c_ts + v_ch[j] * 8) * 2u,
+                         vbuf + lds_row + j * 4 * kD);
       }
     }
     return 3;
   };
 
   // Per-lane LDS element offsets of the fragment reads.
-  // K (A operand of S^T): lane reads key `col` (half col / 16, key col % 16
-  // of it), logical chunk 2*ks + half: element (col/16)*2048 +
-  // (2*ks + half)*128 + (col%16)*8 = k_rd0 + 256*ks.
-  const int k_rd0 = (col / 16) * 16 * kD + half * 16 * 8 + (col % 16) * 8;
+  // K (A operand of S^T): lane reads key `col`, logical chunk 2*ks + half at
+  // position (2*ks + half) ^ swz_k(col): one offset, xored with 16*ks.
+  const int k_rd0 = col * kD + (half ^ swz_k(col)) * 8;
   // V^T (A operand of O^T), read transposed: lane (group gq = lane / 16,
   // s = lane % 16) supplies the 8-byte row of key 16c + 8j + (gq/2)*4 + s/4 at
   // dims db*32 + (gq%2)*16 + 4*(s%4); after the transpose, lane gets
@@ -689,7 +671,7 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < kD / 16; ++ks)
-      s = M::mma(__builtin_bit_cast(vec8, load_pack<R, 8>(kbuf + k_rd0 + 256 * ks)), qf[ks], s);
+      s = M::mma(__builtin_bit_cast(vec8, load_pack<R, 8>(kbuf + (k_rd0 ^ (16 * ks)))), qf[ks], s);
     return s;
   };
 

@@ -31,8 +31,9 @@ from dataclasses import dataclass
 import torch
 from torch.nn import functional as F
 
-from microinfer_amd.layer.hip_dense import (hip_linear, hip_linear_fused, hip_linear_swiglu,
-                                            hip_rms_norm_residual, hip_silu_mul,
+from microinfer_amd.layer.hip_dense import (LINEAR_MAX_ROWS, hip_linear, hip_linear_fused,
+                                            hip_linear_swiglu, hip_rms_norm_residual,
+                                            hip_silu_mul,
                                             prefer_fused_norm, prefer_hip_linear, prefer_hip_rows,
                                             supported_rows)
 from microinfer_amd.layer.hip_paged_attention import hip_qkv_decode, supported_qkv_decode
@@ -145,7 +146,7 @@ class Qwen3Model:
         """Whether this layer's projections take its norms, gate and residual
         sums along: the HIP projections are preferred for all four."""
         rows = hidden.shape[0]
-        return (self.hip_dense and supported_rows(hidden) and layer.gate_up.shape[0] % 32 == 0
+        return (self.hip_dense and 0 < rows <= LINEAR_MAX_ROWS and supported_rows(hidden) and layer.gate_up.shape[0] % 32 == 0
                 and all(w.dtype == hidden.dtype and prefer_hip_rows(rows, w)
                         for w in (layer.qkv, layer.out, layer.gate_up, layer.down)))
 
