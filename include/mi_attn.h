@@ -361,6 +361,20 @@ int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
                      int32_t dtype, void* stream);
 
 /*
+ * mi_gather_kv with cu_seqlens_k in host memory (num_requests + 1 entries,
+ * read before the call returns; at most 64 requests): the offsets travel with
+ * the launch, so the caller uploads nothing.
+ */
+int32_t mi_gather_kv_host(const void* key_cache, const void* value_cache,
+                          int64_t cache_block_stride, int64_t cache_token_stride,
+                          int64_t cache_head_stride, const int32_t* block_tables,
+                          int64_t block_table_stride, int32_t block_table_width,
+                          const int32_t* cu_seqlens_k, int32_t num_requests,
+                          int32_t total_rows, void* key_out, void* value_out,
+                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                          int32_t num_blocks, int32_t dtype, void* stream);
+
+/*
  * Per-step index metadata, expanded on the device from a compact description
  * of the scheduled batch (all pointers device memory, int32 unless noted).
  *

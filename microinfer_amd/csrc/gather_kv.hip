@@ -9,15 +9,31 @@
 namespace mi {
 namespace {
 
+// Context offsets known on the host travel in the kernel's arguments: no
+// upload, which for pageable memory also waits for the device (6 requests of
+// 500-6000 rows: 45 us a call with it, 24 without; the kernel takes 24).
+constexpr int kHostRequests = 64;
+struct HostOffsets {
+  int32_t cu[kHostRequests + 1];
+  __device__ __forceinline__ int32_t operator[](int i) const { return cu[i]; }
+};
+// Offsets in device memory, read with scalar loads.
+struct DeviceOffsets {
+  const int32_t* cu;
+  __device__ __forceinline__ int32_t operator[](int i) const {
+    return ((__attribute__((address_space(4))) const int32_t*)(cu))[i];
+  }
+};
+
 // Rows whose words do not fit the wave kernel below, or that are not 16-byte
 // aligned: thread -> (output row, head, word). The owning request of an
 // output row is found by binary search over cu_seqlens_k (requests are few
 // and the array stays in L1/L2).
-template <typename W>
+template <typename W, typename Offsets>
 __global__ __launch_bounds__(256) void gather_kv_kernel(
     const char* __restrict__ kc, const char* __restrict__ vc, int64_t c_bs, int64_t c_ts,
     int64_t c_hs, const int32_t* __restrict__ tables, int64_t t_stride, int t_width,
-    const int32_t* __restrict__ cu_k, int num_requests, int total_rows,
+    const Offsets cu_k, int num_requests, int total_rows,
     char* __restrict__ k_out, char* __restrict__ v_out, int num_heads, int words_per_row,
     int block_size, int log2_block, int num_blocks) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -61,15 +77,14 @@ __global__ __launch_bounds__(256) void gather_kv_kernel(
 // mixed step's 43926 rows: more, shorter waves keep more loads in flight.)
 constexpr int kMaxWordsPerLane = 4;  // rows of up to 4 KiB (K or V, all heads)
 
-template <int WPL>
+template <int WPL, typename Offsets>
 __global__ __launch_bounds__(256) void gather_kv_row_kernel(
     const char* __restrict__ kc, const char* __restrict__ vc, int64_t c_bs, int64_t c_ts,
     int64_t c_hs, const int32_t* __restrict__ tables, int64_t t_stride, int t_width,
-    const int32_t* __restrict__ cu_k, int num_requests, int total_rows,
+    const Offsets cu_k, int num_requests, int total_rows,
     char* __restrict__ k_out, char* __restrict__ v_out, int num_heads, int words_per_row,
     int block_size, int log2_block, int num_blocks) {
   using ConstI32 = __attribute__((address_space(4))) const int32_t;
-  const ConstI32* cuk = (const ConstI32*)(cu_k);
   const int lane = threadIdx.x % kWave;
   const int row = __builtin_amdgcn_readfirstlane(
       static_cast<int>(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave));
@@ -78,9 +93,9 @@ __global__ __launch_bounds__(256) void gather_kv_row_kernel(
   int req = 0, hi = num_requests - 1;
   while (req < hi) {
     const int mid = (req + hi + 1) >> 1;
-    if (cuk[mid] <= row) req = mid; else hi = mid - 1;
+    if (cu_k[mid] <= row) req = mid; else hi = mid - 1;
   }
-  const int pos = row - cuk[req];
+  const int pos = row - cu_k[req];
   const int logical_block = pos >> log2_block;
   int64_t base = -1;
   if (pos >= 0 && logical_block < t_width) {
@@ -110,10 +125,10 @@ __global__ __launch_bounds__(256) void gather_kv_row_kernel(
   }
 }
 
-template <typename W>
+template <typename W, typename Offsets>
 int32_t launch_gather(const char* kc, const char* vc, int64_t c_bs, int64_t c_ts,
                       int64_t c_hs, const int32_t* tables, int64_t t_stride, int t_width,
-                      const int32_t* cu_k, int num_requests, int total_rows, char* k_out,
+                      const Offsets& cu_k, int num_requests, int total_rows, char* k_out,
                       char* v_out, int num_heads, int row_bytes, int block_size,
                       int num_blocks, hipStream_t stream) {
   const int words = row_bytes / static_cast<int>(sizeof(W));
@@ -127,34 +142,29 @@ int32_t launch_gather(const char* kc, const char* vc, int64_t c_bs, int64_t c_ts
                                          num_heads, words, block_size, ilog2(block_size),
                                          num_blocks);
       };
-      if (wpl == 1) go(gather_kv_row_kernel<1>);
-      else if (wpl == 2) go(gather_kv_row_kernel<2>);
-      else go(gather_kv_row_kernel<4>);
+      if (wpl == 1) go(gather_kv_row_kernel<1, Offsets>);
+      else if (wpl == 2) go(gather_kv_row_kernel<2, Offsets>);
+      else go(gather_kv_row_kernel<4, Offsets>);
       return check_launch("mi_gather_kv");
     }
   }
   const int64_t total = static_cast<int64_t>(total_rows) * num_heads * words;
   const int threads = 256;
   const int grid = static_cast<int>((total + threads - 1) / threads);
-  gather_kv_kernel<W><<<grid, threads, 0, stream>>>(
+  gather_kv_kernel<W, Offsets><<<grid, threads, 0, stream>>>(
       kc, vc, c_bs, c_ts, c_hs, tables, t_stride, t_width, cu_k, num_requests, total_rows,
       k_out, v_out, num_heads, words, block_size, ilog2(block_size), num_blocks);
   return check_launch("mi_gather_kv");
 }
 
-}  // namespace
-}  // namespace mi
-
-extern "C" int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
-                                int64_t cache_block_stride, int64_t cache_token_stride,
-                                int64_t cache_head_stride, const int32_t* block_tables,
-                                int64_t block_table_stride, int32_t block_table_width,
-                                const int32_t* cu_seqlens_k, int32_t num_requests,
-                                int32_t total_rows, void* key_out, void* value_out,
-                                int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
-                                int32_t num_blocks, int32_t dtype, void* stream) {
-  using namespace mi;
-  clear_error();
+template <typename Offsets>
+int32_t gather(const void* key_cache, const void* value_cache, int64_t cache_block_stride,
+               int64_t cache_token_stride, int64_t cache_head_stride,
+               const int32_t* block_tables, int64_t block_table_stride,
+               int32_t block_table_width, const Offsets& cu_k, int32_t num_requests,
+               int32_t total_rows, void* key_out, void* value_out, int32_t num_kv_heads,
+               int32_t head_dim, int32_t block_size, int32_t num_blocks, int32_t dtype,
+               void* stream) {
   if (!valid_dtype(dtype)) return fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv: bad dtype");
   if (num_requests < 0 || total_rows < 0 || num_kv_heads <= 0 || head_dim <= 0 ||
       num_blocks <= 0 || block_table_width < 0)
@@ -164,7 +174,7 @@ extern "C" int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
   if (total_rows == 0) return MI_OK;
   if (num_requests == 0)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv: rows without requests");
-  if (!key_cache || !value_cache || !block_tables || !cu_seqlens_k || !key_out || !value_out)
+  if (!key_cache || !value_cache || !block_tables || !key_out || !value_out)
     return fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv: null pointer");
   const int64_t es = static_cast<int64_t>(dtype_size(dtype));
   const int row_bytes = static_cast<int>(head_dim * es);
@@ -184,7 +194,7 @@ extern "C" int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
   char* vo = static_cast<char*>(value_out);
 #define MI_GATHER(W)                                                                    \
   launch_gather<W>(kc, vc, b_bs, b_ts, b_hs, block_tables, block_table_stride,           \
-                   block_table_width, cu_seqlens_k, num_requests, total_rows, ko, vo,    \
+                   block_table_width, cu_k, num_requests, total_rows, ko, vo,    \
                    num_kv_heads, row_bytes, block_size, num_blocks, s)
   if ((align_bits & 15u) == 0) return MI_GATHER(uint4);
   if ((align_bits & 7u) == 0) return MI_GATHER(uint2);
@@ -192,4 +202,46 @@ extern "C" int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
   if ((align_bits & 1u) == 0) return MI_GATHER(uint16_t);
 #undef MI_GATHER
   return fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv: misaligned pointers or strides");
+}
+
+}  // namespace
+}  // namespace mi
+
+extern "C" int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
+                                int64_t cache_block_stride, int64_t cache_token_stride,
+                                int64_t cache_head_stride, const int32_t* block_tables,
+                                int64_t block_table_stride, int32_t block_table_width,
+                                const int32_t* cu_seqlens_k, int32_t num_requests,
+                                int32_t total_rows, void* key_out, void* value_out,
+                                int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                int32_t num_blocks, int32_t dtype, void* stream) {
+  mi::clear_error();
+  if (total_rows > 0 && num_requests > 0 && !cu_seqlens_k)
+    return mi::fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv: null pointer");
+  return mi::gather(key_cache, value_cache, cache_block_stride, cache_token_stride,
+                    cache_head_stride, block_tables, block_table_stride, block_table_width,
+                    mi::DeviceOffsets{cu_seqlens_k}, num_requests, total_rows, key_out, value_out,
+                    num_kv_heads, head_dim, block_size, num_blocks, dtype, stream);
+}
+
+extern "C" int32_t mi_gather_kv_host(
+    const void* key_cache, const void* value_cache, int64_t cache_block_stride,
+    int64_t cache_token_stride, int64_t cache_head_stride, const int32_t* block_tables,
+    int64_t block_table_stride, int32_t block_table_width, const int32_t* cu_seqlens_k,
+    int32_t num_requests, int32_t total_rows, void* key_out, void* value_out,
+    int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t num_blocks,
+    int32_t dtype, void* stream) {
+  mi::clear_error();
+  if (num_requests > mi::kHostRequests)
+    return mi::fail(MI_ERR_UNSUPPORTED, "mi_gather_kv_host: more than 64 requests");
+  mi::HostOffsets cu{};
+  if (num_requests > 0) {
+    if (!cu_seqlens_k)
+      return mi::fail(MI_ERR_INVALID_ARGUMENT, "mi_gather_kv_host: null pointer");
+    for (int i = 0; i <= num_requests; ++i) cu.cu[i] = cu_seqlens_k[i];
+  }
+  return mi::gather(key_cache, value_cache, cache_block_stride, cache_token_stride,
+                    cache_head_stride, block_tables, block_table_stride, block_table_width, cu,
+                    num_requests, total_rows, key_out, value_out, num_kv_heads, head_dim,
+                    block_size, num_blocks, dtype, stream);
 }

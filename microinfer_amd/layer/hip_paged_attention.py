@@ -24,9 +24,9 @@ capture); the library never allocates.
 
 from __future__ import annotations
 
-from dataclasses import dataclass
-
+import ctypes
 import math
+from dataclasses import dataclass
 
 import torch
 
@@ -511,25 +511,44 @@ def hip_paged_prefill(
     return output
 
 
+GATHER_HOST_REQUESTS = 64  # offsets that fit a launch's arguments
+
+
 def hip_gather_kv(key_cache, value_cache, block_tables, cu_seqlens_k, total_rows: int):
     """One-launch gather of each request's valid rows into contiguous K/V."""
-    _lib.require_device(key_cache, value_cache, block_tables, cu_seqlens_k, what="gather_kv")
+    _lib.require_device(cu_seqlens_k, what="gather_kv")
+    cu_seqlens_k = _index32(cu_seqlens_k)
+    return _gather(key_cache, value_cache, block_tables, total_rows, _lib.load().mi_gather_kv,
+                   cu_seqlens_k.data_ptr())
+
+
+def hip_gather_kv_host(key_cache, value_cache, block_tables, offsets: list[int]):
+    """``hip_gather_kv`` with the ``cu_seqlens_k`` of at most 64 requests on the
+    host: nothing is uploaded and nothing waited for."""
+    if len(offsets) - 1 > GATHER_HOST_REQUESTS or offsets[-1] > 2 ** 31 - 1:
+        raise ValueError("hip_gather_kv_host: at most 64 requests and int32 offsets")
+    host = (ctypes.c_int32 * len(offsets))(*offsets)
+    return _gather(key_cache, value_cache, block_tables, offsets[-1],
+                   _lib.load().mi_gather_kv_host, ctypes.addressof(host))
+
+
+def _gather(key_cache, value_cache, block_tables, total_rows, entry, offsets):
+    _lib.require_device(key_cache, value_cache, block_tables, what="gather_kv")
     key_cache, value_cache = _check_caches(key_cache, value_cache)
     num_blocks, block_size, num_kv_heads, head_dim = key_cache.shape
     if not _is_pow2(block_size):
         raise ValueError("paged kernels require a power-of-two block size")
     block_tables = _index32(block_tables)
-    cu_seqlens_k = _index32(cu_seqlens_k)
     shape = (total_rows, num_kv_heads, head_dim)
     keys = torch.empty(shape, dtype=key_cache.dtype, device=key_cache.device)
     values = torch.empty_like(keys)
     if total_rows == 0:
         return keys, values
-    status = _lib.load().mi_gather_kv(
+    status = entry(
         key_cache.data_ptr(), value_cache.data_ptr(),
         key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
         block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
-        cu_seqlens_k.data_ptr(), block_tables.shape[0], total_rows,
+        offsets, block_tables.shape[0], total_rows,
         keys.data_ptr(), values.data_ptr(), num_kv_heads, head_dim, block_size, num_blocks,
         _lib.dtype_code(key_cache.dtype), _lib.stream_handle(key_cache.device),
     )

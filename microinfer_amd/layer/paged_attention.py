@@ -22,11 +22,16 @@ import math
 import torch
 
 from microinfer_amd.layer.hip_paged_attention import (
+    GATHER_HOST_REQUESTS,
     hip_gather_kv,
+    hip_gather_kv_host,
     hip_paged_decode,
     hip_paged_prefill,
 )
 from microinfer_amd.layer.metadata import AttentionMetadata
+
+
+_INT32_MAX = 2 ** 31 - 1
 
 
 def gather_paged_kv(key_cache, value_cache, block_tables, contexts, block_size):
@@ -46,8 +51,11 @@ def gather_paged_kv(key_cache, value_cache, block_tables, contexts, block_size):
     offsets = [0]
     for length in contexts:
         offsets.append(offsets[-1] + length)
+    tables = block_tables[: len(contexts)]
+    if len(contexts) <= GATHER_HOST_REQUESTS and offsets[-1] <= _INT32_MAX:
+        return hip_gather_kv_host(key_cache, value_cache, tables, offsets)
     cu_k = torch.tensor(offsets, dtype=torch.int32, device=key_cache.device)
-    return hip_gather_kv(key_cache, value_cache, block_tables[: len(contexts)], cu_k, offsets[-1])
+    return hip_gather_kv(key_cache, value_cache, tables, cu_k, offsets[-1])
 
 
 # The reference's name (paged_attention.py:76), for callers bound to it.

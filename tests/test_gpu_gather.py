@@ -101,3 +101,25 @@ def test_gather_rejects_short_tables():
     with pytest.raises(ValueError):
         gather_paged_kv(cache.keys[0], cache.values[0],
                         torch.tensor([[0]], dtype=torch.int32, device=DEV), [5], 4)
+
+
+@pytest.mark.parametrize("requests", [1, 64, 65])
+def test_gather_host_and_device_offsets_agree(requests):
+    # Up to 64 requests' offsets travel with the launch, more are uploaded.
+    contexts = [(7 * i) % 40 for i in range(requests)]
+    contexts[-1] = 33
+    need = [-(-c // 16) for c in contexts]
+    gen = torch.Generator().manual_seed(requests)
+    ids = torch.randperm(sum(need) + 1, generator=gen)
+    tables = torch.full((requests, 3), -1, dtype=torch.int32)
+    at = 0
+    for r, n in enumerate(need):
+        tables[r, :n] = ids[at:at + n]
+        at += n
+    kc, vc = (torch.randn(sum(need) + 1, 16, 2, 64, generator=gen).to(DEV) for _ in range(2))
+    cu = torch.tensor([0, *np.cumsum(contexts)], dtype=torch.int32, device=DEV)
+    want = hip_gather_kv(kc, vc, tables.to(DEV), cu, sum(contexts))
+    got = gather_paged_kv(kc, vc, tables.to(DEV), contexts, 16)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+    oracle = oracle_gather(bits(kc), bits(vc), tables.numpy(), contexts, 16)
+    assert np.array_equal(bits(got[0]), oracle[0]) and np.array_equal(bits(got[1]), oracle[1])
