@@ -64,8 +64,9 @@ int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
  * it differs from mi_rms_norm_residual + mi_linear by that pair's second
  * rounding. The projection's sum is rounded to the element type before the
  * residual is added and the result rounded again, as x + F.linear(...) does;
- * residual may be NULL and may be y itself. norm_weight may be NULL. Shapes,
- * alignment and limits are those of mi_linear / mi_linear_swiglu.
+ * residual may be NULL and may be y itself. norm_weight may be NULL: then m may
+ * be up to 4096. Shapes, alignment and other limits are those of mi_linear /
+ * mi_linear_swiglu.
  */
 int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
                         const void* w, int64_t w_row_stride, const void* residual,

@@ -1,5 +1,5 @@
-// Dense projections of the decoder layer at decode batch sizes on gfx950:
-// y = x . w^T for m <= 64 rows, with the layer's RMSNorm in front of it, the
+// Dense projections of the decoder layer on gfx950, at decode batch sizes and
+// those of short prefill steps: y = x . w^T, with the layer's RMSNorm in front of it, the
 // SwiGLU gate or the residual sum behind it (entry points in
 // include/mi_model.h).
 //
@@ -53,6 +53,10 @@ struct LinMfma<F16> {
 };
 
 constexpr int kLinMaxRows = 64;
+constexpr int kLinMaxFusedRows = 4096;  // mi_linear_fused without a norm
+// s_waitcnt immediate that waits for vmcnt <= n only (vmcnt bits 3:0 and
+// 15:14, the other counters at their maxima).
+constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kLinStep = 32;  // k per MFMA
 
 struct LinArgs {
@@ -103,31 +107,35 @@ __device__ __forceinline__ uint16_t add_residual(uint16_t y, uint16_t res) {
 // ---------------------------------------------------------------------------
 // MFMA kernel.
 // ---------------------------------------------------------------------------
-constexpr int kChunk = 128;  // k per staged chunk (four MFMA steps)
-constexpr int kChunkSteps = kChunk / kLinStep;
-constexpr int kRowBytes = kChunk * 2;    // one row of a chunk: 256 bytes
-constexpr int kTileBytes = 16 * kRowBytes;
-
-// NW waves split k by chunks (wave w: a contiguous range); NT 16-column tiles
-// per workgroup (GLU: tile 0 is gate columns, tile 1 the matching up columns);
-// MT 16-row tiles of x per workgroup, row groups of one column tile on one XCD.
-// S LDS slots of one chunk per wave.
+// NW waves split k by chunks of KC (wave w: a contiguous range); NT 16-column
+// tiles per workgroup (GLU: the first half gate columns, the second the
+// matching up columns); MT 16-row tiles of x per workgroup, row groups of one
+// column tile on one XCD. S LDS slots of one chunk per wave.
 //
 // A wave stages its chunks of w and x in its own LDS slots with direct
-// global->LDS loads, four rows of 256 bytes per instruction, and reads the
+// global->LDS loads, 1 KiB of whole chunk rows per instruction, and reads the
 // MFMA fragments from there. Loading the fragments straight into registers
 // puts 16 different rows in 16 neighbouring lanes, and the address unit then
 // takes about 64 cycles per instruction instead of 16: at 64 rows that alone
 // was 4.1 of the 7.1 us of a 4096 x 1024 projection.
-// LDS rows are 256 bytes; 16-byte piece c of row r sits at place c ^ (r & 15),
-// which makes the fragment reads free of bank conflicts.
-template <typename E, int NW, int NT, int MT, int S, bool GLU, bool NORM>
+// 16-byte piece c of row r sits at place c ^ swz(r): with rows of 256 bytes
+// (KC 128) swz = r & 15, of 128 bytes (KC 64, two rows to a bank cycle)
+// (r >> 1) & 7, either of which leaves a fragment read (16 rows, one piece)
+// without bank conflicts.
+template <typename E, int NW, int NT, int MT, int S, int KC, bool GLU, bool NORM>
 __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
   using M = LinMfma<E>;
   using vec8 = typename M::vec8;
   using R = uint16_t;
-  static_assert(!GLU || NT == 2, "GLU launches: gate and up tiles");
-  constexpr int kUnits = GLU ? MT : NT * MT;  // result tiles to add up and store
+  static_assert(!GLU || NT % 2 == 0, "GLU launches: gate and up tiles");
+  constexpr int kOut = GLU ? NT / 2 : NT;  // 16-column tiles of y
+  constexpr int kUnits = kOut * MT;        // result tiles to add up and store
+  constexpr int kChunkSteps = KC / kLinStep;
+  constexpr int kRowBytes = KC * 2;
+  constexpr int kTileBytes = 16 * kRowBytes;
+  constexpr int kPieces = KC / 8;               // 16-byte pieces of a row
+  constexpr int kLoadRows = kWave / kPieces;    // rows per load
+  constexpr int kLoads = 16 / kLoadRows;        // loads per tile
   constexpr int kSlot = (NT + MT) * kTileBytes;
   constexpr int kSums = NW * NT * MT * kWave * 16;
   constexpr int kRing = NW * S * kSlot;
@@ -141,9 +149,9 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
   const int quad = lane / 16;  // 8-element group of the k-step
   const int xcd = blockIdx.x % 8, rest = blockIdx.x / 8;
   const int r0 = 16 * MT * (rest % a.row_groups);
-  const int n0 = (rest / a.row_groups * 8 + xcd) * (GLU ? 16 : 16 * NT);
+  const int n0 = (rest / a.row_groups * 8 + xcd) * (16 * kOut);
   if (n0 >= (GLU ? a.inter : a.n)) return;
-  const int chunks = (a.k + kChunk - 1) / kChunk;
+  const int chunks = (a.k + KC - 1) / KC;
   const int per_wave = (chunks + NW - 1) / NW;
   const int c_begin = min(wave * per_wave, chunks);
   const int c_end = min(c_begin + per_wave, chunks);
@@ -157,42 +165,44 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
     for (int u = 0; u < NT; ++u) acc[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  // Load i of a tile takes its rows 4 i .. 4 i + 3; lane / 16 is the row of
-  // them, lane % 16 the place in it. n % 16 == 0: a tile's columns exist or
-  // none do (then tile 0 is read in its place). Rows of x past m repeat the
-  // last one; their results are not stored.
-  const R* src[(NT + MT) * 4];
-  int piece[4];
+  // Load i of a tile takes its rows kLoadRows i ..; lane / kPieces is the row
+  // of them, lane % kPieces the place in it. n % 16 == 0: a tile's columns
+  // exist or none do (then tile 0 is read in its place). Rows of x past m
+  // repeat the last one; their results are not stored.
+  auto swz = [](int row) { return KC == 128 ? row & 15 : (row >> 1) & 7; };
+  const R* src[(NT + MT) * kLoads];
+  int piece[kLoads];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 4 * i + quad;
-    piece[i] = (col ^ row) * 8;
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = kLoadRows * i + lane / kPieces;
+    piece[i] = (lane % kPieces ^ swz(row)) * 8;
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      const int wr = GLU ? u * a.inter + n0 : (n0 + 16 * u < a.n ? n0 + 16 * u : n0);
-      src[u * 4 + i] = static_cast<const R*>(a.w) + static_cast<int64_t>(wr + row) * a.ws;
+      const int c = n0 + 16 * (u % kOut);
+      const int wr = (c < (GLU ? a.inter : a.n) ? c : n0) + u / kOut * a.inter;
+      src[u * kLoads + i] = static_cast<const R*>(a.w) + static_cast<int64_t>(wr + row) * a.ws;
     }
 #pragma unroll
     for (int t = 0; t < MT; ++t)
-      src[(NT + t) * 4 + i] = static_cast<const R*>(a.x) +
-                              static_cast<int64_t>(min(r0 + 16 * t + row, a.m - 1)) * a.xs;
+      src[(NT + t) * kLoads + i] = static_cast<const R*>(a.x) +
+                                   static_cast<int64_t>(min(r0 + 16 * t + row, a.m - 1)) * a.xs;
   }
   char* ring = s_mem + wave * S * kSlot;
   auto issue = [&](int slot, int c) {
     char* dst = ring + slot * kSlot;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
       // A last chunk may end early: pieces past the row read its start.
-      int off = c * kChunk + piece[i];
+      int off = c * KC + piece[i];
       off = off < a.k ? off : 0;
 #pragma unroll
       for (int t = 0; t < NT + MT; ++t)
-        lds_load16(src[t * 4 + i] + off, dst + t * kTileBytes + i * 4 * kRowBytes);
+        lds_load16(src[t * kLoads + i] + off, dst + t * kTileBytes + i * 1024);
     }
   };
   auto fragment = [&](const char* tile, int step) {
     return *reinterpret_cast<const Pack<R, 8>*>(tile + col * kRowBytes +
-                                                (((4 * step + quad) ^ col) * 16));
+                                                (((4 * step + quad) ^ swz(col)) * 16));
   };
   const R* nrow = static_cast<const R*>(a.norm) + quad * 8;
   if (c_begin < c_end) {
@@ -204,19 +214,19 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
       if constexpr (NORM) {
 #pragma unroll
         for (int j = 0; j < kChunkSteps; ++j) {
-          const int off = c * kChunk + j * kLinStep;
+          const int off = c * KC + j * kLinStep;
           g[j] = load_pack<R, 8>(nrow + (off < a.k ? off : 0));
         }
       }
       // Chunk c is in its slot once at most the younger one is in flight
       // (and the norm weights, which were issued last).
       if (!NORM && S > 1 && c + 1 < c_end)
-        __builtin_amdgcn_s_waitcnt(0x0F70 | (4 * (NT + MT) & 15) | ((4 * (NT + MT) >> 4) << 14));
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(kLoads * (NT + MT)));
       else
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       const char* cur = ring + slot * kSlot;
-      const int steps = min(kChunkSteps, (a.k - c * kChunk) / kLinStep);
+      const int steps = min(kChunkSteps, (a.k - c * KC) / kLinStep);
 #pragma unroll
       for (int j = 0; j < kChunkSteps; ++j) {
         if (j >= steps) break;  // uniform
@@ -268,13 +278,13 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
   for (int i = 0; i < (kUnits + NW - 1) / NW; ++i) {
     const int unit = wave + i * NW;
     if (unit >= kUnits) break;
-    const int t = unit % MT, u = unit / MT;  // GLU: u = 0
+    const int t = unit % MT, u = unit / MT;
     f32x4_t v = sum_at(0, unit), up = {};
-    if constexpr (GLU) up = sum_at(0, MT + unit);
+    if constexpr (GLU) up = sum_at(0, kUnits + unit);
 #pragma unroll
     for (int wv = 1; wv < NW; ++wv) {
       v += sum_at(wv, unit);
-      if constexpr (GLU) up += sum_at(wv, MT + unit);
+      if constexpr (GLU) up += sum_at(wv, kUnits + unit);
     }
     if constexpr (NORM) {
       float sum = 0.f;
@@ -286,7 +296,7 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
     }
     const int r = r0 + 16 * t + col;
     const int c = n0 + 16 * u + 4 * quad;
-    if (r >= a.m || (!GLU && n0 + 16 * u >= a.n)) continue;
+    if (r >= a.m || n0 + 16 * u >= (GLU ? a.inter : a.n)) continue;
     Pack<R, 4> out;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -400,32 +410,34 @@ __global__ __launch_bounds__(kGemvWaves* kWave) void gemv_kernel(const LinArgs a
 // ---------------------------------------------------------------------------
 // Dispatch.
 // ---------------------------------------------------------------------------
-template <typename E, int NW, int NT, int MT, int S, bool GLU, bool NORM>
+template <typename E, int NW, int NT, int MT, int S, int KC, bool GLU, bool NORM>
 void launch_mfma(LinArgs a, hipStream_t stream) {
+  constexpr int kCols = 16 * (GLU ? NT / 2 : NT);
   a.row_groups = (a.m + 16 * MT - 1) / (16 * MT);
-  const int col_tiles = GLU ? a.inter / 16 : (a.n + 16 * NT - 1) / (16 * NT);
+  const int col_tiles = ((GLU ? a.inter : a.n) + kCols - 1) / kCols;
   const dim3 grid(static_cast<uint32_t>((col_tiles + 7) / 8 * 8 * a.row_groups));
-  linear_kernel<E, NW, NT, MT, S, GLU, NORM><<<grid, NW * kWave, 0, stream>>>(a);
+  linear_kernel<E, NW, NT, MT, S, KC, GLU, NORM><<<grid, NW * kWave, 0, stream>>>(a);
 }
 
 // Two slots per wave while every workgroup has a CU to itself (4096 x 1024 at
 // 64 rows: 4.5 us, 4.9 with one), else one slot and more workgroups per CU
 // (24576 x 4096 at 32 rows: 40.7, 41.6 with two). With the norm, whose weights
 // are waited for with the chunk, one slot.
+// Past 64 rows four waves always: a launch has workgroups enough.
 template <typename E, int NT, int MT, bool GLU, bool NORM>
 void launch_tile(const LinArgs& a, bool eight, bool alone, hipStream_t stream) {
   if (eight) {
     if constexpr (MT <= 2) {
       if constexpr (NT == 1 && MT == 1 && !NORM) {
-        if (alone) return launch_mfma<E, 8, NT, MT, 2, GLU, NORM>(a, stream);
+        if (alone) return launch_mfma<E, 8, NT, MT, 2, 128, GLU, NORM>(a, stream);
       }
-      return launch_mfma<E, 8, NT, MT, 1, GLU, NORM>(a, stream);
+      return launch_mfma<E, 8, NT, MT, 1, 128, GLU, NORM>(a, stream);
     }
   } else {
     if constexpr (MT <= 2 && !NORM) {
-      if (alone) return launch_mfma<E, 4, NT, MT, 2, GLU, NORM>(a, stream);
+      if (alone) return launch_mfma<E, 4, NT, MT, 2, 128, GLU, NORM>(a, stream);
     }
-    return launch_mfma<E, 4, NT, MT, 1, GLU, NORM>(a, stream);
+    return launch_mfma<E, 4, NT, MT, 1, 128, GLU, NORM>(a, stream);
   }
 }
 
@@ -434,21 +446,24 @@ void launch_tile(const LinArgs& a, bool eight, bool alone, hipStream_t stream) {
 // (workgroups per CU, rounded up) x (NT + MT). Measured against the others
 // (us): 4096 x 1024 at 64 rows 2 x 2 4.5, 1 x 1 6.0, 1 x 2 7.0; 2048 x 6144 at
 // 48 rows 1 x 2 11.2, 1 x 1 14.7, 2 x 2 15.0; 24576 x 4096 at 48 rows 2 x 3 45,
-// 2 x 2 55.
+// 2 x 2 55; past 64 rows, 4096 x 1024 at 128 rows 2 x 2 5.9, 4 x 4 8.6, at 333
+// rows 4 x 4 9.7, 2 x 2 12.3.
 struct LinTile {
   int nt, mt;
   bool alone;  // at most one workgroup per CU
 };
 LinTile pick_tile(const LinArgs& a, bool glu, bool eight) {
-  static constexpr int kTiles[][2] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {2, 3}};
+  static constexpr int kTiles[][2] = {{1, 1}, {2, 1}, {1, 2}, {2, 2}, {2, 3}, {4, 4}};
   const int cus = device_cus(), rows = (a.m + 15) / 16;
   LinTile best{0, 0, false};
   int64_t best_cost = 0;
   for (const auto& t : kTiles) {
     const int nt = t[0], mt = t[1];
-    if (mt > rows || (glu && nt != 2) || (!glu && nt == 2 && mt == 1) || (eight && mt == 3))
+    if (mt > rows || (glu && nt < 2) || (!glu && nt == 2 && mt == 1) || (eight && mt == 3) ||
+        (nt == 4 && a.m <= kLinMaxRows))
       continue;
-    const int64_t cols = glu ? a.inter / 16 : (a.n + 16 * nt - 1) / (16 * nt);
+    const int64_t cols =
+        glu ? (a.inter + 8 * nt - 1) / (8 * nt) : (a.n + 16 * nt - 1) / (16 * nt);
     const int64_t groups = cols * ((rows + mt - 1) / mt);
     const int64_t cost = (groups + cus - 1) / cus * (nt + mt);
     if (best.nt == 0 || cost < best_cost) {
@@ -464,13 +479,18 @@ void launch_many_rows(const LinArgs& a, hipStream_t stream) {
   // Narrow outputs: eight waves per tile (1024 x 3072 at 8 rows: 4.35 us, 4.68
   // with four); wider ones have workgroups enough (4096 x 1024: 3.9, 3.7 with
   // four). By n alone, so that the fused gate sums as the projection does.
-  const bool eight = a.n < 4096;
+  const bool eight = a.n < 4096 && a.m <= kLinMaxRows;
   const LinTile t = pick_tile(a, GLU, eight);
   if constexpr (!GLU) {
     if (t.nt == 1 && t.mt == 1) return launch_tile<E, 1, 1, GLU, NORM>(a, eight, t.alone, stream);
     if (t.nt == 1) return launch_tile<E, 1, 2, GLU, NORM>(a, eight, t.alone, stream);
   } else if (t.mt == 1) {
     return launch_tile<E, 2, 1, GLU, NORM>(a, eight, t.alone, stream);
+  }
+  if constexpr (!NORM) {
+    // Chunks of 64 and one slot: two workgroups share a CU (4096 x 1024 at 520
+    // rows 14.9 us, 20.9 with two slots).
+    if (t.mt == 4) return launch_mfma<E, 4, 4, 4, 1, 64, GLU, NORM>(a, stream);
   }
   if (t.mt == 2) return launch_tile<E, 2, 2, GLU, NORM>(a, eight, t.alone, stream);
   return launch_tile<E, 2, 3, GLU, NORM>(a, eight, t.alone, stream);
@@ -507,7 +527,8 @@ void launch_typed(const LinArgs& a, hipStream_t stream) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-int32_t linear(const char* who, const LinArgs& a, bool swiglu, int32_t dtype, void* stream) {
+int32_t linear(const char* who, const LinArgs& a, bool swiglu, int32_t max_rows, int32_t dtype,
+               void* stream) {
   clear_error();
   const std::string fn(who);
   if (!valid_dtype(dtype)) return fail(MI_ERR_INVALID_ARGUMENT, fn + ": bad dtype");
@@ -516,7 +537,8 @@ int32_t linear(const char* who, const LinArgs& a, bool swiglu, int32_t dtype, vo
     return fail(MI_ERR_INVALID_ARGUMENT,
                 fn + ": need m >= 0, the output width a positive multiple of 16, k of 32");
   if (dtype == MI_DTYPE_F32) return fail(MI_ERR_UNSUPPORTED, fn + ": 16-bit types only");
-  if (a.m > kLinMaxRows) return fail(MI_ERR_UNSUPPORTED, fn + ": m above 64");
+  if (a.m > max_rows)
+    return fail(MI_ERR_UNSUPPORTED, fn + ": m above " + std::to_string(max_rows));
   if (a.m == 0) return MI_OK;
   if (!a.x || !a.w || !a.y) return fail(MI_ERR_INVALID_ARGUMENT, fn + ": null pointer");
   if (a.xs < a.k || a.ws < a.k || a.ys < out || (a.res && a.rs < out))
@@ -556,7 +578,7 @@ extern "C" int32_t mi_linear(const void* x, int64_t x_row_stride, const void* w,
   a.m = m;
   a.n = n;
   a.k = k;
-  return mi::linear("mi_linear", a, false, dtype, stream);
+  return mi::linear("mi_linear", a, false, mi::kLinMaxRows, dtype, stream);
 }
 
 extern "C" int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
@@ -574,7 +596,7 @@ extern "C" int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const v
   a.n = 2 * inter;
   a.inter = inter;
   a.k = k;
-  return mi::linear("mi_linear_swiglu", a, true, dtype, stream);
+  return mi::linear("mi_linear_swiglu", a, true, mi::kLinMaxRows, dtype, stream);
 }
 
 extern "C" int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const void* norm_weight,
@@ -601,5 +623,6 @@ extern "C" int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const vo
     mi::clear_error();
     return mi::fail(MI_ERR_INVALID_ARGUMENT, "mi_linear_fused: gate/up needs an even n");
   }
-  return mi::linear("mi_linear_fused", a, swiglu != 0, dtype, stream);
+  return mi::linear("mi_linear_fused", a, swiglu != 0,
+                    norm_weight ? mi::kLinMaxRows : mi::kLinMaxFusedRows, dtype, stream);
 }

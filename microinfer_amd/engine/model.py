@@ -33,9 +33,8 @@ from torch.nn import functional as F
 
 from microinfer_amd.layer.hip_dense import (LINEAR_MAX_ROWS, hip_linear, hip_linear_fused,
                                             hip_linear_swiglu, hip_rms_norm_residual,
-                                            hip_silu_mul,
-                                            prefer_fused_norm, prefer_hip_linear, prefer_hip_rows,
-                                            supported_rows)
+                                            hip_silu_mul, prefer_fused_norm, prefer_hip_linear,
+                                            prefer_hip_prefill, prefer_hip_rows, supported_rows)
 from microinfer_amd.layer.hip_paged_attention import hip_qkv_decode, supported_qkv_decode
 from microinfer_amd.layer.hip_qk_norm_rope import qk_norm_rope_append, rope_tables
 from microinfer_amd.layer.paged_attention import paged_attention_meta, varlen_attention
@@ -117,8 +116,11 @@ class Qwen3Model:
         return F.rms_norm(combined, (combined.shape[-1],), weight, self.config.norm_eps), combined
 
     def _linear(self, x, weight):
-        if self.hip_dense and prefer_hip_linear(x, weight):
-            return hip_linear(x, weight)
+        if self.hip_dense:
+            if prefer_hip_linear(x, weight):
+                return hip_linear(x, weight)
+            if x.shape[0] > LINEAR_MAX_ROWS and prefer_hip_prefill(x, weight):
+                return hip_linear_fused(x, weight)
         return F.linear(x, weight)
 
     def _swiglu(self, gate_up):
@@ -130,8 +132,11 @@ class Qwen3Model:
     def _ffn_gate(self, x, gate_up):
         """SwiGLU of the gate/up projection: one fused launch where the HIP
         projection is preferred, else the projection and then the gate."""
-        if self.hip_dense and prefer_hip_linear(x, gate_up) and gate_up.shape[0] % 32 == 0:
-            return hip_linear_swiglu(x, gate_up)
+        if self.hip_dense and gate_up.shape[0] % 32 == 0:
+            if prefer_hip_linear(x, gate_up):
+                return hip_linear_swiglu(x, gate_up)
+            if x.shape[0] > LINEAR_MAX_ROWS and prefer_hip_prefill(x, gate_up):
+                return hip_linear_fused(x, gate_up, swiglu=True)
         return self._swiglu(self._linear(x, gate_up))
 
     def _norm_project(self, x, norm_weight, weight, swiglu=False):

@@ -21,6 +21,7 @@ from microinfer_amd import _lib
 
 _HALF = (torch.bfloat16, torch.float16)
 LINEAR_MAX_ROWS = 64
+FUSED_MAX_ROWS = 4096  # hip_linear_fused without a norm
 
 
 def _rows_aligned(t: torch.Tensor) -> bool:
@@ -29,9 +30,10 @@ def _rows_aligned(t: torch.Tensor) -> bool:
             and (t.stride(0) * es) % 16 == 0)
 
 
-def supported_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def supported_linear(x: torch.Tensor, weight: torch.Tensor,
+                     max_rows: int = LINEAR_MAX_ROWS) -> bool:
     return (x.is_cuda and x.dtype in _HALF and weight.dtype == x.dtype and x.dim() == 2
-            and weight.dim() == 2 and 0 < x.shape[0] <= LINEAR_MAX_ROWS
+            and weight.dim() == 2 and 0 < x.shape[0] <= max_rows
             and x.shape[1] == weight.shape[1] and weight.shape[0] % 16 == 0
             and x.shape[1] % 32 == 0 and _rows_aligned(x) and _rows_aligned(weight))
 
@@ -57,6 +59,20 @@ def prefer_hip_rows(rows: int, weight: torch.Tensor) -> bool:
     return (0 < rows <= LINEAR_MAX_ROWS and weight.is_cuda and weight.dtype in _HALF
             and weight.dim() == 2 and weight.shape[0] % 16 == 0 and weight.shape[1] % 32 == 0
             and _rows_aligned(weight) and _measured_faster(rows, weight))
+
+
+def prefer_hip_prefill(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``hip_linear_fused`` (no norm) beats torch's product past 64 rows.
+
+    Measured (us, HIP against hipBLASLt): 4096 x 1024 at 128 / 256 / 333 / 520
+    rows 5.9 / 8.7 / 9.7 / 14.9 against 9.4 / 9.1 / 10.0 / 13.1; 1024 x 3072 7.0
+    / 7.2 / 10.7 / 15 against 8.1 / 8.9 / 11.9 / 13.8; 6144 x 1024 with the gate
+    8.7 / 10.3 / 16.3 / 18.7 against 13.6 / 16.9 / 17.7 / 18.6 without it. Past
+    about 600 rows, and for larger weights, the library's tiles win. A call
+    also takes half the host time of torch's (9 against 18 us), which bounds
+    eager prefill steps of this size."""
+    return (x.shape[0] <= 640 and weight.shape[0] * weight.shape[1] <= 1 << 23
+            and supported_linear(x, weight, FUSED_MAX_ROWS))
 
 
 def prefer_fused_norm(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -123,8 +139,9 @@ def hip_linear_fused(x: torch.Tensor, weight: torch.Tensor, *,
     applied to the float32 sum; the other roundings are those of the separate
     calls."""
     _lib.require_device(x, weight, norm_weight, residual, what="fused projection")
-    if not supported_linear(x, weight) or (swiglu and weight.shape[0] % 32):
-        raise ValueError("hip_linear_fused: x [m <= 64, k] and weight [n % 16 == 0, k % 32 == 0] "
+    limit = FUSED_MAX_ROWS if norm_weight is None else LINEAR_MAX_ROWS
+    if not supported_linear(x, weight, limit) or (swiglu and weight.shape[0] % 32):
+        raise ValueError("hip_linear_fused: x [m <= 4096 (64 with a norm), k] and weight [n % 16 == 0, k % 32 == 0] "
                          "(gate/up: n % 32 == 0) of one 16-bit dtype with 16-byte aligned rows "
                          "are required")
     m, k = x.shape

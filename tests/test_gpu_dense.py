@@ -231,6 +231,24 @@ def test_linear_fused_is_norm_projection_and_sum(dtype, m, n, k):
         assert bool(((got - want).abs() <= bound + 1e-6).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [65, 128, 200, 333, 641])
+@pytest.mark.parametrize("n,k", [(4096, 1024), (1024, 3072), (6144, 1024), (48, 64), (2080, 160)])
+def test_linear_fused_past_64_rows(dtype, m, n, k):
+    torch.manual_seed(m * 13 + n + k)
+    x = torch.randn(m, k, device=DEV).to(dtype)
+    w = (0.05 * torch.randn(n, k, device=DEV)).to(dtype)
+    r = torch.randn(m, n, device=DEV).to(dtype)
+    y = hip_linear_fused(x, w)
+    _assert_close(y, _reference(x, w))
+    assert torch.equal(hip_linear_fused(x, w, residual=r), r + y)
+    if n % 32 == 0:
+        gate, up = _reference(x, w).chunk(2, dim=-1)
+        ref = F.silu(gate) * up
+        err = (hip_linear_fused(x, w, swiglu=True).float() - ref).abs()
+        assert bool((err <= 2.5e-2 * ref.abs() + 2e-3 * ref.abs().max() + 1e-6).all())
+
+
 def test_linear_fused_rejects():
     x = torch.randn(8, 1024, device=DEV).to(torch.bfloat16)
     w = torch.randn(64, 1024, device=DEV).to(torch.bfloat16)
@@ -240,3 +258,6 @@ def test_linear_fused_rejects():
         hip_linear_fused(x, w, residual=torch.zeros(8, 32, device=DEV, dtype=torch.bfloat16))
     with pytest.raises(ValueError):
         hip_linear_fused(x, w[:48], swiglu=True)
+    with pytest.raises(ValueError):
+        hip_linear_fused(torch.zeros(65, 1024, device=DEV, dtype=torch.bfloat16), w,
+                         norm_weight=torch.ones(1024, device=DEV, dtype=torch.bfloat16))
