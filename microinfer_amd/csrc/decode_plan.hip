@@ -6,7 +6,7 @@
 // (microinfer/layer/triton_paged_attention.py:342-349) and stripes tiles over
 // the splits (:76-79). Here partitions are contiguous block ranges sized from
 // the step's total context: about kTargetItems (item, KV head) workgroups of
-// at least kMinPartBlocks blocks each. A sequence's partitions occupy
+// at least kMinPartBlocks blocks each; short sequences stay whole. A sequence's partitions occupy
 // consecutive slots (first_item + part: where their partials go), but the
 // launch dispatches items largest first, whatever their sequence: the
 // hardware does not start a later workgroup on a CU that an early small item
@@ -18,11 +18,27 @@
 namespace mi {
 namespace {
 
-// About this many (item, KV head) workgroups per launch, each covering at
-// least kMinPartBlocks cache blocks. Fixed: the plan's size, and so the
-// workspace a caller sizes, depends only on the call's arguments.
+// About this many (item, KV head) workgroups per launch. Fixed: the plan's
+// size, and so the workspace a caller sizes, depends only on the call's
+// arguments.
 constexpr int32_t kTargetItems = 192;
+// Merging partitions costs a launch about 2.5 us and more with their number,
+// so a part covers at least kMinPartBlocks cache blocks, and an eighth of the
+// longest sequence up to kMaxMinPart (one sequence of 2000 tokens, 16-token
+// blocks: 9.0 us with parts of 16, 9.9 of 8, 11.0 of 4; of 1000: 8.1 of 8,
+// 8.7 of 16, 9.3 of 4; of 300: 6.9 of 4, 7.2 of 8).
 constexpr int32_t kMinPartBlocks = 4;
+constexpr int32_t kMaxMinPart = 32;
+// Sequences of up to this many positions are one item (one sequence of 130
+// tokens 5.5 us whole, 6.8 in parts; float32 6.8, 9.3), and longer ones where
+// the sequences alone make workgroups for a quarter of the chip (8 of 215: 6.9
+// whole, 8.5 in parts; float32 8.5, 10.8). One CU streams a cold context more
+// slowly than several: at 300 and at 512 the whole 300-token sequence of a
+// decode step and eight float32 ones of 64-512 lost (181 against 179 us for
+// four layers, 153 against 133 for eight).
+constexpr int32_t kWholePositions = 160;
+constexpr int32_t kWholePositionsMany = 256;
+constexpr int32_t kManyItems = 64;
 
 // Four waves: fewer waves per barrier than 1024 threads (0.06 us less per
 // decode launch of a 28-layer step, whose launches share one plan).
@@ -33,15 +49,28 @@ __device__ __forceinline__ int blocks_of(int ctx, int block_size, int lb) {
   return (ctx + block_size - 1) >> lb;
 }
 
-__device__ __forceinline__ int part_blocks(int nb, int split_k, int pb_global) {
-  if (split_k == 0) return pb_global;
+// Blocks per partition of a sequence of nb blocks (all but its last).
+__device__ __forceinline__ int part_blocks(int nb, int split_k, int pb_global, int whole) {
+  if (split_k == 0) return nb <= whole ? max(nb, 1) : pb_global;
   const int k = min(split_k, max(nb, 1));
   return max(1, (nb + k - 1) / k);
 }
 
+// The step's part size from its blocks in all and its longest sequence's.
+__device__ __forceinline__ int step_part_blocks(int64_t total_blocks, int longest,
+                                                int num_kv_heads, int target) {
+  const int64_t want = total_blocks * num_kv_heads;
+  const int least = min(max(longest / 8, kMinPartBlocks), kMaxMinPart);
+  return max(least, static_cast<int>((want + target - 1) / target));
+}
+
+__device__ __forceinline__ int whole_blocks(int num_seqs, int num_kv_heads, int lb) {
+  return (num_seqs * num_kv_heads >= kManyItems ? kWholePositionsMany : kWholePositions) >> lb;
+}
+
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     const int32_t* __restrict__ context_lens, int num_seqs, int num_kv_heads, int block_size,
-    int lb, int width, int split_k, int target, int min_pb, int max_items,
+    int lb, int width, int split_k, int target, int max_items,
     PlanItem* __restrict__ plan, int32_t* __restrict__ counters, int num_counters) {
   __shared__ int s_ctx[kMaxPlanSeqs];
   __shared__ int s_order[kMaxPlanSeqs];  // rank -> sequence
@@ -51,6 +80,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   __shared__ int s_rank[kSortLimit];  // slot -> plan position
   __shared__ int s_total_blocks;
   __shared__ int s_total_items;
+  __shared__ int s_longest;
+  const int whole = whole_blocks(num_seqs, num_kv_heads, lb);
   const int tid = threadIdx.x;
   const int max_ctx = width * block_size;
 
@@ -62,21 +93,21 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   if (tid == 0) {
     s_total_blocks = 0;
     s_total_items = 0;
+    s_longest = 0;
   }
   __syncthreads();
-  int local = 0;
+  int local = 0, longest = 0;
   for (int r = tid; r < num_seqs; r += kPlanThreads) {
     const int c = min(max(context_lens[r], 0), max_ctx);
     s_ctx[r] = c;
     local += blocks_of(c, block_size, lb);
+    longest = max(longest, blocks_of(c, block_size, lb));
   }
   atomicAdd(&s_total_blocks, local);
+  atomicMax(&s_longest, longest);
   __syncthreads();
-  int pb_global = 1;
-  if (split_k == 0) {
-    const int64_t want = static_cast<int64_t>(s_total_blocks) * num_kv_heads;
-    pb_global = max(min_pb, max(1, static_cast<int>((want + target - 1) / target)));
-  }
+  const int pb_global =
+      split_k == 0 ? step_part_blocks(s_total_blocks, s_longest, num_kv_heads, target) : 1;
 
   // Rank sequences by block count, longest first (ties keep batch order).
   const bool sort = num_seqs <= kSortLimit;
@@ -102,8 +133,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   int run = 0;
   for (int k = k0; k < k1; ++k) {
     const int nb = blocks_of(s_ctx[s_order[k]], block_size, lb);
-    run += max(1, (nb + part_blocks(nb, split_k, pb_global) - 1) /
-                      part_blocks(nb, split_k, pb_global));
+    run += max(1, (nb + part_blocks(nb, split_k, pb_global, whole) - 1) /
+                      part_blocks(nb, split_k, pb_global, whole));
   }
   s_scan[tid] = run;
   __syncthreads();
@@ -117,7 +148,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   for (int k = k0; k < k1; ++k) {
     s_first[k] = first;
     const int nb = blocks_of(s_ctx[s_order[k]], block_size, lb);
-    const int pb = part_blocks(nb, split_k, pb_global);
+    const int pb = part_blocks(nb, split_k, pb_global, whole);
     first += max(1, (nb + pb - 1) / pb);
   }
   if (tid == kPlanThreads - 1) s_total_items = s_scan[tid];
@@ -133,7 +164,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   if (by_size) {
     for (int k = tid; k < num_seqs; k += kPlanThreads) {
       const int nb = blocks_of(s_ctx[s_order[k]], block_size, lb);
-      const int pb = part_blocks(nb, split_k, pb_global);
+      const int pb = part_blocks(nb, split_k, pb_global, whole);
       const int np = max(1, (nb + pb - 1) / pb);
       for (int p = 0; p < np && s_first[k] + p < max_items; ++p)
         s_size[s_first[k] + p] = min(nb, (p + 1) * pb) - p * pb;
@@ -156,7 +187,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     const int r = s_order[k];
     const int c = s_ctx[r];
     const int nb = blocks_of(c, block_size, lb);
-    const int pb = part_blocks(nb, split_k, pb_global);
+    const int pb = part_blocks(nb, split_k, pb_global, whole);
     const int np = max(1, (nb + pb - 1) / pb);
     const int f = s_first[k];
     for (int p = 0; p < np && f + p < max_items; ++p) {
@@ -183,13 +214,13 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
 // partitions, the shape of every ordinary decode step: one lane per sequence
 // and no LDS, so the launch is little more than one load and one store. Every
 // wave derives the plan and each emits a quarter of it. All parts but a
-// sequence's last have the global part size, so an item's rank by size needs
-// only counts over sequences, not a sort over items.
+// sequence's last (or only) one have the step's part size, so an item's rank
+// by size needs only counts over sequences, not a sort over items.
 // Per launch in a graph: one sequence of 16384 tokens 10.1 -> 4.3 us, 32 of
 // 128-2048 8.6 -> 4.5.
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_wave_kernel(
     const int32_t* __restrict__ context_lens, int num_seqs, int num_kv_heads, int block_size,
-    int lb, int width, int target, int min_pb, int max_items, PlanItem* __restrict__ plan,
+    int lb, int width, int target, int max_items, PlanItem* __restrict__ plan,
     int32_t* __restrict__ counters, int num_counters) {
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
@@ -200,56 +231,62 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_wave_kernel(
   if (counters != nullptr)
     for (int i = tid; i < num_counters; i += kPlanThreads) counters[i] = 0;
   const int nb = blocks_of(ctx, block_size, lb);
-  const int64_t want = static_cast<int64_t>(wave_sum_int(nb)) * num_kv_heads;
-  const int pb = max(min_pb, max(1, static_cast<int>((want + target - 1) / target)));
-  const int np = max(1, (nb + pb - 1) / pb);
-  const int last = nb - (np - 1) * pb;
-  const int full = last < pb ? np - 1 : np;  // parts of the global size
+  int longest = nb;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) longest = max(longest, __shfl_xor(longest, o, kWave));
+  const int pb = step_part_blocks(wave_sum_int(nb), longest, num_kv_heads, target);
+  const int np = nb <= whole_blocks(num_seqs, num_kv_heads, lb) ? 1 : (nb + pb - 1) / pb;
+  const int last = nb - (np - 1) * pb;  // blocks of the last part, the odd one
   // Over the sequences ahead of this lane's (longer, or as long and earlier
-  // in the batch): items, full parts, and the smaller last parts ranked ahead.
-  int first = 0, full_ahead = 0, small_ahead = 0, items = 0, all_full = 0;
+  // in the batch): items and full parts; and the odd parts dispatched before this lane's
+  // full parts (larger, or as large in an earlier slot) and before its own.
+  int first = 0, full_ahead = 0, items = 0, odd_before_full = 0, odd_before_odd = 0;
   for (int s = 0; s < num_seqs; ++s) {
     const int nb_s = __builtin_amdgcn_readlane(nb, s);
     const int np_s = __builtin_amdgcn_readlane(np, s);
-    const int full_s = __builtin_amdgcn_readlane(full, s);
     const int last_s = __builtin_amdgcn_readlane(last, s);
     const bool ahead = nb_s > nb || (nb_s == nb && s < lane);
     first += ahead ? np_s : 0;
-    full_ahead += ahead ? full_s : 0;
-    if (full_s < np_s) small_ahead += last_s > last || (last_s == last && ahead);
+    full_ahead += ahead ? np_s - 1 : 0;
+    odd_before_full += last_s > pb || (last_s == pb && ahead);
+    odd_before_odd += last_s > last || (last_s == last && ahead);
     items += np_s;
-    all_full += full_s;
   }
-  auto emit = [&](int seq, int c, int blocks, int parts, int fulls, int slot, int full_rank,
-                  int small_rank, int p) {
+  const int all_full = items - num_seqs;
+  // Full parts smaller than this lane's odd one come after it.
+  const int full_before_odd =
+      pb > last ? all_full : pb == last ? full_ahead + np - 1 : 0;
+  const int full_rank = odd_before_full + full_ahead;
+  const int odd_rank = odd_before_odd + full_before_odd;
+  auto emit = [&](int seq, int c, int blocks, int parts, int slot, int full_at, int odd_at,
+                  int p) {
     if (slot + p >= max_items) return;
+    const bool odd = p == parts - 1;
     PlanItem it;
     it.seq = seq;
     it.blk_begin = p * pb;
-    it.blk_end = min(blocks, (p + 1) * pb);
+    it.blk_end = odd ? blocks : (p + 1) * pb;
     it.nparts = parts;
     it.first_item = slot;
     it.ctx = c;
     it.part = p;
     it.unused = 0;
-    plan[min(p < fulls ? full_rank + p : all_full + small_rank, max_items - 1)] = it;
+    plan[min(odd ? odd_at : full_at + p, max_items - 1)] = it;
   };
   if (__ballot(np > 2 * kWaves) == 0) {
     // Few parts each: every lane emits its own sequence's.
     if (mine)
       for (int p = wave; p < np; p += kWaves)
-        emit(lane, ctx, nb, np, full, first, full_ahead, small_ahead, p);
+        emit(lane, ctx, nb, np, first, full_rank, odd_rank, p);
   } else {
     // Long sequences: a lane per part.
     for (int s = wave; s < num_seqs; s += kWaves) {
       const int parts = __builtin_amdgcn_readlane(np, s);
       const int c = __builtin_amdgcn_readlane(ctx, s), blocks = __builtin_amdgcn_readlane(nb, s);
-      const int fulls = __builtin_amdgcn_readlane(full, s);
       const int slot = __builtin_amdgcn_readlane(first, s);
-      const int full_rank = __builtin_amdgcn_readlane(full_ahead, s);
-      const int small_rank = __builtin_amdgcn_readlane(small_ahead, s);
-      for (int p = lane; p < parts; p += kWave)
-        emit(s, c, blocks, parts, fulls, slot, full_rank, small_rank, p);
+      const int full_at = __builtin_amdgcn_readlane(full_rank, s);
+      const int odd_at = __builtin_amdgcn_readlane(odd_rank, s);
+      for (int p = lane; p < parts; p += kWave) emit(s, c, blocks, parts, slot, full_at, odd_at, p);
     }
   }
   for (int i = items + tid; i < max_items; i += kPlanThreads) {
@@ -277,13 +314,13 @@ int32_t launch_decode_plan(const int32_t* context_lens, int32_t num_seqs, int32_
   if (num_seqs <= kWave && split_k == 0) {
     decode_plan_wave_kernel<<<1, kPlanThreads, 0, stream>>>(
         context_lens, num_seqs, num_kv_heads, block_size, ilog2(block_size), block_table_width,
-        kTargetItems, kMinPartBlocks, decode_max_items(num_seqs, num_kv_heads, split_k), plan,
+        kTargetItems, decode_max_items(num_seqs, num_kv_heads, split_k), plan,
         counters, counters != nullptr ? num_seqs * num_kv_heads : 0);
     return check_launch("decode plan");
   }
   decode_plan_kernel<<<1, kPlanThreads, 0, stream>>>(
       context_lens, num_seqs, num_kv_heads, block_size, ilog2(block_size), block_table_width,
-      split_k, kTargetItems, kMinPartBlocks,
+      split_k, kTargetItems,
       decode_max_items(num_seqs, num_kv_heads, split_k), plan, counters,
       counters != nullptr ? num_seqs * num_kv_heads : 0);
   return check_launch("decode plan");

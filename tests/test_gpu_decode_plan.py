@@ -10,17 +10,18 @@ import torch
 from microinfer_amd.layer.hip_paged_attention import decode_plan
 
 pytestmark = pytest.mark.gpu
-TARGET, MIN_BLOCKS = 192, 4
+TARGET = 192
 
 
 def _expected(contexts, hkv, block_size):
     blocks = [-(-c // block_size) for c in contexts]
-    part = max(MIN_BLOCKS, 1, -(-sum(blocks) * hkv // TARGET))
+    part = max(min(max(max(blocks) // 8, 4), 32), -(-sum(blocks) * hkv // TARGET))
+    whole = (256 if len(contexts) * hkv >= 64 else 160) // block_size
     items, slot = [], 0
     for r in sorted(range(len(blocks)), key=lambda r: (-blocks[r], r)):
-        parts = max(1, -(-blocks[r] // part))
+        parts = 1 if blocks[r] <= whole else -(-blocks[r] // part)
         for p in range(parts):
-            end = min(blocks[r], (p + 1) * part)
+            end = blocks[r] if p == parts - 1 else (p + 1) * part
             items.append((end - p * part, slot + p,
                           [r, p * part, end, parts, slot, contexts[r], p, 0]))
         slot += parts
@@ -30,6 +31,7 @@ def _expected(contexts, hkv, block_size):
 @pytest.mark.parametrize("hkv,block_size", [(8, 16), (1, 16), (2, 64)])
 @pytest.mark.parametrize("contexts", [
     [1], [0, 0], [64, 65, 1], [32768], [5000, 16, 4999, 0, 16], [100] * 64,
+    [161, 160, 130, 400, 1, 2000], [256, 257, 300, 129, 4000] * 3,
     list(range(1, 2049, 32)), [31 * i % 700 for i in range(65)],
 ])
 def test_plan_items_and_order(contexts, hkv, block_size):
