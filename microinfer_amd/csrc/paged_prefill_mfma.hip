@@ -109,7 +109,7 @@ __device__ __forceinline__ int swz_v(int key) { return 4 * (key & 3); }
 // A (row block, KV head) split along its keys has at most kMaxParts
 // partitions; the last one to finish merges them kMergeBatch at a time.
 constexpr int kMaxParts = 8;
-constexpr int kMergeBatch = 4;
+constexpr int kMergeBatch = 2;
 
 // Largest exponent a probability may reach before the running maximum is
 // moved (p <= 2^15 fits f16 as well as bf16).
@@ -831,8 +831,8 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     // every other partition has already arrived; the last arrival merges
     // all partitions in partition order (its own from registers: the values
     // its slot would hold), so the result does not depend on which one
-    // arrives last. Partial region of (slot, head, wave): o as [db*16 + i]
-    // [lane] floats, (m, l) as [2][lane].
+    // arrives last. Partial region of (slot, head, wave): o as [db*8 + i/2]
+    // [lane][2] floats, (m, l) as [lane][2].
     int32_t* ctr = a.counters + static_cast<int64_t>(counter) * a.num_kv_heads + head;
     auto region = [&](int p) {
       return (static_cast<int64_t>(slot + p) * a.num_kv_heads + head) * kWaves + wave;
@@ -844,13 +844,13 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     __syncthreads();  // s_arrived is written again below
     if (!last_now) {
       const int64_t r = region(part);
-      float* acc = a.ws_acc + r * (kD / 32 * 16 * kWave) + lane;
+      float* acc = a.ws_acc + r * (kD / 32 * 16 * kWave) + 2 * lane;
 #pragma unroll
       for (int db = 0; db < kD / 32; ++db)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) store_coherent(acc + (db * 16 + i) * kWave, o[db][i]);
-      store_coherent(a.ws_ml + r * 2 * kWave + lane, m);
-      store_coherent(a.ws_ml + r * 2 * kWave + kWave + lane, l);
+        for (int i = 0; i < 16; i += 2)
+          store_coherent2(acc + (db * 16 + i) * kWave, o[db][i], o[db][i + 1]);
+      store_coherent2(a.ws_ml + (r * kWave + lane) * 2, m, l);
       wait_stores();
       __syncthreads();  // every wave's partial is at the coherent level
       if (tid == 0)
@@ -860,48 +860,90 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     }
     // Merge: mx = max m_p; o = sum_p 2^(m_p - mx) o_p, l likewise (m_p =
     // -inf: nothing of that partition is visible to the row, weight 0), in
-    // partition order, the loads of kMergeBatch partitions in flight at once.
-    float f[kMaxParts], lsum = 0.f, mx = -INFINITY;
+    // partition order.
+    auto weight = [](float mp, float mx) { return mp == -INFINITY ? 0.f : fast_exp2(mp - mx); };
+    if (nparts == 2) {
+      // The other partition comes in two round trips of 16 loads (as batches
+      // of one block of O the merge took five; four chunks of 93-199 rows on
+      // 700 keys: 30.6 -> 24.1 us a launch).
+      const int64_t r = region(1 - part);
+      const float* src = a.ws_acc + r * (kD / 32 * 16 * kWave) + 2 * lane;
+      const Float2 ml = load_coherent2(a.ws_ml + (r * kWave + lane) * 2);
+      const float mx = fmaxf(m, ml.x);
+      const float mine = weight(m, mx), other = weight(ml.x, mx);
+      // fma(f1, o1, f0 * o0) whichever of the two this one is.
+      auto both = [&](float own, float far) {
+        return part == 0 ? fmaf(other, far, mine * own) : fmaf(mine, own, other * far);
+      };
 #pragma unroll
-    for (int p = 0; p < kMaxParts; ++p) {
-      f[p] = -INFINITY;
-      if (p < nparts) f[p] = p == part ? m : load_coherent(a.ws_ml + region(p) * 2 * kWave + lane);
-    }
+      for (int h = 0; h < kD / 32; h += 2) {
+        Float2 v[2][8];
 #pragma unroll
-    for (int p = 0; p < kMaxParts; ++p) mx = fmaxf(mx, f[p]);
+        for (int d = 0; d < 2; ++d)
 #pragma unroll
-    for (int p = 0; p < kMaxParts; ++p) {
-      f[p] = f[p] == -INFINITY ? 0.f : fast_exp2(f[p] - mx);
-      if (p < nparts)
-        lsum = fmaf(f[p], p == part ? l : load_coherent(a.ws_ml + region(p) * 2 * kWave + kWave + lane),
-                    lsum);
-    }
+          for (int i = 0; i < 8; ++i)
+            v[d][i] = load_coherent2(src + ((h + d) * 16 + 2 * i) * kWave);
 #pragma unroll
-    for (int db = 0; db < kD / 32; ++db) {
-      f32x16_t acc;
+        for (int d = 0; d < 2; ++d)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-      for (int p0 = 0; p0 < kMaxParts; p0 += kMergeBatch) {
-        if (p0 >= nparts) break;
-        float v[kMergeBatch][16];
-#pragma unroll
-        for (int j = 0; j < kMergeBatch; ++j) {
-          const int p = p0 + j;
-          const float* src =
-              a.ws_acc + region(p) * (kD / 32 * 16 * kWave) + db * 16 * kWave + lane;
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-            v[j][i] = p < nparts && p != part ? load_coherent(src + i * kWave) : o[db][i];
-        }
-#pragma unroll
-        for (int j = 0; j < kMergeBatch; ++j)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[i] = fmaf(f[p0 + j], v[j][i], acc[i]);
+          for (int i = 0; i < 8; ++i) {
+            o[h + d][2 * i] = both(o[h + d][2 * i], v[d][i].x);
+            o[h + d][2 * i + 1] = both(o[h + d][2 * i + 1], v[d][i].y);
+          }
       }
-      o[db] = acc;
+      l = both(l, ml.y);
+    } else {
+      // Own values from registers (those its slot would hold), the loads of
+      // kMergeBatch partitions in flight at once.
+      float f[kMaxParts], lsum = 0.f, mx = -INFINITY;
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p) {
+        f[p] = -INFINITY;
+        if (p < nparts)
+          f[p] = p == part ? m : load_coherent(a.ws_ml + (region(p) * kWave + lane) * 2);
+      }
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p) mx = fmaxf(mx, f[p]);
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p) {
+        f[p] = weight(f[p], mx);
+        if (p < nparts)
+          lsum = fmaf(f[p], p == part ? l : load_coherent(a.ws_ml + (region(p) * kWave + lane) * 2 + 1),
+                      lsum);
+      }
+#pragma unroll
+      for (int db = 0; db < kD / 32; ++db) {
+        f32x16_t acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+        for (int p0 = 0; p0 < kMaxParts; p0 += kMergeBatch) {
+          if (p0 >= nparts) break;
+          Float2 v[kMergeBatch][8];
+#pragma unroll
+          for (int j = 0; j < kMergeBatch; ++j) {
+            const int p = p0 + j;
+            const float* src =
+                a.ws_acc + region(p) * (kD / 32 * 16 * kWave) + db * 16 * kWave + 2 * lane;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              v[j][i] = p < nparts && p != part ? load_coherent2(src + 2 * i * kWave)
+                                                : Float2{o[db][2 * i], o[db][2 * i + 1]};
+          }
+#pragma unroll
+          for (int j = 0; j < kMergeBatch; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              acc[2 * i] = fmaf(f[p0 + j], v[j][i].x, acc[2 * i]);
+              acc[2 * i + 1] = fmaf(f[p0 + j], v[j][i].y, acc[2 * i + 1]);
+            }
+        }
+        o[db] = acc;
+        // One block of O at a time: hoisting the next one's loads would spill.
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      l = lsum;
     }
-    l = lsum;
     if (tid == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   // The row's sum: both halves add (lane l & 31) + (lane l | 32).
