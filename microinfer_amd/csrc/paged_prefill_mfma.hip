@@ -997,7 +997,7 @@ int64_t max_cache_offset(const AttnArgs& a) {
 // step: 111.1 us at 48, 113.3 at 96, 112.4 at 40; A/B on two boxes).
 // ---------------------------------------------------------------------------
 constexpr int kPlanThreads = 256;
-constexpr int kPlanPer = 16;  // row blocks per plan thread (registers)
+constexpr int kPlanPer = 16;  // row blocks per plan thread at most (registers)
 constexpr int kMaxPlanBlocks = kPlanThreads * kPlanPer;
 constexpr int kMaxPlanReqs = 2048;
 constexpr int kPlanBuckets = 2 * kPlanThreads;  // sizes >= 511 share the first
@@ -1036,6 +1036,10 @@ __device__ __forceinline__ int block_sum(int v, int* s_wave) {
   return total;
 }
 
+// PER: row blocks per thread. Launches of at most kPlanThreads row blocks take
+// one each: the loops over kPlanPer unroll to sixteen times the code, most of
+// it skipped but all of it fetched (@@).
+template <int PER>
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, int num_seqs, int bm,
     int ctx_cap, int64_t kv_rows, int cus, int heads, int part_cap, int max_entries,
@@ -1079,10 +1083,10 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(
 
   // This thread's row blocks q = tid + k * kPlanThreads: request, block,
   // key tiles (the attention kernel's kv_end) and work estimate.
-  int req[kPlanPer], rb[kPlanPer], tiles[kPlanPer], units[kPlanPer];
+  int req[PER], rb[PER], tiles[PER], units[PER];
   int work = 0;
 #pragma unroll
-  for (int k = 0; k < kPlanPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     const int q = tid + k * kPlanThreads;
     req[k] = -1;
     rb[k] = tiles[k] = units[k] = 0;
@@ -1115,7 +1119,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(
   for (int iter = 0;; ++iter) {  // raise the target until the partitions fit
     int need = 0;
 #pragma unroll
-    for (int k = 0; k < kPlanPer; ++k) {
+    for (int k = 0; k < PER; ++k) {
       const int n = parts_of(tiles[k], target);
       need += n > 1 ? n : 0;
     }
@@ -1130,7 +1134,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(
   auto bucket_of = [](int size) { return kPlanBuckets - 1 - min(size, kPlanBuckets - 1); };
   int nsplit = 0, nslots = 0;
 #pragma unroll
-  for (int k = 0; k < kPlanPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     if (req[k] < 0) continue;
     const int n = parts_of(tiles[k], target);
     for (int p = 0; p < n; ++p) {
@@ -1153,7 +1157,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(
   if (tid == 0) count[0] = min(items, max_entries);
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kPlanPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     if (req[k] < 0) continue;
     const int t = tiles[k] < 0 ? -tiles[k] - 1 : tiles[k];
     const int n = parts_of(tiles[k], target);
@@ -1270,13 +1274,20 @@ int32_t launch_prefill_plan(const AttnArgs& a, void* workspace, hipStream_t stre
   const PrefillLayout l = prefill_layout(a.num_rows, a.num_seqs, a.group, a.num_kv_heads);
   char* ws = static_cast<char*>(workspace);
   const bool paged = a.tables != nullptr;
-  prefill_plan_kernel<<<1, kPlanThreads, 0, stream>>>(
-      a.cu_q, a.cu_k, a.num_seqs, kRows * kWaves / a.group,
-      paged ? a.t_width * a.block_size : INT_MAX, paged ? int64_t(-1) : int64_t(a.num_blocks),
-      device_cus(), a.num_kv_heads, part_cap_of(a.num_kv_heads),
-      static_cast<int>(l.max_entries), reinterpret_cast<PrefillItem*>(ws + l.plan_off),
-      reinterpret_cast<int32_t*>(ws), reinterpret_cast<int32_t*>(ws + l.counters_off),
-      prefill_counters(a.num_kv_heads));
+  const int bm = kRows * kWaves / a.group;
+  auto go = [&](auto kernel) {
+    kernel<<<1, kPlanThreads, 0, stream>>>(
+        a.cu_q, a.cu_k, a.num_seqs, bm, paged ? a.t_width * a.block_size : INT_MAX,
+        paged ? int64_t(-1) : int64_t(a.num_blocks), device_cus(), a.num_kv_heads,
+        part_cap_of(a.num_kv_heads), static_cast<int>(l.max_entries),
+        reinterpret_cast<PrefillItem*>(ws + l.plan_off), reinterpret_cast<int32_t*>(ws),
+        reinterpret_cast<int32_t*>(ws + l.counters_off), prefill_counters(a.num_kv_heads));
+  };
+  // Every request's row blocks fit in this many.
+  if ((static_cast<int64_t>(a.num_rows) + bm - 1) / bm + a.num_seqs <= kPlanThreads)
+    go(prefill_plan_kernel<1>);
+  else
+    go(prefill_plan_kernel<kPlanPer>);
   return check_launch("paged prefill plan");
 }
 
