@@ -425,6 +425,57 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_attention_vector_kernel(c
   auto item_row = [&](int part, int g) {
     return (static_cast<int64_t>(first_item + part) * a.num_kv_heads + head) * G + g;
   };
+  // Few partitions: every lane group reads up to kMine of them, all their
+  // loads in one round trip (the passes below take three: 8 float32 sequences
+  // of 64-512 tokens, eight layers: 132.6 -> 121.4 us).
+  constexpr int kMine = GMAX * VEC <= 16 ? 4 : 0;
+  if constexpr (kMine > 0) {
+    if (nparts <= kMine * PPW) {
+      float pm[kMine][GMAX], pl[kMine][GMAX], po[kMine][GMAX][VEC];
+#pragma unroll
+      for (int k = 0; k < kMine; ++k) {
+        const int p = grp + k * PPW;
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) {
+          const bool valid = p < nparts && (EXACT || g < G);
+          const int64_t row = item_row(valid ? p : 0, valid ? g : 0);
+          pm[k][g] = load_coherent(a.ws_ml + row * 2);
+          pl[k][g] = load_coherent(a.ws_ml + row * 2 + 1);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) po[k][g][j] = load_coherent(a.ws_acc + row * D + d0 + j);
+          if (!valid) pm[k][g] = -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < GMAX; ++g) {
+        if (!EXACT && g >= G) continue;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < kMine; ++k) mx = fmaxf(mx, pm[k][g]);
+        mx = xor_max<LPR, kWave>(mx);
+        float t = 0.f, out[VEC];
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) out[j] = 0.f;
+#pragma unroll
+        for (int k = 0; k < kMine; ++k) {
+          if (pm[k][g] == -INFINITY) continue;  // empty or not there
+          const float w = fast_exp2(pm[k][g] - mx);
+          t = fmaf(w, pl[k][g], t);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) out[j] = fmaf(w, po[k][g][j], out[j]);
+        }
+        t = xor_sum<LPR, kWave>(t);
+        const float inv = t > 0.f ? 1.f / t : 0.f;
+        Pack<R, VEC> o;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) o.v[j] = E::store(xor_sum<LPR, kWave>(out[j]) * inv);
+        if (grp == 0) store_pack<R, VEC>(obase + (head * G + g) * a.o_hs, o);
+      }
+      if (lane == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
+
   // Pass 1: lane i reads partition i's maxima.
   float mx[GMAX];
 #pragma unroll
