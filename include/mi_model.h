@@ -60,9 +60,10 @@ int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
  *   y = silu(gate) * up               (swiglu = 1; w holds n = 2 inter rows,
  *                                      gate's then up's, y is [m, inter])
  * The norm (FuseLayerNorm, microinfer/layer/norm.py:26-35, on a sum already
- * made) is applied as (1 / rms) * ((x * norm_weight rounded once) . w^T), so
- * it differs from mi_rms_norm_residual + mi_linear by that pair's second
- * rounding. The projection's sum is rounded to the element type before the
+ * made): for float16 the row is normalised as mi_rms_norm_residual does it,
+ * and the result is that call's and mi_linear's (mi_linear_swiglu's) bit for
+ * bit; for bf16 it is applied as (1 / rms) * ((x * norm_weight rounded once)
+ * . w^T), which lacks that pair's second rounding. The projection's sum is rounded to the element type before the
  * residual is added and the result rounded again, as x + F.linear(...) does;
  * residual may be NULL and may be y itself. norm_weight may be NULL: then m may
  * be up to 4096. Shapes, alignment and other limits are those of mi_linear /

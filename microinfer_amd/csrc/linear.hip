@@ -20,9 +20,15 @@
 //    outputs (1024 columns) then still give all CUs work, where 16-column
 //    tiles leave three quarters of them idle.
 //
-// RMSNorm in front: y[m] = (1 / rms(x[m])) * (x[m] * weight) . w^T. The
+// RMSNorm in front, bf16: y[m] = (1 / rms(x[m])) * (x[m] * weight) . w^T. The
 // product x * weight is rounded once to the element type (torch's norm rounds
-// twice), 1 / rms scales the float32 sum.
+// twice), 1 / rms scales the float32 sum, so no pass over the row comes first.
+// float16: x * weight may lie outside the type's range where the normalised
+// row does not (kNormFirst), so the row is normalised first, with the
+// additions and roundings of rms_norm_residual_kernel: the result is that
+// launch's and the projection's, bit for bit. The pass over the row costs
+// (4096 x 1024, us, against scaling the sum) 0.2 at one row, 1.2 at 16, 2.4
+// at 64, where the norm's own launch is the cheaper (8.6 against 7.7 in all).
 #include "mi_common.h"
 #include "mi_model.h"
 
@@ -75,6 +81,12 @@ struct LinArgs {
   int64_t rs;
 };
 
+// Whether rows are normalised before they are rounded again. float16 holds
+// 6e-8 to 65504: a row with a channel of 6000 under a weight of 12 is finite
+// once normalised, its product before that is not.
+template <typename E>
+constexpr bool kNormFirst = std::is_same<E, F16>::value;
+
 // x[i] * w[i] over an 8-element fragment, rounded once.
 template <typename E>
 __device__ __forceinline__ Pack<uint16_t, 8> scale8(const Pack<uint16_t, 8>& x,
@@ -85,6 +97,57 @@ __device__ __forceinline__ Pack<uint16_t, 8> scale8(const Pack<uint16_t, 8>& x,
     r.v[i] = __builtin_bit_cast(
         uint16_t, static_cast<typename LinMfma<E>::el>(E::load(x.v[i]) * E::load(w.v[i])));
   return r;
+}
+
+// round(round(x[i] * inv) * w[i]) over an 8-element fragment.
+template <typename E>
+__device__ __forceinline__ Pack<uint16_t, 8> norm8(const Pack<uint16_t, 8>& x, float inv,
+                                                   const Pack<uint16_t, 8>& w) {
+  Pack<uint16_t, 8> r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    r.v[i] = E::store(E::load(E::store(E::load(x.v[i]) * inv)) * E::load(w.v[i]));
+  return r;
+}
+
+template <typename E>
+__device__ __forceinline__ float add_squares(const Pack<uint16_t, 8>& x, float ss) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float f = E::load(x.v[i]);
+    ss = fmaf(f, f, ss);
+  }
+  return ss;
+}
+
+// 1 / rms of ROWS rows of k elements by a wave, summed in the order of
+// rms_norm_residual_kernel: lane i takes the 8-element pieces i, i + 64, ...
+template <typename E, int ROWS>
+__device__ __forceinline__ void inverse_rms(const uint16_t* const (&row)[ROWS], int k, float eps,
+                                            int lane, float (&inv)[ROWS]) {
+  constexpr int kAhead = 2;  // pieces of each row in flight
+  float ss[ROWS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) ss[r] = 0.f;
+  for (int k0 = 0; k0 < k; k0 += kAhead * 8 * kWave) {
+    Pack<uint16_t, 8> x[kAhead][ROWS];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int off = k0 + (i * kWave + lane) * 8;
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) x[i][r] = load_pack<uint16_t, 8>(row[r] + (off < k ? off : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (k0 + (i * kWave + lane) * 8 < k) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) ss[r] = add_squares<E>(x[i][r], ss[r]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+    inv[r] = rsqrtf(group_sum<kWave>(ss[r]) / static_cast<float>(k) + eps);
 }
 
 // acc + sum of x[i] * w[i] over the fragment.
@@ -141,7 +204,9 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
   constexpr int kRing = NW * S * kSlot;
   // The ring, then (after every wave has read its last chunk) the sums.
   __shared__ __attribute__((aligned(16))) char s_mem[kRing > kSums ? kRing : kSums];
-  __shared__ float s_ss[NORM ? NW : 1][MT * 16];
+  constexpr bool kFirst = NORM && kNormFirst<E>;
+  constexpr bool kAfter = NORM && !kNormFirst<E>;
+  __shared__ float s_ss[kAfter ? NW : 1][MT * 16];  // squares by wave, or the rows' 1 / rms
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -204,11 +269,28 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
     return *reinterpret_cast<const Pack<R, 8>*>(tile + col * kRowBytes +
                                                 (((4 * step + quad) ^ swz(col)) * 16));
   };
-  const R* nrow = static_cast<const R*>(a.norm) + quad * 8;
-  if (c_begin < c_end) {
 #pragma unroll
-    for (int s = 0; s < S; ++s)
-      if (c_begin + s < c_end) issue(s, c_begin + s);
+  for (int s = 0; s < S; ++s)
+    if (c_begin + s < c_end) issue(s, c_begin + s);
+  const R* nrow = static_cast<const R*>(a.norm) + quad * 8;
+  [[maybe_unused]] float inv[MT];
+  if constexpr (kFirst) {
+    constexpr int kRows = MT * 16 / NW;
+    const R* row[kRows];
+    float row_inv[kRows];
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+      row[i] = static_cast<const R*>(a.x) +
+               static_cast<int64_t>(min(r0 + wave * kRows + i, a.m - 1)) * a.xs;
+    inverse_rms<E>(row, a.k, a.eps, lane, row_inv);
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+      if (lane == i) s_ss[0][wave * kRows + i] = row_inv[i];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) inv[t] = s_ss[0][16 * t + col];
+  }
+  if (c_begin < c_end) {
     for (int c = c_begin, slot = 0; c < c_end; ++c, slot = slot + 1 == S ? 0 : slot + 1) {
       Pack<R, 8> g[NORM ? kChunkSteps : 1];
       if constexpr (NORM) {
@@ -237,7 +319,8 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
           Pack<R, 8> x = fragment(cur + (NT + t) * kTileBytes, j);
-          if constexpr (NORM) {
+          if constexpr (kFirst) x = norm8<E>(x, inv[t], g[j]);
+          if constexpr (kAfter) {
             ss[t] = dot8<E>(x, x, ss[t]);
             x = scale8<E>(x, g[j]);
           }
@@ -265,7 +348,7 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
   for (int u = 0; u < NT; ++u)
 #pragma unroll
     for (int t = 0; t < MT; ++t) sum_at(wave, u * MT + t) = acc[u][t];
-  if constexpr (NORM) {
+  if constexpr (kAfter) {
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const float v = xor_sum<16, kWave>(ss[t]);
@@ -286,7 +369,7 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
       v += sum_at(wv, unit);
       if constexpr (GLU) up += sum_at(wv, kUnits + unit);
     }
-    if constexpr (NORM) {
+    if constexpr (kAfter) {
       float sum = 0.f;
 #pragma unroll
       for (int wv = 0; wv < NW; ++wv) sum += s_ss[wv][16 * t + col];
@@ -338,10 +421,12 @@ __global__ __launch_bounds__(kGemvWaves* kWave) void gemv_kernel(const LinArgs a
     xrow[i] = static_cast<const R*>(a.x) + static_cast<int64_t>(min(i, a.m - 1)) * a.xs;
   const R* nrow = static_cast<const R*>(a.norm);
 
-  float acc[RW][M], ss[M];
+  constexpr bool kFirst = NORM && kNormFirst<E>;
+  constexpr bool kAfter = NORM && !kNormFirst<E>;
+  float acc[RW][M], ss[M], inv[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    ss[i] = 0.f;
+    ss[i] = inv[i] = 0.f;
 #pragma unroll
     for (int r = 0; r < RW; ++r) acc[r][i] = 0.f;
   }
@@ -358,13 +443,28 @@ __global__ __launch_bounds__(kGemvWaves* kWave) void gemv_kernel(const LinArgs a
 #pragma unroll
       for (int i = 0; i < M; ++i) x[u][i] = load_pack<R, 8>(xrow[i] + at);
     }
+    if constexpr (kFirst) {
+      // A row that is all here needs no loads of its own for its squares.
+      if (a.k <= U * kGemvChunk) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (u * kGemvChunk + lane * 8 < a.k) ss[i] = add_squares<E>(x[u][i], ss[i]);
+          inv[i] = rsqrtf(group_sum<kWave>(ss[i]) / static_cast<float>(a.k) + a.eps);
+        }
+      } else if (k0 == 0) {
+        inverse_rms<E>(xrow, a.k, a.eps, lane, inv);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (k0 + u * kGemvChunk + lane * 8 < a.k) {
 #pragma unroll
         for (int i = 0; i < M; ++i) {
           Pack<R, 8> xv = x[u][i];
-          if constexpr (NORM) {
+          if constexpr (kFirst) xv = norm8<E>(xv, inv[i], g[u]);
+          if constexpr (kAfter) {
             ss[i] = dot8<E>(xv, xv, ss[i]);
             xv = scale8<E>(xv, g[u]);
           }
@@ -376,10 +476,10 @@ __global__ __launch_bounds__(kGemvWaves* kWave) void gemv_kernel(const LinArgs a
   }
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    if constexpr (NORM) {
-      const float inv = rsqrtf(group_sum<kWave>(ss[i]) / static_cast<float>(a.k) + a.eps);
+    if constexpr (kAfter) {
+      const float scale = rsqrtf(group_sum<kWave>(ss[i]) / static_cast<float>(a.k) + a.eps);
 #pragma unroll
-      for (int r = 0; r < RW; ++r) acc[r][i] = group_sum<kWave>(acc[r][i]) * inv;
+      for (int r = 0; r < RW; ++r) acc[r][i] = group_sum<kWave>(acc[r][i]) * scale;
     } else {
 #pragma unroll
       for (int r = 0; r < RW; ++r) acc[r][i] = group_sum<kWave>(acc[r][i]);

@@ -78,10 +78,14 @@ def prefer_hip_prefill(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def prefer_fused_norm(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether the norm in front of a preferred projection is better done
     inside it: every workgroup then scales the x rows it reads again, which
-    past 16 rows and 2048 elements costs more than the norm's own launch (3.6
-    us; 24576 x 4096 at 64 rows 67 against 59 + 3.6, 12288 x 2048 22.7
-    against 19.4 + 3.6, 4096 x 1024 6.2 against 4.5 + 3.6)."""
-    return prefer_hip_linear(x, weight) and (x.shape[0] <= 16 or x.shape[1] <= 2048)
+    past 16 rows and 2048 elements costs more than the norm's own launch (one
+    launch against two, us: 24576 x 4096 at 33 rows 67 / 53, at 64 69 / 70;
+    12288 x 2048 at 64 rows 23.2 / 25.7, 4096 x 1024 6.7 / 8.3).
+    float16 rows are normalised before they are scaled, a pass more: worth it
+    up to 16 rows (4096 x 1024 at 1 / 16 / 17 / 64 rows 4.2 / 6.1 / 7.8 / 8.6
+    against 6.1 / 6.9 / 7.3 / 7.7; 24576 x 4096 at 16 rows 43 against 44)."""
+    narrow = x.shape[1] <= 2048 and x.dtype != torch.float16
+    return prefer_hip_linear(x, weight) and (x.shape[0] <= 16 or narrow)
 
 
 def hip_linear(x: torch.Tensor, weight: torch.Tensor, *,
@@ -135,9 +139,9 @@ def hip_linear_fused(x: torch.Tensor, weight: torch.Tensor, *,
     or with ``swiglu`` the gate ``silu(gate) * up`` of a ``[2 I, k]`` weight;
     ``norm_weight`` and ``residual`` are optional (``FuseLayerNorm.forward``,
     norm.py:26-35, around the projections of ``TransformerLayer.forward``,
-    transformer.py:245-252). The norm's product is rounded once and its scale
-    applied to the float32 sum; the other roundings are those of the separate
-    calls."""
+    transformer.py:245-252). The roundings are those of the separate calls,
+    except that with bf16 the norm's product is rounded once and its scale
+    applied to the float32 sum."""
     _lib.require_device(x, weight, norm_weight, residual, what="fused projection")
     limit = FUSED_MAX_ROWS if norm_weight is None else LINEAR_MAX_ROWS
     if not supported_linear(x, weight, limit) or (swiglu and weight.shape[0] % 32):

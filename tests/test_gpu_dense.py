@@ -232,6 +232,44 @@ def test_linear_fused_is_norm_projection_and_sum(dtype, m, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 2, 3, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(4096, 1024), (1024, 2080), (6144, 4096), (48, 64), (96, 5152)])
+def test_norm_inside_over_the_range_of_the_type(dtype, m, n, k):
+    """Rows with a channel near float16's largest value under a weight that
+    takes their product past it, rows of subnormals and zero rows. float16
+    normalises first, with the additions and roundings of the norm's own
+    launch: bit for bit the two launches. bf16 rounds x * weight once: within
+    that rounding (k of them, independent) and the output's of float64."""
+    torch.manual_seed(m * 7 + n + k)
+    x = torch.randn(m, k, device=DEV)
+    g = 1 + 0.1 * torch.randn(k, device=DEV)
+    x[0::3, 5] = 3e4
+    x[0::3, 40] = -6e4
+    g[5], g[40] = 3.0, 12.0
+    x[1::3] *= 1e-5
+    x[2::6] = 0
+    x, g = x.to(dtype), g.to(dtype)
+    w = (0.05 * torch.randn(n, k, device=DEV)).to(dtype)
+    res = torch.randn(m, n, device=DEV).to(dtype)
+    for eps in (1e-6, 1e-12):
+        got = hip_linear_fused(x, w, norm_weight=g, eps=eps)
+        if dtype == torch.bfloat16:
+            normed = F.rms_norm(x.double(), (k,), g.double(), eps)
+            y, unit = normed @ w.double().t(), 2.0 ** -8
+            spread = unit * (normed.square() @ w.double().square().t()).sqrt()
+            assert bool(((got.double() - y).abs() <= 4 * spread + unit * y.abs()).all())
+            continue
+        normed, _ = hip_rms_norm_residual(x, None, g, eps)
+        want = hip_linear(normed, w)
+        assert bool(want.isfinite().all()) and torch.equal(got, want)
+        assert torch.equal(hip_linear_fused(x, w, norm_weight=g, eps=eps, residual=res),
+                           res + want)
+        if n % 32 == 0:
+            assert torch.equal(hip_linear_fused(x, w, norm_weight=g, eps=eps, swiglu=True),
+                               hip_linear_swiglu(normed, w))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m", [65, 128, 200, 333, 641])
 @pytest.mark.parametrize("n,k", [(4096, 1024), (1024, 3072), (6144, 1024), (48, 64), (2080, 160)])
 def test_linear_fused_past_64_rows(dtype, m, n, k):
