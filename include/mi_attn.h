@@ -362,8 +362,9 @@ int32_t mi_gather_kv(const void* key_cache, const void* value_cache,
 
 /*
  * mi_gather_kv with cu_seqlens_k in host memory (num_requests + 1 entries,
- * read before the call returns; at most 64 requests): the offsets travel with
- * the launch, so the caller uploads nothing.
+ * all of them read, before the call returns; at most 64 requests): the offsets
+ * travel with the launch, so the caller uploads nothing. A captured launch
+ * keeps the offsets of its capture.
  */
 int32_t mi_gather_kv_host(const void* key_cache, const void* value_cache,
                           int64_t cache_block_stride, int64_t cache_token_stride,

@@ -524,9 +524,14 @@ def hip_gather_kv(key_cache, value_cache, block_tables, cu_seqlens_k, total_rows
 
 def hip_gather_kv_host(key_cache, value_cache, block_tables, offsets: list[int]):
     """``hip_gather_kv`` with the ``cu_seqlens_k`` of at most 64 requests on the
-    host: nothing is uploaded and nothing waited for."""
-    if len(offsets) - 1 > GATHER_HOST_REQUESTS or offsets[-1] > 2 ** 31 - 1:
-        raise ValueError("hip_gather_kv_host: at most 64 requests and int32 offsets")
+    host: nothing is uploaded and nothing waited for. The library reads one
+    offset per table row and one more."""
+    if len(offsets) != block_tables.shape[0] + 1 or len(offsets) - 1 > GATHER_HOST_REQUESTS:
+        raise ValueError("hip_gather_kv_host: one offset per table row and one more, at most 64 "
+                         "rows")
+    if (offsets[0] != 0 or any(b < a for a, b in zip(offsets, offsets[1:]))
+            or offsets[-1] > 2 ** 31 - 1):
+        raise ValueError("hip_gather_kv_host: offsets must rise from 0 within int32")
     host = (ctypes.c_int32 * len(offsets))(*offsets)
     return _gather(key_cache, value_cache, block_tables, offsets[-1],
                    _lib.load().mi_gather_kv_host, ctypes.addressof(host))

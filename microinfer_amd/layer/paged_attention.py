@@ -52,7 +52,8 @@ def gather_paged_kv(key_cache, value_cache, block_tables, contexts, block_size):
     for length in contexts:
         offsets.append(offsets[-1] + length)
     tables = block_tables[: len(contexts)]
-    if len(contexts) <= GATHER_HOST_REQUESTS and offsets[-1] <= _INT32_MAX:
+    if (len(contexts) == tables.shape[0] <= GATHER_HOST_REQUESTS
+            and offsets[-1] <= _INT32_MAX):
         return hip_gather_kv_host(key_cache, value_cache, tables, offsets)
     cu_k = torch.tensor(offsets, dtype=torch.int32, device=key_cache.device)
     return hip_gather_kv(key_cache, value_cache, tables, cu_k, offsets[-1])

@@ -10,7 +10,8 @@ import pytest
 import torch
 
 from microinfer_amd.layer.cached_attention import CachedAttention
-from microinfer_amd.layer.hip_paged_attention import hip_paged_decode, hip_paged_prefill
+from microinfer_amd.layer.hip_paged_attention import (hip_gather_kv_host, hip_paged_decode,
+                                                      hip_paged_prefill)
 from microinfer_amd.layer.metadata import AttentionMetadata
 from microinfer_amd.layer.paged_attention import paged_attention_meta
 from microinfer_amd.worker.hip_kv_store import store_kv
@@ -148,3 +149,14 @@ def test_wrapper_value_errors_mirror_reference():
     with pytest.raises(ValueError, match="inner dimensions"):
         store_kv(cache, cache, torch.zeros(1), torch.zeros(1), torch.zeros(1, 32, 2).transpose(1, 2),
                  torch.zeros(1, 2, 32), 16)
+
+
+@pytest.mark.parametrize("rows,offsets", [
+    (3, [0, 5]), (3, [0, 1, 2]), (3, [0, 1, 2, 3, 4]), (1, []), (0, []), (0, [0, 1]),
+    (65, list(range(66))), (2, [1, 2, 3]), (2, [0, 3, 2]), (2, [0, -1, 2]), (1, [0, 2 ** 31]),
+])
+def test_gather_host_offsets_are_one_per_table_row_and_one_more(rows, offsets):
+    # Refused before anything is read or launched: these are CPU tensors.
+    cache = torch.zeros(4, 16, 2, 8)
+    with pytest.raises(ValueError):
+        hip_gather_kv_host(cache, cache, torch.zeros(rows, 4, dtype=torch.int32), offsets)
