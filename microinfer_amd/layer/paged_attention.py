@@ -39,6 +39,8 @@ def gather_paged_kv(key_cache, value_cache, block_tables, contexts, block_size):
 
     Same arguments as ``_gather_paged_kv`` (paged_attention.py:76): host-side
     ``contexts``; returns ``(keys, values)`` of shape ``[sum(contexts), Hkv, D]``.
+    Not under graph capture, which would fix the lengths: ``hip_gather_kv``
+    takes them from the device.
     """
     if block_size != key_cache.shape[1]:
         raise ValueError("block_size does not match the cache")
@@ -51,6 +53,8 @@ def gather_paged_kv(key_cache, value_cache, block_tables, contexts, block_size):
     offsets = [0]
     for length in contexts:
         offsets.append(offsets[-1] + length)
+    if key_cache.is_cuda and torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("gather_paged_kv takes its lengths from the host: not under capture")
     tables = block_tables[: len(contexts)]
     if (len(contexts) == tables.shape[0] <= GATHER_HOST_REQUESTS
             and offsets[-1] <= _INT32_MAX):

@@ -103,6 +103,23 @@ def test_gather_rejects_short_tables():
                         torch.tensor([[0]], dtype=torch.int32, device=DEV), [5], 4)
 
 
+@pytest.mark.parametrize("requests", [1, 65])
+def test_gather_of_host_lengths_is_refused_under_capture(requests):
+    cache = KVCache(1, 80, 16, 2, 64, dtype=torch.float16, device=DEV)
+    tables = torch.arange(requests, dtype=torch.int32, device=DEV)[:, None]
+    contexts = [3] * requests
+    cache.keys[0].fill_(1)
+    keys, _ = gather_paged_kv(cache.keys[0], cache.values[0], tables, contexts, 16)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError):
+            gather_paged_kv(cache.keys[0], cache.values[0], tables, contexts, 16)
+        doubled = keys * 2
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(doubled, keys * 2)
+
+
 @pytest.mark.parametrize("requests", [1, 64, 65])
 def test_gather_host_and_device_offsets_agree(requests):
     # Up to 64 requests' offsets travel with the launch, more are uploaded.
