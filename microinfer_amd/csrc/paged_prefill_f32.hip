@@ -28,9 +28,12 @@
 //    scores have used the registers: each half hides the other's loads.
 //
 // Chunks of 118 / 325 / 210 rows on contexts of 155 / 325 / 359 (16 / 8
-// heads), graph-replayed: 27.5 us a launch, 76.3 on the vector kernel; 1000
-// rows on 1700 keys: 127 us, 77 TFLOP/s. Error against 64 bits 1.5e-7, as
-// the vector kernel's (1.4e-7), through short summation chains.
+// heads), a pass of four layers: 28.2 us a launch, 76.5 on the vector kernel;
+// 1000 rows on 1700 keys: 132 us, 74 TFLOP/s. Error against 64 bits, geometric mean
+// over 25 cases of 8 to 937 rows on up to 1100 keys: 1.17e-7, the vector
+// kernel's 1.20e-7, through summation chains of 8 terms and a scale that is
+// applied to a score and its maximum in one rounding (chains of 16 and two
+// roundings: 1.31e-7; 27.3 and 143 us).
 #include "paged_attention.h"
 
 namespace mi {
@@ -159,7 +162,7 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
 
   int nonfinite = 0;
   f32x4_t kf[8];
-    bool ok = false;
+  bool ok = false;
   int64_t base = 0;
   if (wave < ntiles) {
     base = tile_base(wave, tile_block(wave), ok);
@@ -179,16 +182,16 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
     }
     // The compiler would sink these loads below the products that hide them.
     __builtin_amdgcn_sched_barrier(0);
-    // Eight chains of 16 terms, added as a tree: a score's rounding error is
-    // that of short sums (one chain of 128 had 1.6 times the error).
+    // Sixteen chains of 8 terms, added as a tree: a score's rounding error is
+    // that of short sums.
     f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 4; ++h) {
       f32x4_t c[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) c[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 4 * h; j < 4 * h + 4; ++j)
+      for (int j = 2 * h; j < 2 * h + 2; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           c[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[j][e], c[e], 0, 0, 0);
@@ -203,12 +206,11 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
     // s[i]: key p0 + 4 quad + i, query row `col`.
     const bool masked = !ok || p0 + kRows > keys_all;  // uniform
     const int lim = masked ? (ok ? limit : 0) : INT32_MAX;
-    float sc[4], tmax = -INFINITY;
+    float tmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float v = s[i] * a.scale_log2;
-      sc[i] = p0 + 4 * quad + i < lim ? v : -INFINITY;
-      tmax = fmaxf(tmax, sc[i]);
+      if (p0 + 4 * quad + i >= lim) s[i] = -INFINITY;
+      tmax = fmaxf(tmax, s[i] * a.scale_log2);
     }
     tmax = fmaxf(tmax, swap16(tmax, lane));
     tmax = fmaxf(tmax, swap32(tmax, lane));
@@ -223,10 +225,8 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
     const float base_m = m == -INFINITY ? 0.f : m;
     float pr[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pr[i] = fast_exp2(sc[i] - base_m);
-      l += pr[i];
-    }
+    for (int i = 0; i < 4; ++i) pr[i] = fast_exp2(fmaf(s[i], a.scale_log2, -base_m));
+    l += (pr[0] + pr[1]) + (pr[2] + pr[3]);
     if (masked) {
       // A key no row sees weighs 0, but 0 * NaN is NaN: its V becomes 0. A
       // non-finite V that only some rows see must not reach the others: the
@@ -249,19 +249,25 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
         break;
       }
     }
-    // The tile's own sums, then added to the running ones (short chains again).
+    // The tile's own sums, in two halves, then added to the running ones
+    // (short chains again).
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      f32x4_t c[4];
+      f32x4_t c[2][4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) c[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int e = 0; e < 4; ++e) c[h][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          c[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][j][e], pr[i], c[e], 0, 0, 0);
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[4 * j + e] += c[e];
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            c[h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[2 * h + i][j][e], pr[2 * h + i],
+                                                           c[h][e], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[4 * j + e] += c[0][e] + c[1][e];
     }
     ok = next_ok;
     base = next_base;
