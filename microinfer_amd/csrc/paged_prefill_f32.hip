@@ -284,12 +284,14 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
       float mr = -INFINITY, lr = 0.f, oa = 0.f, ob = 0.f;
       for (int p = 0; p < seen; ++p) {
         bool ok;
-        const int64_t off = tile_base(p / kRows, tile_block(p / kRows), ok) + p % kRows * a.c_ts + 2 * lane;
+        const int64_t off =
+            tile_base(p / kRows, tile_block(p / kRows), ok) + p % kRows * a.c_ts + 2 * lane;
         if (!ok) continue;
         const float sc = xor_sum<1, kWave>(fmaf(qb, kc[off + 1], qa * kc[off])) * a.scale_log2;
         const float mnew = fmaxf(mr, sc);
-        const float alpha = mnew == -INFINITY ? 1.f : fast_exp2(mr - mnew);
-        const float w = fast_exp2(sc - mnew);
+        const float base_r = mnew == -INFINITY ? 0.f : mnew;  // -inf scores weigh 0
+        const float alpha = fast_exp2(mr - base_r);
+        const float w = fast_exp2(sc - base_r);
         mr = mnew;
         lr = fmaf(lr, alpha, w);
         oa = fmaf(w, vc[off], oa * alpha);

@@ -122,3 +122,21 @@ def test_error_against_64_bits_is_the_vector_kernels():
         vector = _run(q, *narrow, halves.contiguous(), cu_q, cu_k).double() - exact
         log_ratio += math.log(float(mfma.norm() / vector.norm()))
     assert math.exp(log_ratio / len(cases)) <= 1.03
+
+
+def test_rows_taken_one_by_one_weigh_scores_of_minus_infinity_by_zero():
+    """A NaN in V that only some rows see sends a workgroup's rows through the
+    serial path; scores of -inf before any finite one are still weights of 0."""
+    q_lens, prefixes = [400], [30]
+    q, kc, vc, tables, contexts, cu_q, cu_k = _paged_case(q_lens, prefixes, 16, 8, 16,
+                                                          torch.float32, 9)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    kc[tables[0, 0].item(), :3, :, 0] = -math.inf  # positions 0-2
+    want = _exact(q, kc, vc, tables, contexts, cu_q)
+    assert bool(want.isfinite().all())
+    vc[tables[0, 50 // 16].item(), 50 % 16, 3, 7] = float("nan")  # seen by rows 20.. only
+    got = _run(q, kc, vc, tables, cu_q, cu_k).double()
+    bad = torch.zeros_like(got, dtype=torch.bool)
+    bad[20:, 6:8, 7] = True
+    assert bool(got[bad].isnan().all())
+    assert float((got - want)[~bad].abs().max()) <= TOL
