@@ -155,9 +155,17 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_attention_vector_kernel(c
   const int lb = paged ? a.log2_block : 30;
   const int bmask = paged ? a.block_size - 1 : (1 << 30) - 1;
   // Scalar part of a row address (block, row-in-block, head) + per-lane part
-  // (row within the load group, column). Masked loads read row 0 of block 0.
+  // (row within the load group, column). Masked loads read the first row of
+  // the partition, whose weight of 0 a finite value keeps at 0 (another
+  // request's row, or an unused one, may hold NaN).
   const int64_t head_off = head * a.c_hs + row0 * a.c_ts;
-  const int64_t safe_head_off = head * a.c_hs;
+  int64_t safe_head_off = head * a.c_hs;
+  if (paged) {
+    const int blk = trow[max(min(blk_begin, a.t_width - 1), 0)];
+    if (blk > 0 && blk < a.num_blocks) safe_head_off += blk * a.c_bs;
+  } else if (row0 > 0 && row0 < a.num_blocks) {
+    safe_head_off += row0 * a.c_ts;
+  }
   const int lane_off = grp * static_cast<int>(a.c_ts) + d0;
   int pos_begin, pos_end;
   if (paged) {
@@ -246,8 +254,9 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_attention_vector_kernel(c
       float tmax = s[0][g];
 #pragma unroll
       for (int u = 1; u < UNROLL; ++u) tmax = fmaxf(tmax, s[u][g]);
-      const float mnew = fmaxf(m[g], tmax);
-      const float alpha = (mnew == -INFINITY) ? 1.f : fast_exp2(m[g] - mnew);
+      // Finite from the first tile on, so that scores of -inf weigh 0.
+      const float mnew = fmaxf(fmaxf(m[g], tmax), -3.4e38f);
+      const float alpha = fast_exp2(m[g] - mnew);
       m[g] = mnew;
       lsum[g] *= alpha;
 #pragma unroll

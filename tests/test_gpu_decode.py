@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 import torch
 
-from microinfer_amd.layer.hip_paged_attention import hip_paged_decode
+from microinfer_amd.layer.hip_paged_attention import hip_paged_decode, hip_paged_prefill
 from microinfer_amd.runner import capture_graph
 from microinfer_amd.worker.kv_cache import KVCache
 from microinfer_amd.workloads import QWEN3_06B, QWEN3_8B, make_decode_batch
@@ -373,3 +373,44 @@ def test_many_sequences_take_half_width_groups(dtype, hq, hkv, d):
     assert torch.equal(kc2, kc) and torch.equal(vc2, vc)
     expected = oracle_decode(q, kc, vc, t, lens, 1 / math.sqrt(d))
     assert max_abs(fused, expected) <= TOLERANCE[dtype]
+
+
+@pytest.mark.parametrize("dtype,head_dim,hq", [(torch.float32, 128, 16), (torch.float32, 128, 8),
+                                               (torch.bfloat16, 64, 8)])
+def test_vector_kernel_reads_nothing_into_masked_positions(dtype, head_dim, hq):
+    """NaN everywhere but in the contexts (block 0 is no request's), and scores
+    of -inf for the first 40 positions of the longest: both weigh nothing, in
+    decode and in prefill (float32: few rows)."""
+    contexts, hkv, bs = [1, 5, 33, 300, 70], 8, 16
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    need = [-(-c // bs) for c in contexts]
+    tables = torch.full((len(contexts), max(need)), -1, dtype=torch.int32)
+    kc, vc = (torch.full((sum(need) + 1, bs, hkv, head_dim), float("nan"), dtype=dtype, device=DEV)
+              for _ in range(2))
+    at = 1
+    for r, (c, n) in enumerate(zip(contexts, need)):
+        tables[r, :n] = torch.arange(at, at + n, dtype=torch.int32)
+        for pool in (kc, vc):
+            rows = pool[at:at + n].view(n * bs, hkv, head_dim)
+            rows[:c] = torch.randn(c, hkv, head_dim, generator=gen, device=DEV).to(dtype)
+        at += n
+    q = torch.randn(len(contexts), hq, head_dim, generator=gen, device=DEV).to(dtype)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    kc.view(-1, hkv, head_dim)[int(tables[3, 0]) * bs:, :, 0][:40] = -math.inf
+    tables = tables.to(DEV)
+    lens = torch.tensor(contexts, dtype=torch.int32, device=DEV)
+    scale = head_dim ** -0.5
+    want = torch.empty(q.shape, dtype=torch.float64, device=DEV)
+    for r, c in enumerate(contexts):
+        k, v = (p[tables[r, :need[r]].long()].reshape(-1, hkv, head_dim)[:c].double()
+                .repeat_interleave(hq // hkv, 1) for p in (kc, vc))
+        s = (q[r].double()[None] * k).sum(-1) * scale
+        want[r] = (torch.softmax(s, 0)[..., None] * v).sum(0)
+    assert bool(want.isfinite().all())
+    cu_q = torch.arange(len(contexts) + 1, dtype=torch.int32, device=DEV)
+    cu_k = torch.tensor([0, *torch.tensor(contexts).cumsum(0).tolist()], dtype=torch.int32,
+                        device=DEV)
+    tol = 2e-5 if dtype == torch.float32 else 2e-2
+    for got in (hip_paged_decode(q, kc, vc, tables, lens, scale=scale),
+                hip_paged_prefill(q, kc, vc, cu_q, cu_k, tables, max_seqlen_q=1, scale=scale)):
+        assert float((got.double() - want).abs().max()) <= tol
