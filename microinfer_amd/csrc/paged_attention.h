@@ -84,8 +84,10 @@ int32_t launch_prefill_mfma_planned(AttnArgs args, int32_t dtype, void* workspac
                                     bool plan_ready, hipStream_t stream);
 
 // float32 MFMA varlen kernel (paged_prefill_f32.hip): float32 with head_dim
-// 128, contiguous K/V or a block size of at least 16.
+// 128, contiguous K/V or a block size of at least 16; preferred where it is
+// the faster one.
 bool prefill_f32_supported(const AttnArgs& args, int32_t dtype);
+bool prefill_f32_preferred(const AttnArgs& args);
 int32_t launch_prefill_f32(const AttnArgs& args, hipStream_t stream);
 
 // Norm and rotation of the fused QKV rows [q heads | k heads | v heads] that

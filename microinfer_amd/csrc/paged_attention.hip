@@ -342,7 +342,7 @@ int32_t paged_prefill(
   a.varlen = 1;
   // bf16/f16 with head_dim 128 and GQA groups 1, 2, 4 run on MFMA (planned
   // when a workspace is given), float32 with head_dim 128 on the float32
-  // MFMA; every other supported shape on the vector kernel.
+  // MFMA unless the rows are few; every other supported shape on the vector kernel.
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (prefill_mfma_supported(a, dtype)) {
     if (workspace == nullptr) return launch_prefill_mfma(a, dtype, s);
@@ -354,7 +354,7 @@ int32_t paged_prefill(
     return launch_prefill_mfma_planned(a, dtype, workspace, (flags & MI_PREFILL_PLAN_READY) != 0,
                                        s);
   }
-  if (prefill_f32_supported(a, dtype)) return launch_prefill_f32(a, s);
+  if (prefill_f32_supported(a, dtype) && prefill_f32_preferred(a)) return launch_prefill_f32(a, s);
   return dispatch_vector(a, dtype, s);
 }
 }  // namespace

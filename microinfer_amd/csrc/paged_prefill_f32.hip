@@ -362,6 +362,36 @@ bool prefill_f32_supported(const AttnArgs& a, int32_t dtype) {
              (int64_t(1) << 31);
 }
 
+// Few rows go to the vector kernel: a workgroup per (row, KV head) whose waves
+// share the keys fills the chip where tiles of 16 rows leave most of it idle.
+// It needs a round per CU's worth of workgroups and reads K and V once for
+// each, so its reach falls with the group (heads on one read), the rounds and
+// the keys. Measured, us a launch, vector / MFMA, 8 KV heads:
+//   one head a group: 8 rows, 256 keys 8.5 / 14.1, 4000 keys 64 / 96; 48 rows
+//     128 / 512 / 1024 keys 8.4 / 11.9, 18.7 / 20.9, 31.3 / 32.6, 4000 keys
+//     100 / 96; 128 rows 128 / 256 keys 11.4 / 11.9, 18.1 / 15.2;
+//   two: 32 rows, 4000 keys 78 / 98; 64 rows 256 / 512 keys 13.9 / 15.2, 22.5
+//     / 21.1; 80 rows, 128 keys 12.2 / 11.9;
+//   four: 32 rows 256 / 512 keys 14.5 / 15.6, 22.3 / 21.1; 40 rows, 64 keys
+//     11.2 / 9.6. Eight: MFMA from 16 keys on (9.4 / 9.3).
+// At 2 KV heads, the same workgroups, likewise, except that the rows of a
+// request then lie on several XCDs and each reads its K and V for itself: many
+// requests of 4 rows and 300 keys, 128 / 192 / 256 / 320 workgroups 11.7 /
+// 15.2, 14.3 / 15.3, 16.9 / 15.4, 21 / 15.7 (8 KV heads, 320: 13.7 / 15.8).
+// The keys are the most that the table or the rows can hold: the contexts are
+// on the device.
+bool prefill_f32_preferred(const AttnArgs& a) {
+  const int64_t groups = static_cast<int64_t>(a.num_rows) * a.num_kv_heads;
+  if (a.num_kv_heads % 8 != 0 && a.num_seqs > 8 && 4 * groups > 3 * device_cus()) return true;
+  const int64_t rounds = (groups + device_cus() - 1) / device_cus();
+  const int64_t keys = a.tables != nullptr ? static_cast<int64_t>(a.t_width) * a.block_size
+                                           : static_cast<int64_t>(a.num_blocks);
+  if (a.group == 1) return rounds > 1 && keys > (rounds <= 2 ? 1024 : rounds <= 4 ? 128 : 0);
+  if (a.group == 2) return rounds > 1 && keys > (rounds <= 2 ? 256 : 0);
+  if (a.group == 4) return rounds > 1 || keys > 256;
+  return true;
+}
+
 int32_t launch_prefill_f32(const AttnArgs& a, hipStream_t stream) {
   // Every request's rows / 16, rounded up, fit in this many tiles.
   const int64_t tiles = static_cast<int64_t>(a.num_rows) * a.group / kRows + a.num_seqs;

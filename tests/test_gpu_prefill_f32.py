@@ -140,3 +140,25 @@ def test_rows_taken_one_by_one_weigh_scores_of_minus_infinity_by_zero():
     bad[20:, 6:8, 7] = True
     assert bool(got[bad].isnan().all())
     assert float((got - want)[~bad].abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("paged", [True, False])
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (32, 8), (64, 8), (4, 2), (4, 4)])
+def test_few_and_many_rows_agree(hq, hkv, paged):
+    """The rows at which the vector kernel hands over to the matrix cores
+    (2 to 4 workgroups per CU of rows x KV heads, by the group and the keys):
+    the same request, alone and as the last of enough rows."""
+    for rows, prefix in ((32, 0), (33, 200), (64, 900), (65, 10), (129, 0)):
+        prefix = prefix if paged else 0
+        q, kc, vc, tables, contexts, cu_q, cu_k = _paged_case([rows, 400], [prefix, 0], hq, hkv, 16,
+                                                              torch.float32, rows)
+        want = _exact(q, kc, vc, tables, contexts, cu_q)
+        for n, cut in ((1, rows), (2, rows + 400)):
+            part = tables[:n, :-(-max(contexts[:n]) // 16)].contiguous()
+            if paged:
+                got = _run(q[:cut], kc, vc, part, cu_q[:n + 1], cu_k[:n + 1])
+            else:
+                k, v = (torch.cat([p[tables[r, :-(-c // 16)].long()].reshape(-1, hkv, D)[:c]
+                                   for r, c in enumerate(contexts[:n])]) for p in (kc, vc))
+                got = _run(q[:cut], k, v, None, cu_q[:n + 1], cu_k[:n + 1])
+            assert float((got.double() - want[:cut]).abs().max()) <= TOL
