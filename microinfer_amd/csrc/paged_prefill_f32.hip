@@ -28,12 +28,12 @@
 //    scores have used the registers: each half hides the other's loads.
 //
 // Chunks of 118 / 325 / 210 rows on contexts of 155 / 325 / 359 (16 / 8
-// heads), a pass of four layers: 28.2 us a launch, 76.5 on the vector kernel;
-// 1000 rows on 1700 keys: 132 us, 74 TFLOP/s. Error against 64 bits, geometric mean
-// over 25 cases of 8 to 937 rows on up to 1100 keys: 1.17e-7, the vector
-// kernel's 1.20e-7, through summation chains of 8 terms and a scale that is
-// applied to a score and its maximum in one rounding (chains of 16 and two
-// roundings: 1.31e-7; 27.3 and 143 us).
+// heads), a pass of four layers: 27.3 us a launch, 76.5 on the vector kernel;
+// 1000 rows on 1700 keys: 138 us, 71 TFLOP/s. Error against 64 bits, geometric
+// mean over 25 cases of 8 to 937 rows on up to 1100 keys: 1.196e-7, the vector
+// kernel's 1.201e-7, through short summation chains, a score scaled and its
+// maximum subtracted in one rounding, and a division at the end (one chain of
+// 16 for a tile's P.V, two roundings and a reciprocal: 1.31e-7).
 #include "paged_attention.h"
 
 namespace mi {
@@ -182,16 +182,16 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
     }
     // The compiler would sink these loads below the products that hide them.
     __builtin_amdgcn_sched_barrier(0);
-    // Sixteen chains of 8 terms, added as a tree: a score's rounding error is
+    // Eight chains of 16 terms, added as a tree: a score's rounding error is
     // that of short sums.
     f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
+    for (int h = 0; h < 2; ++h) {
       f32x4_t c[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) c[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 2 * h; j < 2 * h + 2; ++j)
+      for (int j = 4 * h; j < 4 * h + 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           c[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[j][e], c[e], 0, 0, 0);
@@ -250,25 +250,28 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
       }
     }
     // The tile's own sums, in two halves, then added to the running ones
-    // (short chains again).
+    // (short chains again). Two of four blocks at a time: with all four the
+    // kernel passes 168 registers, a wave less per SIMD and 15 % more time.
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      f32x4_t c[2][4];
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[h][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int e0 = 0; e0 < 4; e0 += 2) {
+        f32x4_t c[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            c[h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[2 * h + i][j][e], pr[2 * h + i],
-                                                           c[h][e], 0, 0, 0);
+          for (int e = 0; e < 2; ++e) c[h][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[4 * j + e] += c[0][e] + c[1][e];
-    }
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+              c[h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[2 * h + i][j][e0 + e],
+                                                             pr[2 * h + i], c[h][e], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) o[4 * j + e0 + e] += c[0][e] + c[1][e];
+      }
     ok = next_ok;
     base = next_base;
   }
@@ -338,9 +341,11 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum[e] = fmaf(f, part[e], sum[e]);
     }
-    const float inv = ls > 0.f ? 1.f / ls : 0.f;
+    f32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = ls > 0.f ? sum[e] / ls : 0.f;
     *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.out) + (q0 + rr / G) * a.o_ts +
-                                (head * G + rr % G) * a.o_hs + d) = sum * inv;
+                                (head * G + rr % G) * a.o_hs + d) = out;
   }
 }
 
