@@ -23,21 +23,31 @@ namespace {
 // arguments.
 constexpr int32_t kTargetItems = 192;
 // Merging partitions costs a launch about 2.5 us and more with their number,
-// so a part covers at least kMinPartBlocks cache blocks, and an eighth of the
-// longest sequence up to kMaxMinPart (one sequence of 2000 tokens, 16-token
-// blocks: 9.0 us with parts of 16, 9.9 of 8, 11.0 of 4; of 1000: 8.1 of 8,
-// 8.7 of 16, 9.3 of 4; of 300: 6.9 of 4, 7.2 of 8).
-constexpr int32_t kMinPartBlocks = 4;
-constexpr int32_t kMaxMinPart = 32;
+// so a part covers an eighth of the longest sequence, but at least
+// kMinPartPositions, and at most kMaxMinPart of up to kLongPositions and in
+// proportion of longer ones; or as many as make kTargetItems. In positions,
+// whatever the block size (at least one block): at 16, 64 and 256 tokens a
+// block, parts of as many positions measured the same. One sequence, 8 KV
+// heads, us with parts of 64 / 128 / 256 / 512 positions: of 300 tokens 7.0 /
+// 7.4 / 8.4 / -, 1000 9.2 / 8.1 / 8.7 / 10.4, 2000 (96) 11.2 / 10.1 / 9.1 /
+// 10.6, 4096 (176) 12.3 / - / 11.0 / 10.9, 8192 (352) 14.1 / - / - / 12.9,
+// with 768 14.0; 2 KV heads, 256 / 512 / 1024: 4096 13.1 / 13.1 / 16.0, 16384
+// 26.3 / 19.3 / 18.5, 32768 (352) 35.8 / 28.0 / 22.9.
+constexpr int32_t kMinPartPositions = 64;
+constexpr int32_t kMaxMinPart = 512;
+constexpr int32_t kLongPositions = 16384;
 // Sequences of up to this many positions are one item (one sequence of 130
 // tokens 5.5 us whole, 6.8 in parts; float32 6.8, 9.3), and longer ones where
 // the sequences alone make workgroups for a quarter of the chip (8 of 215: 6.9
 // whole, 8.5 in parts; float32 8.5, 10.8). One CU streams a cold context more
 // slowly than several: at 300 and at 512 the whole 300-token sequence of a
 // decode step and eight float32 ones of 64-512 lost (181 against 179 us for
-// four layers, 153 against 133 for eight).
+// four layers, 153 against 133 for eight). Up to kWholeBlocks blocks of up to
+// kMaxMinPart positions too, whose parts would be few and uneven (300 tokens
+// in blocks of 256: 7.3 whole, 8.8 in two; 200 in blocks of 64: 6.7, 7.4).
 constexpr int32_t kWholePositions = 160;
 constexpr int32_t kWholePositionsMany = 256;
+constexpr int32_t kWholeBlocks = 4;
 constexpr int32_t kManyItems = 64;
 
 // Four waves: fewer waves per barrier than 1024 threads (0.06 us less per
@@ -57,15 +67,18 @@ __device__ __forceinline__ int part_blocks(int nb, int split_k, int pb_global, i
 }
 
 // The step's part size from its blocks in all and its longest sequence's.
-__device__ __forceinline__ int step_part_blocks(int64_t total_blocks, int longest,
+__device__ __forceinline__ int step_part_blocks(int64_t total_blocks, int longest, int lb,
                                                 int num_kv_heads, int target) {
   const int64_t want = total_blocks * num_kv_heads;
-  const int least = min(max(longest / 8, kMinPartBlocks), kMaxMinPart);
-  return max(least, static_cast<int>((want + target - 1) / target));
+  const int most = max(kMaxMinPart >> lb, longest / (kLongPositions / kMaxMinPart));
+  const int least = min(max(longest / 8, kMinPartPositions >> lb), most);
+  return max(max(least, 1), static_cast<int>((want + target - 1) / target));
 }
 
 __device__ __forceinline__ int whole_blocks(int num_seqs, int num_kv_heads, int lb) {
-  return (num_seqs * num_kv_heads >= kManyItems ? kWholePositionsMany : kWholePositions) >> lb;
+  const int positions =
+      num_seqs * num_kv_heads >= kManyItems ? kWholePositionsMany : kWholePositions;
+  return max(positions >> lb, min(kWholeBlocks, kMaxMinPart >> lb));
 }
 
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
@@ -107,7 +120,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   atomicMax(&s_longest, longest);
   __syncthreads();
   const int pb_global =
-      split_k == 0 ? step_part_blocks(s_total_blocks, s_longest, num_kv_heads, target) : 1;
+      split_k == 0 ? step_part_blocks(s_total_blocks, s_longest, lb, num_kv_heads, target) : 1;
 
   // Rank sequences by block count, longest first (ties keep batch order).
   const bool sort = num_seqs <= kSortLimit;
@@ -234,7 +247,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_wave_kernel(
   int longest = nb;
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) longest = max(longest, __shfl_xor(longest, o, kWave));
-  const int pb = step_part_blocks(wave_sum_int(nb), longest, num_kv_heads, target);
+  const int pb = step_part_blocks(wave_sum_int(nb), longest, lb, num_kv_heads, target);
   const int np = nb <= whole_blocks(num_seqs, num_kv_heads, lb) ? 1 : (nb + pb - 1) / pb;
   const int last = nb - (np - 1) * pb;  // blocks of the last part, the odd one
   // Over the sequences ahead of this lane's (longer, or as long and earlier

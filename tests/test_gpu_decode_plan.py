@@ -15,8 +15,12 @@ TARGET = 192
 
 def _expected(contexts, hkv, block_size):
     blocks = [-(-c // block_size) for c in contexts]
-    part = max(min(max(max(blocks) // 8, 4), 32), -(-sum(blocks) * hkv // TARGET))
-    whole = (256 if len(contexts) * hkv >= 64 else 160) // block_size
+    # 64 to 512 positions, past 16384 in proportion.
+    most = max(512 // block_size, max(blocks) // 32)
+    least = min(max(max(blocks) // 8, 64 // block_size), most)
+    part = max(least, 1, -(-sum(blocks) * hkv // TARGET))
+    whole = max((256 if len(contexts) * hkv >= 64 else 160) // block_size,
+                min(4, 512 // block_size))
     items, slot = [], 0
     for r in sorted(range(len(blocks)), key=lambda r: (-blocks[r], r)):
         parts = 1 if blocks[r] <= whole else -(-blocks[r] // part)
@@ -28,9 +32,9 @@ def _expected(contexts, hkv, block_size):
     return [i[2] for i in sorted(items, key=lambda i: (-i[0], i[1]))]
 
 
-@pytest.mark.parametrize("hkv,block_size", [(8, 16), (1, 16), (2, 64)])
+@pytest.mark.parametrize("hkv,block_size", [(8, 16), (1, 16), (2, 64), (8, 256), (4, 8), (8, 1024)])
 @pytest.mark.parametrize("contexts", [
-    [1], [0, 0], [64, 65, 1], [32768], [5000, 16, 4999, 0, 16], [100] * 64,
+    [1], [0, 0], [64, 65, 1], [32768], [40000, 300], [5000, 16, 4999, 0, 16], [100] * 64,
     [161, 160, 130, 400, 1, 2000], [256, 257, 300, 129, 4000] * 3,
     list(range(1, 2049, 32)), [31 * i % 700 for i in range(65)],
 ])
@@ -42,3 +46,19 @@ def test_plan_items_and_order(contexts, hkv, block_size):
     want = _expected(contexts, hkv, block_size)
     assert got[:len(want)].tolist() == want
     assert (got[len(want):, 0] == -1).all()
+
+
+@pytest.mark.parametrize("context", [1000, 4096, 16384, 32768])
+def test_parts_cover_as_many_positions_at_every_block_size(context):
+    """The launch's workgroups depend on the context, not on how it is cut into
+    blocks: no part is longer than the 16-token blocks' by more than a block."""
+    longest = {}
+    for block_size in (16, 64, 256):
+        plan = decode_plan(torch.tensor([context], dtype=torch.int32, device="cuda"),
+                           num_kv_heads=8, block_size=block_size,
+                           block_table_width=-(-context // block_size))
+        items = plan.cpu().numpy().view(np.int32).reshape(-1, 8)
+        items = items[items[:, 0] >= 0]
+        assert (items[:, 2] - items[:, 1]).sum() == -(-context // block_size)
+        longest[block_size] = int((items[:, 2] - items[:, 1]).max()) * block_size
+    assert longest[64] <= longest[16] + 64 and longest[256] <= longest[16] + 256
