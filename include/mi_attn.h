@@ -132,6 +132,17 @@ int32_t mi_decode_plan(const int32_t* context_lens, int32_t num_seqs, int32_t nu
                        int32_t block_size, int32_t block_table_width, int32_t split_k,
                        void* plan, int64_t plan_bytes, void* stream);
 
+/*
+ * mi_decode_plan with the rest of the decode call's shape: partitions of the
+ * size that is best for the kernel it takes (the plan mi_paged_decode makes
+ * when it is given none). mi_decode_plan sizes them for 16-bit caches with
+ * head_dim 128; either plan gives the right result for every call.
+ */
+int32_t mi_decode_plan_for(const int32_t* context_lens, int32_t num_seqs, int32_t num_q_heads,
+                           int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                           int32_t block_size, int32_t block_table_width, int32_t split_k,
+                           void* plan, int64_t plan_bytes, void* stream);
+
 int32_t mi_paged_decode(const void* query, int64_t q_token_stride, int64_t q_head_stride,
                         const void* key_cache, const void* value_cache,
                         int64_t cache_block_stride, int64_t cache_token_stride,

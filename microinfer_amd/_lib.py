@@ -67,6 +67,8 @@ SIGNATURES = {
     ),
     "mi_decode_plan_bytes": (_I64, [_I32, _I32, _I32]),
     "mi_decode_plan": (_I32, [_P, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
+    "mi_decode_plan_for": (
+        _I32, [_P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I64, _P]),
     "mi_paged_prefill": (
         _I32,
         [_P, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P, _P, _I64, _I32, _P, _I64,

@@ -33,8 +33,14 @@ constexpr int32_t kTargetItems = 192;
 // 10.6, 4096 (176) 12.3 / - / 11.0 / 10.9, 8192 (352) 14.1 / - / - / 12.9,
 // with 768 14.0; 2 KV heads, 256 / 512 / 1024: 4096 13.1 / 13.1 / 16.0, 16384
 // 26.3 / 19.3 / 18.5, 32768 (352) 35.8 / 28.0 / 22.9.
+// The vector kernel goes through a part's positions more slowly: half as many
+// (float32, 8 KV heads, 128 / 256 / 512: 2000 tokens 12.3 / 12.0 / 16.3, 4096
+// (176) 16.4 / 14.6 / 16.6; 2 KV heads, 4096 31.4 / 31.4 / 40.7, 8192 44 / 38
+// / 44, 32768 (352) 69 / - / 62; head_dim 64 bf16 16.8 / 15.8 / 16.3 at 4096,
+// float32 13.7 / 12.4 / 15.7, head_dim 256 bf16 32.6 / 28.3 / 33.2).
 constexpr int32_t kMinPartPositions = 64;
 constexpr int32_t kMaxMinPart = 512;
+constexpr int32_t kMaxMinPartVector = 256;
 constexpr int32_t kLongPositions = 16384;
 // Sequences of up to this many positions are one item (one sequence of 130
 // tokens 5.5 us whole, 6.8 in parts; float32 6.8, 9.3), and longer ones where
@@ -68,9 +74,9 @@ __device__ __forceinline__ int part_blocks(int nb, int split_k, int pb_global, i
 
 // The step's part size from its blocks in all and its longest sequence's.
 __device__ __forceinline__ int step_part_blocks(int64_t total_blocks, int longest, int lb,
-                                                int num_kv_heads, int target) {
+                                                int num_kv_heads, int target, int max_min_part) {
   const int64_t want = total_blocks * num_kv_heads;
-  const int most = max(kMaxMinPart >> lb, longest / (kLongPositions / kMaxMinPart));
+  const int most = max(max_min_part >> lb, longest / (kLongPositions / max_min_part));
   const int least = min(max(longest / 8, kMinPartPositions >> lb), most);
   return max(max(least, 1), static_cast<int>((want + target - 1) / target));
 }
@@ -83,7 +89,7 @@ __device__ __forceinline__ int whole_blocks(int num_seqs, int num_kv_heads, int 
 
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
     const int32_t* __restrict__ context_lens, int num_seqs, int num_kv_heads, int block_size,
-    int lb, int width, int split_k, int target, int max_items,
+    int lb, int width, int split_k, int target, int max_min_part, int max_items,
     PlanItem* __restrict__ plan, int32_t* __restrict__ counters, int num_counters) {
   __shared__ int s_ctx[kMaxPlanSeqs];
   __shared__ int s_order[kMaxPlanSeqs];  // rank -> sequence
@@ -120,7 +126,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
   atomicMax(&s_longest, longest);
   __syncthreads();
   const int pb_global =
-      split_k == 0 ? step_part_blocks(s_total_blocks, s_longest, lb, num_kv_heads, target) : 1;
+      split_k == 0 ? step_part_blocks(s_total_blocks, s_longest, lb, num_kv_heads, target,
+                                    max_min_part) : 1;
 
   // Rank sequences by block count, longest first (ties keep batch order).
   const bool sort = num_seqs <= kSortLimit;
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(
 // 128-2048 8.6 -> 4.5.
 __global__ __launch_bounds__(kPlanThreads) void decode_plan_wave_kernel(
     const int32_t* __restrict__ context_lens, int num_seqs, int num_kv_heads, int block_size,
-    int lb, int width, int target, int max_items, PlanItem* __restrict__ plan,
+    int lb, int width, int target, int max_min_part, int max_items, PlanItem* __restrict__ plan,
     int32_t* __restrict__ counters, int num_counters) {
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
@@ -247,7 +254,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_wave_kernel(
   int longest = nb;
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) longest = max(longest, __shfl_xor(longest, o, kWave));
-  const int pb = step_part_blocks(wave_sum_int(nb), longest, lb, num_kv_heads, target);
+  const int pb = step_part_blocks(wave_sum_int(nb), longest, lb, num_kv_heads, target,
+                                    max_min_part);
   const int np = nb <= whole_blocks(num_seqs, num_kv_heads, lb) ? 1 : (nb + pb - 1) / pb;
   const int last = nb - (np - 1) * pb;  // blocks of the last part, the odd one
   // Over the sequences ahead of this lane's (longer, or as long and earlier
@@ -323,17 +331,18 @@ int64_t decode_plan_bytes(int32_t num_seqs, int32_t num_kv_heads, int32_t split_
 
 int32_t launch_decode_plan(const int32_t* context_lens, int32_t num_seqs, int32_t num_kv_heads,
                            int32_t block_size, int32_t block_table_width, int32_t split_k,
-                           PlanItem* plan, int32_t* counters, hipStream_t stream) {
+                           bool vector, PlanItem* plan, int32_t* counters, hipStream_t stream) {
+  const int32_t max_min_part = vector ? kMaxMinPartVector : kMaxMinPart;
   if (num_seqs <= kWave && split_k == 0) {
     decode_plan_wave_kernel<<<1, kPlanThreads, 0, stream>>>(
         context_lens, num_seqs, num_kv_heads, block_size, ilog2(block_size), block_table_width,
-        kTargetItems, decode_max_items(num_seqs, num_kv_heads, split_k), plan,
+        kTargetItems, max_min_part, decode_max_items(num_seqs, num_kv_heads, split_k), plan,
         counters, counters != nullptr ? num_seqs * num_kv_heads : 0);
     return check_launch("decode plan");
   }
   decode_plan_kernel<<<1, kPlanThreads, 0, stream>>>(
       context_lens, num_seqs, num_kv_heads, block_size, ilog2(block_size), block_table_width,
-      split_k, kTargetItems,
+      split_k, kTargetItems, max_min_part,
       decode_max_items(num_seqs, num_kv_heads, split_k), plan, counters,
       counters != nullptr ? num_seqs * num_kv_heads : 0);
   return check_launch("decode plan");
@@ -347,25 +356,51 @@ extern "C" int64_t mi_decode_plan_bytes(int32_t num_seqs, int32_t num_kv_heads,
   return mi::decode_plan_bytes(num_seqs, num_kv_heads, split_k);
 }
 
+namespace {
+int32_t decode_plan(const char* who, const int32_t* context_lens, int32_t num_seqs,
+                    int32_t num_kv_heads, int32_t block_size, int32_t block_table_width,
+                    int32_t split_k, bool vector, void* plan, int64_t plan_bytes, void* stream) {
+  using namespace mi;
+  clear_error();
+  const std::string fn(who);
+  if (num_seqs < 0 || num_kv_heads <= 0 || split_k < 0 || block_table_width < 0)
+    return fail(MI_ERR_INVALID_ARGUMENT, fn + ": invalid sizes");
+  if (!is_pow2(block_size))
+    return fail(MI_ERR_INVALID_ARGUMENT, fn + ": block_size must be a power of two");
+  if (num_seqs > kMaxPlanSeqs)
+    return fail(MI_ERR_UNSUPPORTED, fn + ": more than 4096 sequences");
+  if (num_seqs == 0) return MI_OK;
+  if (!context_lens || !plan) return fail(MI_ERR_INVALID_ARGUMENT, fn + ": null pointer");
+  if (plan_bytes < decode_plan_bytes(num_seqs, num_kv_heads, split_k) ||
+      reinterpret_cast<uintptr_t>(plan) % 32 != 0)
+    return fail(MI_ERR_WORKSPACE, fn + ": plan buffer too small or misaligned");
+  return launch_decode_plan(context_lens, num_seqs, num_kv_heads, block_size,
+                            block_table_width, split_k, vector, static_cast<PlanItem*>(plan),
+                            nullptr, static_cast<hipStream_t>(stream));
+}
+}  // namespace
+
 extern "C" int32_t mi_decode_plan(const int32_t* context_lens, int32_t num_seqs,
                                   int32_t num_kv_heads, int32_t block_size,
                                   int32_t block_table_width, int32_t split_k, void* plan,
                                   int64_t plan_bytes, void* stream) {
-  using namespace mi;
-  clear_error();
-  if (num_seqs < 0 || num_kv_heads <= 0 || split_k < 0 || block_table_width < 0)
-    return fail(MI_ERR_INVALID_ARGUMENT, "mi_decode_plan: invalid sizes");
-  if (!is_pow2(block_size))
-    return fail(MI_ERR_INVALID_ARGUMENT, "mi_decode_plan: block_size must be a power of two");
-  if (num_seqs > kMaxPlanSeqs)
-    return fail(MI_ERR_UNSUPPORTED, "mi_decode_plan: more than 4096 sequences");
-  if (num_seqs == 0) return MI_OK;
-  if (!context_lens || !plan)
-    return fail(MI_ERR_INVALID_ARGUMENT, "mi_decode_plan: null pointer");
-  if (plan_bytes < decode_plan_bytes(num_seqs, num_kv_heads, split_k) ||
-      reinterpret_cast<uintptr_t>(plan) % 32 != 0)
-    return fail(MI_ERR_WORKSPACE, "mi_decode_plan: plan buffer too small or misaligned");
-  return launch_decode_plan(context_lens, num_seqs, num_kv_heads, block_size,
-                            block_table_width, split_k, static_cast<PlanItem*>(plan), nullptr,
-                            static_cast<hipStream_t>(stream));
+  return decode_plan("mi_decode_plan", context_lens, num_seqs, num_kv_heads, block_size,
+                     block_table_width, split_k, false, plan, plan_bytes, stream);
+}
+
+extern "C" int32_t mi_decode_plan_for(const int32_t* context_lens, int32_t num_seqs,
+                                      int32_t num_q_heads, int32_t num_kv_heads,
+                                      int32_t head_dim, int32_t dtype, int32_t block_size,
+                                      int32_t block_table_width, int32_t split_k, void* plan,
+                                      int64_t plan_bytes, void* stream) {
+  if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      head_dim <= 0 || !mi::valid_dtype(dtype)) {
+    mi::clear_error();
+    return mi::fail(MI_ERR_INVALID_ARGUMENT, "mi_decode_plan_for: invalid heads or dtype");
+  }
+  const int32_t group = num_q_heads / num_kv_heads;
+  return decode_plan("mi_decode_plan_for", context_lens, num_seqs, num_kv_heads, block_size,
+                     block_table_width, split_k,
+                     !mi::decode_mfma_takes(dtype, head_dim, group, block_size), plan, plan_bytes,
+                     stream);
 }

@@ -107,6 +107,7 @@ struct QkvRows {
 
 // MFMA decode kernel (paged_decode_mfma.hip): 16-bit caches, head_dim 128,
 // up to 16 query heads per KV head, block size >= 16, paged.
+bool decode_mfma_takes(int32_t dtype, int32_t head_dim, int32_t group, int32_t block_size);
 bool decode_mfma_supported(const AttnArgs& args, int32_t dtype);
 int32_t launch_decode_mfma(const AttnArgs& args, const QkvRows& qkv, int32_t dtype,
                            hipStream_t stream);
@@ -118,10 +119,11 @@ int32_t decode_max_items(int32_t num_seqs, int32_t num_kv_heads, int32_t split_k
 // entries; unused ones carry seq = -1.
 int64_t decode_plan_bytes(int32_t num_seqs, int32_t num_kv_heads, int32_t split_k);
 // counters (optional): the (sequence, KV head) arrival counters of the
-// decode launch that follows, zeroed by the plan kernel.
+// decode launch that follows, zeroed by the plan kernel. vector: the launch
+// runs on the vector kernel, not on MFMA.
 int32_t launch_decode_plan(const int32_t* context_lens, int32_t num_seqs, int32_t num_kv_heads,
                            int32_t block_size, int32_t block_table_width, int32_t split_k,
-                           PlanItem* plan, int32_t* counters, hipStream_t stream);
+                           bool vector, PlanItem* plan, int32_t* counters, hipStream_t stream);
 
 constexpr int32_t kMaxPlanSeqs = 4096;
 

@@ -166,8 +166,9 @@ int32_t paged_decode(
     // The plan kernel also zeroes the counters this launch uses.
     PlanItem* own = reinterpret_cast<PlanItem*>(ws);
     st = launch_decode_plan(context_lens, num_seqs, num_kv_heads, block_size,
-                            block_table_width, split_k, own, partials > 0 ? counters : nullptr,
-                            s);
+                            block_table_width, split_k,
+                            !decode_mfma_takes(dtype, head_dim, a.group, block_size), own,
+                            partials > 0 ? counters : nullptr, s);
     if (st != MI_OK) return st;
     a.plan = own;
   } else {

@@ -683,10 +683,14 @@ int32_t launch_typed(const ArgsOf<QKV>& a, hipStream_t stream) {
 
 }  // namespace
 
+bool decode_mfma_takes(int32_t dtype, int32_t head_dim, int32_t group, int32_t block_size) {
+  return (dtype == MI_DTYPE_BF16 || dtype == MI_DTYPE_F16) && head_dim == kD && group >= 1 &&
+         group <= kHeads && block_size >= kTile;
+}
+
 bool decode_mfma_supported(const AttnArgs& a, int32_t dtype) {
-  return (dtype == MI_DTYPE_BF16 || dtype == MI_DTYPE_F16) && !a.varlen &&
-         a.head_dim == kD && a.group >= 1 && a.group <= kHeads && a.tables != nullptr &&
-         a.block_size >= kTile && a.c_ts >= 0 && a.c_ts * kTile < (int64_t(1) << 30);
+  return decode_mfma_takes(dtype, a.head_dim, a.group, a.block_size) && !a.varlen &&
+         a.tables != nullptr && a.c_ts >= 0 && a.c_ts * kTile < (int64_t(1) << 30);
 }
 
 int32_t launch_decode_mfma(const AttnArgs& a, const QkvRows& qkv, int32_t dtype,

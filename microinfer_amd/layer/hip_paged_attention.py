@@ -103,12 +103,25 @@ def decode_workspace_bytes(num_seqs: int, num_q_heads: int, num_kv_heads: int,
     )
 
 
+def vector_heads(query: torch.Tensor, num_kv_heads: int, block_size: int):
+    """``(Hq, D, dtype)`` of a query ``[R, Hq, D]`` whose decode runs on the
+    vector kernel, None where it runs on MFMA (``decode_plan``'s ``heads``)."""
+    _, num_q_heads, head_dim = query.shape
+    mfma = (query.dtype in (torch.float16, torch.bfloat16) and head_dim == 128
+            and num_q_heads <= 16 * num_kv_heads and block_size >= 16)
+    return None if mfma else (num_q_heads, head_dim, query.dtype)
+
+
 def decode_plan(context_lens: torch.Tensor, *, num_kv_heads: int, block_size: int,
-                block_table_width: int, split_k: int | None = None) -> torch.Tensor:
+                block_table_width: int, split_k: int | None = None,
+                heads: tuple[int, int, torch.dtype] | None = None) -> torch.Tensor:
     """Partition plan for one decode step (shared by every layer of the step).
 
     Computed on the device from ``context_lens`` (int32 ``[R]``), so it can be
     captured in a hipGraph; pass it to ``hip_paged_decode(..., plan=...)``.
+    ``heads``: query heads, head_dim and dtype of the calls (``vector_heads``);
+    without it the partitions suit 16-bit caches with head_dim 128, and other
+    calls give the same result, more slowly on long contexts.
     """
     _lib.require_device(context_lens, what="decode_plan")
     context_lens = _index32(context_lens)
@@ -117,10 +130,14 @@ def decode_plan(context_lens: torch.Tensor, *, num_kv_heads: int, block_size: in
     lib = _lib.load()
     nbytes = int(lib.mi_decode_plan_bytes(num_seqs, num_kv_heads, split))
     plan = torch.empty(max(nbytes, 32), dtype=torch.uint8, device=context_lens.device)
-    status = lib.mi_decode_plan(
-        context_lens.data_ptr(), num_seqs, num_kv_heads, block_size, block_table_width, split,
-        plan.data_ptr(), plan.numel(), _lib.stream_handle(context_lens.device),
-    )
+    rest = (block_size, block_table_width, split, plan.data_ptr(), plan.numel(),
+            _lib.stream_handle(context_lens.device))
+    if heads is None:
+        status = lib.mi_decode_plan(context_lens.data_ptr(), num_seqs, num_kv_heads, *rest)
+    else:
+        num_q_heads, head_dim, dtype = heads
+        status = lib.mi_decode_plan_for(context_lens.data_ptr(), num_seqs, num_q_heads,
+                                        num_kv_heads, head_dim, _lib.dtype_code(dtype), *rest)
     _lib.check(status, "mi_decode_plan")
     return plan
 

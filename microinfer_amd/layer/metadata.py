@@ -96,18 +96,19 @@ class AttentionMetadata:
             self._slot_block_size = block_size
         return self._slot_blocks, self._slot_offsets
 
-    def decode_plan(self, num_kv_heads: int, block_size: int) -> torch.Tensor:
+    def decode_plan(self, num_kv_heads: int, block_size: int, heads=None) -> torch.Tensor:
         """Device partition plan for this decode step, built once and reused
-        by every layer (like ``slot_indices``)."""
+        by every layer (like ``slot_indices``). ``heads``: ``vector_heads`` of
+        the layer's query."""
         if self.context_lens is None or self.block_tables is None:
             raise ValueError("decode plan needs context_lens and block_tables")
         from microinfer_amd.layer.hip_paged_attention import decode_plan
 
-        key = (num_kv_heads, block_size, self.block_tables.shape[1])
+        key = (num_kv_heads, block_size, self.block_tables.shape[1], heads)
         plan = self._decode_plans.get(key)
         if plan is None:
             plan = decode_plan(self.context_lens, num_kv_heads=num_kv_heads,
-                               block_size=block_size, block_table_width=key[2])
+                               block_size=block_size, block_table_width=key[2], heads=heads)
             self._decode_plans[key] = plan
         return plan
 

@@ -27,6 +27,7 @@ from microinfer_amd.layer.hip_paged_attention import (
     hip_gather_kv_host,
     hip_paged_decode,
     hip_paged_prefill,
+    vector_heads,
 )
 from microinfer_amd.layer.metadata import AttentionMetadata
 
@@ -93,7 +94,9 @@ def paged_attention_meta(
             raise RuntimeError("decode metadata requires context_lens")
         plan = None
         if metadata.context_lens.is_cuda:
-            plan = metadata.decode_plan(key_cache.shape[2], key_cache.shape[1])
+            block_size, num_kv_heads = key_cache.shape[1:3]
+            plan = metadata.decode_plan(num_kv_heads, block_size,
+                                        vector_heads(query, num_kv_heads, block_size))
         return hip_paged_decode(
             query,
             key_cache,

@@ -98,6 +98,15 @@ def test_decode_plan_validation_and_size():
     assert lib.mi_decode_plan(None, 0, 8, 16, 128, 0, None, 0, None) == 0
 
 
+def test_decode_plan_for_validation():
+    lib = _lib.load()
+    fake = ctypes.c_void_p(1 << 20)
+    assert lib.mi_decode_plan_for(None, 0, 16, 8, 128, 0, 16, 128, 0, None, 0, None) == 0
+    assert lib.mi_decode_plan_for(fake, 32, 12, 8, 128, 0, 16, 128, 0, fake, 10 ** 6, None) == 1
+    assert lib.mi_decode_plan_for(fake, 32, 16, 8, 128, 9, 16, 128, 0, fake, 10 ** 6, None) == 1
+    assert lib.mi_decode_plan_for(fake, 32, 16, 8, 128, 0, 16, 128, 0, fake, 64, None) == 3
+
+
 @pytest.mark.parametrize("split_k", [1, 0, 4])
 def test_workspace_size_formula(split_k):
     lib = _lib.load()

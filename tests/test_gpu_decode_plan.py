@@ -7,16 +7,16 @@ import numpy as np
 import pytest
 import torch
 
-from microinfer_amd.layer.hip_paged_attention import decode_plan
+from microinfer_amd.layer.hip_paged_attention import decode_plan, hip_paged_decode, vector_heads
 
 pytestmark = pytest.mark.gpu
 TARGET = 192
 
 
-def _expected(contexts, hkv, block_size):
+def _expected(contexts, hkv, block_size, cap=512):
     blocks = [-(-c // block_size) for c in contexts]
-    # 64 to 512 positions, past 16384 in proportion.
-    most = max(512 // block_size, max(blocks) // 32)
+    # 64 to cap positions, past 16384 in proportion.
+    most = max(cap // block_size, max(blocks) // (16384 // cap))
     least = min(max(max(blocks) // 8, 64 // block_size), most)
     part = max(least, 1, -(-sum(blocks) * hkv // TARGET))
     whole = max((256 if len(contexts) * hkv >= 64 else 160) // block_size,
@@ -42,10 +42,40 @@ def test_plan_items_and_order(contexts, hkv, block_size):
     lens = torch.tensor(contexts, dtype=torch.int32, device="cuda")
     width = max(-(-max(contexts) // block_size), 1)
     plan = decode_plan(lens, num_kv_heads=hkv, block_size=block_size, block_table_width=width)
+    _assert_items(plan, _expected(contexts, hkv, block_size))
+    # The vector kernel's parts are half as long at most.
+    plan = decode_plan(lens, num_kv_heads=hkv, block_size=block_size, block_table_width=width,
+                       heads=(2 * hkv, 128, torch.float32))
+    _assert_items(plan, _expected(contexts, hkv, block_size, cap=256))
+
+
+def _assert_items(plan, want):
     got = plan.cpu().numpy().view(np.int32).reshape(-1, 8)
-    want = _expected(contexts, hkv, block_size)
     assert got[:len(want)].tolist() == want
     assert (got[len(want):, 0] == -1).all()
+
+
+@pytest.mark.parametrize("dtype,head_dim,block_size", [
+    (torch.float32, 128, 16), (torch.bfloat16, 128, 16), (torch.bfloat16, 64, 16),
+    (torch.bfloat16, 128, 8),
+])
+def test_a_call_without_a_plan_makes_the_shape_s(dtype, head_dim, block_size):
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    contexts, hkv = [5000, 300, 17], 2
+    blocks = [-(-c // block_size) for c in contexts]
+    tables = torch.zeros(3, max(blocks), dtype=torch.int32)
+    for r, n in enumerate(blocks):
+        tables[r, :n] = torch.arange(n) + sum(blocks[:r])
+    kc, vc = (torch.randn(sum(blocks), block_size, hkv, head_dim, generator=gen,
+                          device="cuda").to(dtype) for _ in range(2))
+    q = torch.randn(3, 4, head_dim, generator=gen, device="cuda").to(dtype)
+    tables, lens = tables.cuda(), torch.tensor(contexts, dtype=torch.int32, device="cuda")
+    heads = vector_heads(q, hkv, block_size)
+    assert (heads is None) == (dtype == torch.bfloat16 and head_dim == 128 and block_size == 16)
+    plan = decode_plan(lens, num_kv_heads=hkv, block_size=block_size,
+                       block_table_width=tables.shape[1], heads=heads)
+    own = hip_paged_decode(q, kc, vc, tables, lens)
+    assert torch.equal(own, hip_paged_decode(q, kc, vc, tables, lens, plan=plan))
 
 
 @pytest.mark.parametrize("context", [1000, 4096, 16384, 32768])
