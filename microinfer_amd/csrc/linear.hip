@@ -15,7 +15,7 @@
 //    its waves split k. A operand: 16 weight rows as stored; B operand: 16
 //    rows of x. All waves then add the partial sums, wave by wave in order,
 //    each wave a share of the tiles.
-//  * gemv_kernel (m <= 4): a wave owns whole weight rows, a lane 8 elements
+//  * gemv_kernel (one or two rows): a wave owns whole weight rows, a lane 8 elements
 //    of every 512, so a load instruction takes 1 KiB of one row; narrow
 //    outputs (1024 columns) then still give all CUs work, where 16-column
 //    tiles leave three quarters of them idle.
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Few rows (m <= 4).
+// One or two rows.
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 4;
 constexpr int kGemvChunk = 8 * kWave;  // elements of a row one load takes
@@ -614,12 +614,17 @@ void launch_gemv(const LinArgs& a, hipStream_t stream) {
 
 // One or two rows take the vector kernel (1024 x 2048: 3.1 / 3.2 us, 3.5 / 3.6
 // on MFMA; 4096 x 1024 3.6, 3.8; the gate/up 6144 x 1024 4.7 / 5.1, 5.2 / 5.3);
-// four take MFMA (3.8 against 3.7, 4.1 against 3.7, 6.6 against 5.3).
+// four take MFMA (3.8 against 3.7, 4.1 against 3.7, 6.6 against 5.3). Two rows
+// of a wide, deep weight too, whose waves wait on six pieces of it and of both
+// rows at once (151936 x 4096: 275 us, 220 on MFMA; 32768 x 4096 63, 51; 151936
+// x 2048 stays: 104, 109; one row 210, 220). By the weight alone, so that all
+// forms of a projection sum alike.
 template <typename E, bool GLU, bool NORM>
 void launch_typed(const LinArgs& a, hipStream_t stream) {
+  const bool deep = a.n >= 32768 && a.k >= 4096;
   if (a.m == 1)
     launch_gemv<E, 1, GLU, NORM>(a, stream);
-  else if (a.m == 2)
+  else if (a.m == 2 && !deep)
     launch_gemv<E, 2, GLU, NORM>(a, stream);
   else
     launch_many_rows<E, GLU, NORM>(a, stream);

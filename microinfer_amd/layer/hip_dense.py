@@ -44,14 +44,18 @@ def prefer_hip_linear(x: torch.Tensor, weight: torch.Tensor) -> bool:
     Measured on MI355X (hipGraph-replayed, the Qwen3-0.6B projections, us per
     launch, HIP against hipBLASLt): at 64 rows QKV 4.5 / 8.5, output 4.3 /
     8.0, gate/up 8.0 / 11.9, down 4.7 / 9.7; at 8 rows 3.7 / 5.9, 3.8 /
-    8.1, 5.3 / 8.0, 4.4 / 9.1. The vocabulary projection (151936 columns)
-    goes to hipBLASLt past 48 rows (1 row 50 / 60, 16 rows 64 / 62, 32 rows
-    70 / 75, 48 rows 77 / 78, 64 rows 104 / 82)."""
+    8.1, 5.3 / 8.0, 4.4 / 9.1. A vocabulary projection (more than 32768
+    columns) goes to hipBLASLt past 32 rows, 40 where k is at most 2048
+    (151936 x 1024 at 1 / 32 / 40 / 48 / 64 rows 52 / 72 / 78.5 / 80 / 107
+    against 62 / 75 / 78.7 / 79 / 83; x 2048 at 32 / 40 / 48 rows 137 / 147 /
+    151 against 149 / 152 / 146; x 4096 at 24 / 32 / 33 / 48 rows 243 / 258 /
+    267 / 281 against 268 / 272 / 258 / 257)."""
     return supported_linear(x, weight) and _measured_faster(x.shape[0], weight)
 
 
 def _measured_faster(rows: int, weight: torch.Tensor) -> bool:
-    return rows <= 48 or weight.shape[0] <= 32768
+    n, k = weight.shape
+    return rows <= (40 if k <= 2048 else 32) or n <= 32768
 
 
 def prefer_hip_rows(rows: int, weight: torch.Tensor) -> bool:

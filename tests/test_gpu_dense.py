@@ -299,3 +299,20 @@ def test_linear_fused_rejects():
     with pytest.raises(ValueError):
         hip_linear_fused(torch.zeros(65, 1024, device=DEV, dtype=torch.bfloat16), w,
                          norm_weight=torch.ones(1024, device=DEV, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 2, 3])
+@pytest.mark.parametrize("n,k", [(32784, 4096), (32768, 4064), (32752, 4096)])
+def test_few_rows_of_a_wide_deep_weight(dtype, m, n, k):
+    """On both sides of the line where two rows go to MFMA."""
+    torch.manual_seed(m)
+    x = torch.randn(m, k, device=DEV).to(dtype)
+    w = (0.05 * torch.randn(n, k, device=DEV)).to(dtype)
+    y = hip_linear(x, w)
+    _assert_close(y, _reference(x, w))
+    assert torch.equal(hip_linear_fused(x, w, residual=y), y + y)
+    if dtype == torch.float16:
+        g = torch.ones(k, device=DEV, dtype=dtype)
+        normed, _ = hip_rms_norm_residual(x, None, g, 1e-6)
+        assert torch.equal(hip_linear_fused(x, w, norm_weight=g, eps=1e-6), hip_linear(normed, w))
