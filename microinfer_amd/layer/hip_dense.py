@@ -84,12 +84,17 @@ def prefer_fused_norm(x: torch.Tensor, weight: torch.Tensor) -> bool:
     inside it: every workgroup then scales the x rows it reads again, which
     past 16 rows and 2048 elements costs more than the norm's own launch (one
     launch against two, us: 24576 x 4096 at 33 rows 67 / 53, at 64 69 / 70;
-    12288 x 2048 at 64 rows 23.2 / 25.7, 4096 x 1024 6.7 / 8.3).
+    12288 x 2048 at 64 rows 23.4 / 26.3, 4096 x 1024 6.7 / 8.3), and with 33
+    to 48 rows where the columns make more workgroups of 32 than there are CUs
+    (at 33 / 48 rows 12288 x 1024 16.1 / 16.6 against 13.3 / 14.2, 16384 x
+    2048 28 / 29 against 24 / 26; 8192 x 2048 15.4 / 15.9 against 18.4 / 19.2).
     float16 rows are normalised before they are scaled, a pass more: worth it
     up to 16 rows (4096 x 1024 at 1 / 16 / 17 / 64 rows 4.2 / 6.1 / 7.8 / 8.6
     against 6.1 / 6.9 / 7.3 / 7.7; 24576 x 4096 at 16 rows 43 against 44)."""
-    narrow = x.shape[1] <= 2048 and x.dtype != torch.float16
-    return prefer_hip_linear(x, weight) and (x.shape[0] <= 16 or narrow)
+    rows, k = x.shape
+    one = (rows <= 16 or (k <= 2048 and x.dtype != torch.float16
+                          and not (32 < rows <= 48 and weight.shape[0] > 8192)))
+    return one and prefer_hip_linear(x, weight)
 
 
 def hip_linear(x: torch.Tensor, weight: torch.Tensor, *,
