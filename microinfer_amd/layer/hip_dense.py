@@ -7,10 +7,10 @@ ops are compiled), the FFN's SwiGLU (``_compiled_swiglu``,
 microinfer/layer/transformer.py:12-15, ``FFN.forward`` :82-88) and every
 projection as ``F.linear``. Each function here is one HIP launch with the
 same result up to float32 summation order; ``supported_*`` tell the caller
-when a request is outside what the kernels take (32-bit tensors, more than
-64 rows for a projection, unaligned rows) and ``prefer_hip_linear`` when the
-HIP projection is measured faster than torch's, so the caller keeps torch for
-the rest.
+when a request is outside what the kernels take (32-bit tensors, unaligned
+rows, more than 64 rows, or 4096 for ``hip_linear_fused`` without a norm) and
+``prefer_*`` when the HIP projection is measured faster than torch's, so the
+caller keeps torch for the rest.
 """
 
 from __future__ import annotations
@@ -68,13 +68,24 @@ def prefer_hip_rows(rows: int, weight: torch.Tensor) -> bool:
 def prefer_hip_prefill(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``hip_linear_fused`` (no norm) beats torch's product past 64 rows.
 
-    Measured (us, HIP against hipBLASLt): 4096 x 1024 at 128 / 256 / 333 / 520
-    rows 5.9 / 8.7 / 9.7 / 14.9 against 9.4 / 9.1 / 10.0 / 13.1; 1024 x 3072 7.0
-    / 7.2 / 10.7 / 15 against 8.1 / 8.9 / 11.9 / 13.8; 6144 x 1024 with the gate
-    8.7 / 10.3 / 16.3 / 18.7 against 13.6 / 16.9 / 17.7 / 18.6 without it. Past
-    about 600 rows, and for larger weights, the library's tiles win. A call
-    also takes half the host time of torch's (9 against 18 us), which bounds
-    eager prefill steps of this size."""
+    Prefill steps are launched eagerly, and a call takes half the host time of
+    torch's (9 against 18 us), so the line follows whole steps of the engine
+    (four chunks, us a step, HIP against hipBLASLt): 1024-wide layers, 28 of
+    them on prefixes of 700, at 128 / 512 / 566 / 640 rows 2964 / 2970 / 3174 /
+    3220 against 4320 / 4340 / 4379 / 4590, 8 of them on prefixes of 4000, where
+    the device bounds the step, 1002 / 1197 / 1344 / 1372 against 1407 / 1413 /
+    1435 / 1466, at 1024 rows 1552 against 1479; 2048-wide layers at 400 / 640
+    rows without a prefix 2023 / 2110 against 2223 / 2188, on prefixes of 2000
+    2137 / 2563 against 2107 / 2469.
+    On the device alone the tiles of up to 512 rows win, the library's past
+    that: 4096 x 1024 at 128 / 333 / 512 / 520 / 640 rows 6.1 / 10.1 / 10.6 /
+    15.5 / 16.1 against 9.6 / 10.2 / 11.0 / 13.4 / 12.0, 1024 x 3072 6.6 / 10.5 /
+    11.7 / 14.9 / 15.6 against 8.2 / 12.0 / 12.3 / 13.9 / 13.9, 6144 x 1024 with
+    the gate 9.3 / 16.8 / 16.9 / 18.8 / 19.0 against 12.7 / 17.9 / 18.8 / 19.2 /
+    19.8; weights of 2^23 elements from about 256 rows on (4096 x 2048 at 192 /
+    333 / 640 rows 12.4 / 15.5 / 25.7 against 16.4 / 13.8 / 21.7). Larger ones
+    are the library's: 6144 x 2048 at 128 / 333 / 640 rows 15.8 / 28.7 / 36.5
+    against 15.6 / 24.9 / 25.8."""
     return (x.shape[0] <= 640 and weight.shape[0] * weight.shape[1] <= 1 << 23
             and supported_linear(x, weight, FUSED_MAX_ROWS))
 
@@ -154,9 +165,9 @@ def hip_linear_fused(x: torch.Tensor, weight: torch.Tensor, *,
     _lib.require_device(x, weight, norm_weight, residual, what="fused projection")
     limit = FUSED_MAX_ROWS if norm_weight is None else LINEAR_MAX_ROWS
     if not supported_linear(x, weight, limit) or (swiglu and weight.shape[0] % 32):
-        raise ValueError("hip_linear_fused: x [m <= 4096 (64 with a norm), k] and weight [n % 16 == 0, k % 32 == 0] "
-                         "(gate/up: n % 32 == 0) of one 16-bit dtype with 16-byte aligned rows "
-                         "are required")
+        raise ValueError("hip_linear_fused: x [m <= 4096 (64 with a norm), k] and weight "
+                         "[n % 16 == 0, k % 32 == 0] (gate/up: n % 32 == 0) of one 16-bit dtype "
+                         "with 16-byte aligned rows are required")
     m, k = x.shape
     n = weight.shape[0]
     width = n // 2 if swiglu else n
