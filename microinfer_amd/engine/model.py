@@ -35,7 +35,8 @@ from microinfer_amd.layer.hip_dense import (LINEAR_MAX_ROWS, hip_linear, hip_lin
                                             hip_linear_swiglu, hip_rms_norm_residual,
                                             hip_silu_mul, prefer_fused_norm, prefer_hip_linear,
                                             prefer_hip_prefill, prefer_hip_rows, supported_rows)
-from microinfer_amd.layer.hip_paged_attention import hip_qkv_decode, supported_qkv_decode
+from microinfer_amd.layer.hip_paged_attention import (hip_qkv_decode, prefer_qkv_decode,
+                                                      supported_qkv_decode)
 from microinfer_amd.layer.hip_qk_norm_rope import qk_norm_rope_append, rope_tables
 from microinfer_amd.layer.paged_attention import paged_attention_meta, varlen_attention
 
@@ -151,7 +152,8 @@ class Qwen3Model:
         """Whether this layer's projections take its norms, gate and residual
         sums along: the HIP projections are preferred for all four."""
         rows = hidden.shape[0]
-        return (self.hip_dense and 0 < rows <= LINEAR_MAX_ROWS and supported_rows(hidden) and layer.gate_up.shape[0] % 32 == 0
+        return (self.hip_dense and 0 < rows <= LINEAR_MAX_ROWS and supported_rows(hidden)
+                and layer.gate_up.shape[0] % 32 == 0
                 and all(w.dtype == hidden.dtype and prefer_hip_rows(rows, w)
                         for w in (layer.qkv, layer.out, layer.gate_up, layer.down)))
 
@@ -160,7 +162,8 @@ class Qwen3Model:
         c = self.config
         tokens = qkv.shape[0]
         if (metadata.is_decode and metadata.slots_at_end
-                and supported_qkv_decode(qkv, cache.keys, cache.values, c.num_q_head)):
+                and supported_qkv_decode(qkv, cache.keys, cache.values, c.num_q_head)
+                and prefer_qkv_decode(qkv, cache.keys, metadata.block_tables)):
             attn = hip_qkv_decode(
                 qkv, cache.keys, cache.values, metadata.block_tables, metadata.context_lens,
                 metadata.slot_mapping, positions, q_weight=layer.q_norm, k_weight=layer.k_norm,

@@ -274,6 +274,21 @@ def supported_qkv_decode(qkv: torch.Tensor, key_cache: torch.Tensor, value_cache
             and key_cache.stride(-1) == 1 and 0 < qkv.shape[0] <= 4096 and aligned)
 
 
+def prefer_qkv_decode(qkv: torch.Tensor, key_cache: torch.Tensor,
+                      block_tables: torch.Tensor) -> bool:
+    """Whether ``hip_qkv_decode`` is the faster of it and the two launches: not
+    for many short sequences, whose workgroups outnumber four a CU and each
+    norm their rows with little to stream behind it (8 KV heads, one launch
+    against two, us: 128 sequences of 64 / 200 tokens 18.3 / 30.4 against 18.9
+    / 32.6; 160 of 64 / 200 22.8 / 37.8, 21.9 / 39.1; 256 of 64 / 200 / 300 /
+    500 34.7 / 53.9 / 70.7 / 106, 31.5 / 54.0 / 70.7 / 108; 1024 of 64 / 128 /
+    300 140 / 168 / 279, 124 / 160 / 278). The contexts are on the device: the
+    tables' width bounds them."""
+    _, block_size, num_kv_heads, _ = key_cache.shape
+    return (block_tables.shape[1] * block_size > 256
+            or qkv.shape[0] * num_kv_heads <= 4 * _device_cus(qkv.device))
+
+
 def hip_qkv_decode(
     qkv: torch.Tensor,
     key_cache: torch.Tensor,

@@ -113,3 +113,26 @@ def test_rejects():
     with pytest.raises(ValueError):
         hip_qkv_decode(qkv[:, :512], cache.keys, cache.values, tables, lens, slots, positions,
                        num_q_heads=16, **args)
+
+
+@pytest.mark.parametrize("seqs,context", [(128, 40), (129, 40), (129, 300)])
+def test_model_attends_alike_on_both_routes(seqs, context):
+    """Both sides of the line by sequences and table width, through the model's
+    own choice, against the two launches."""
+    from types import SimpleNamespace
+
+    from microinfer_amd.engine.model import QwenConfig, Qwen3Model
+    from microinfer_amd.layer.metadata import AttentionMetadata
+
+    contexts = [1 + (37 * i) % context for i in range(seqs - 1)] + [context]
+    case = _case(contexts, 16, 8, 16, torch.bfloat16, "paired")
+    qkv, tables, lens, slots, positions, args, (_, cache) = case
+    want = _two_launches(case, 16, 8, False)
+    metadata = AttentionMetadata.build(is_prefill=False, slot_mapping=slots, context_lens=lens,
+                                       block_tables=tables, validate_cache_write=False)
+    metadata.slots_at_end = True
+    model = Qwen3Model.__new__(Qwen3Model)
+    model.config, model.cos, model.sin = QwenConfig(), args["cos_table"], args["sin_table"]
+    layer = SimpleNamespace(q_norm=args["q_weight"], k_norm=args["k_weight"])
+    got = model._attend(layer, cache, qkv[:, :32 * D].contiguous(), positions, metadata)
+    _assert_same(case, want, got.view_as(want), torch.bfloat16)
