@@ -578,7 +578,9 @@ template <typename E, bool GLU, bool NORM>
 void launch_many_rows(const LinArgs& a, hipStream_t stream) {
   // Narrow outputs: eight waves per tile (1024 x 3072 at 8 rows: 4.35 us, 4.68
   // with four); wider ones have workgroups enough (4096 x 1024: 3.9, 3.7 with
-  // four). By n alone, so that the fused gate sums as the projection does.
+  // four). By n alone, so that up to 64 rows the fused gate sums as the
+  // projection does (past them the tiles split k at other places, unless it is
+  // a multiple of 512).
   const bool eight = a.n < 4096 && a.m <= kLinMaxRows;
   const LinTile t = pick_tile(a, GLU, eight);
   if constexpr (!GLU) {

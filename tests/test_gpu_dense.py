@@ -221,7 +221,7 @@ def test_linear_fused_is_norm_projection_and_sum(dtype, m, n, k):
     assert bool(((got - y).abs() <= 4 * spread + unit * y.abs() + 1e-6).all())
     if n % 32 == 0:
         fused = hip_linear_fused(x, w, swiglu=True)
-        assert torch.equal(fused, hip_linear_swiglu(x, w))
+        assert torch.equal(fused, hip_silu_mul(hip_linear(x, w)))
         gate, up = y.chunk(2, dim=-1)
         e_gate, e_up = (4 * spread + unit * y.abs() + 1e-6).chunk(2, dim=-1)
         want = F.silu(gate) * up
@@ -281,10 +281,17 @@ def test_linear_fused_past_64_rows(dtype, m, n, k):
     _assert_close(y, _reference(x, w))
     assert torch.equal(hip_linear_fused(x, w, residual=r), r + y)
     if n % 32 == 0:
-        gate, up = _reference(x, w).chunk(2, dim=-1)
-        ref = F.silu(gate) * up
-        err = (hip_linear_fused(x, w, swiglu=True).float() - ref).abs()
-        assert bool((err <= 2.5e-2 * ref.abs() + 2e-3 * ref.abs().max() + 1e-6).all())
+        # The gate of the projection: the same sums where every tile shape
+        # splits k alike (multiples of 512); else gate and up may each round to
+        # the next value (|silu'| <= 1.1), and so the gate and the product.
+        gated, want = hip_linear_fused(x, w, swiglu=True), hip_silu_mul(y)
+        if k % 512 == 0:
+            assert torch.equal(gated, want)
+        else:
+            gate, up = (t.float() for t in y.chunk(2, dim=-1))
+            unit = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+            bound = unit * (1.1 * gate.abs() * up.abs() + 4 * want.float().abs())
+            assert bool(((gated.float() - want.float()).abs() <= bound + 1e-6).all())
 
 
 def test_linear_fused_rejects():
