@@ -63,11 +63,11 @@ int32_t mi_linear_swiglu(const void* x, int64_t x_row_stride, const void* w,
  * made): for float16 the row is normalised as mi_rms_norm_residual does it,
  * and the result is that call's and mi_linear's (mi_linear_swiglu's) bit for
  * bit; for bf16 it is applied as (1 / rms) * ((x * norm_weight rounded once)
- * . w^T), which lacks that pair's second rounding. The projection's sum is rounded to the element type before the
- * residual is added and the result rounded again, as x + F.linear(...) does;
- * residual may be NULL and may be y itself. norm_weight may be NULL: then m may
- * be up to 4096. Shapes, alignment and other limits are those of mi_linear /
- * mi_linear_swiglu.
+ * . w^T), which lacks that pair's second rounding. The projection's sum is
+ * rounded to the element type before the residual is added and the result
+ * rounded again, as x + F.linear(...) does; residual may be NULL and may be y
+ * itself. norm_weight may be NULL: then m may be up to 4096. Shapes, alignment
+ * and other limits are those of mi_linear / mi_linear_swiglu.
  */
 int32_t mi_linear_fused(const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
                         const void* w, int64_t w_row_stride, const void* residual,

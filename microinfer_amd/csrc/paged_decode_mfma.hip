@@ -283,8 +283,8 @@ __global__ __launch_bounds__(kWave * NW) void paged_decode_mfma_kernel(const Arg
       const bool is_k = r == G;
       if (is_k && !append) continue;
       norm_rope_row<E>(a.qkv, row + (is_k ? a.num_kv_heads * G + head : head * G + r) * kD,
-                       static_cast<const R*>(is_k ? a.qkv.k_weight : a.qkv.q_weight), ctx - 1, pos_true,
-                       lane, s_q + (is_k ? kHeads : r) * kD);
+                       static_cast<const R*>(is_k ? a.qkv.k_weight : a.qkv.q_weight), ctx - 1,
+                       pos_true, lane, s_q + (is_k ? kHeads : r) * kD);
     }
     if (owner) {
       const int slot = pos_true >= 0 && pos_true < a.qkv.table_len ? a.qkv.slots[seq] : -1;

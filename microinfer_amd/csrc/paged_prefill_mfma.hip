@@ -27,7 +27,7 @@
 //    three workgroups (12 waves) share a CU.
 //  * Per tile and wave the scalar work is one block-id load, a multiply-add
 //    for the block's offset (the scalar offset of buffer loads from the
-//    head's K and V bases) and three M0 writes.
+//    head's K and V bases) and two M0 writes.
 #include "paged_attention.h"
 
 namespace mi {
@@ -756,7 +756,8 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
   // scores, issue tile t + 2 into the buffer tile t - 1 used, finish tile t.
   // The loop sits inside the prologue's branch so that every path into it
   // has passed the prologue (the compiler's wait insertion is static).
-  auto wait_tile = [&](bool next_in_flight, int tile, int tmask, R* vbuf) __attribute__((always_inline)) {
+  auto wait_tile = [&](bool next_in_flight, int tile, int tmask,
+                       R* vbuf) __attribute__((always_inline)) {
     // vmcnt(4) leaves the next tile's four loads in flight; vmcnt(0) waits
     // for everything (s_waitcnt encoding: vmcnt in bits 3:0, expcnt 6:4 = 7
     // (no wait), lgkmcnt 11:8).
@@ -908,8 +909,9 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
       for (int p = 0; p < kMaxParts; ++p) {
         f[p] = weight(f[p], mx);
         if (p < nparts)
-          lsum = fmaf(f[p], p == part ? l : load_coherent(a.ws_ml + (region(p) * kWave + lane) * 2 + 1),
-                      lsum);
+          lsum = fmaf(
+              f[p], p == part ? l : load_coherent(a.ws_ml + (region(p) * kWave + lane) * 2 + 1),
+              lsum);
       }
 #pragma unroll
       for (int db = 0; db < kD / 32; ++db) {

@@ -15,8 +15,9 @@ Same positional/keyword arguments, same ValueError checks (:280-302,
   ``context_lens`` (the reference picks 4 or 1 on the host from R*Hq); an int
   forces at most that many partitions per sequence. The launch shape depends
   only on the batch size, so hipGraph capture stays valid as contexts grow.
-* Prefill also accepts float32 (vector kernel) and contiguous varlen K/V
-  (``block_tables=None``), which serves the no-prefix prefill.
+* Prefill also accepts float32 (float32 MFMA with head_dim 128, else and for
+  few rows the vector kernel) and contiguous varlen K/V (``block_tables=None``),
+  which serves the no-prefix prefill.
 
 Workspace comes from torch's caching allocator (the graph pool under
 capture); the library never allocates.

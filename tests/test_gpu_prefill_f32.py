@@ -108,10 +108,11 @@ def _exact(q, kc, vc, tables, contexts, cu_q):
 
 def test_error_against_64_bits_is_the_vector_kernels():
     """On the same rows: blocks of 8 take the vector kernel. The ratio of the
-    two errors is about 0.98 in the mean; summation chains of 16 terms and a
-    second rounding of the scaled scores made it 1.06 here."""
+    two errors is about 1 in the mean; longer summation chains and a second
+    rounding of the scaled scores made it 1.06 here."""
     log_ratio = 0.0
-    cases = [([200, 90], [100, 0]), ([64] * 4, [0, 30, 300, 7]), ([400], [300]), ([300, 25], [0, 9])]
+    cases = [([200, 90], [100, 0]), ([64] * 4, [0, 30, 300, 7]), ([400], [300]),
+             ([300, 25], [0, 9])]
     for seed, (q_lens, prefixes) in enumerate(cases):
         q, kc, vc, tables, contexts, cu_q, cu_k = _paged_case(q_lens, prefixes, 16, 8, 16,
                                                               torch.float32, seed)
