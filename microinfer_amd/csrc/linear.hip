@@ -178,9 +178,9 @@ __device__ __forceinline__ uint16_t add_residual(uint16_t y, uint16_t res) {
 // A wave stages its chunks of w and x in its own LDS slots with direct
 // global->LDS loads, 1 KiB of whole chunk rows per instruction, and reads the
 // MFMA fragments from there. Loading the fragments straight into registers
-// puts 16 different rows in 16 neighbouring lanes, and the address unit then
-// takes about 64 cycles per instruction instead of 16: at 64 rows that alone
-// was 4.1 of the 7.1 us of a 4096 x 1024 projection.
+// puts 16 different rows in 16 neighbouring lanes: the address unit was then
+// busy 69 cycles per vector memory instruction, 31 as it is (TA_TA_BUSY /
+// SQ_INSTS_VMEM of the 4096 x 1024 projection at 64 rows, 8.0 and 4.5 us).
 // 16-byte piece c of row r sits at place c ^ swz(r): with rows of 256 bytes
 // (KC 128) swz = r & 15, of 128 bytes (KC 64, two rows to a bank cycle)
 // (r >> 1) & 7, either of which leaves a fragment read (16 rows, one piece)
