@@ -264,9 +264,11 @@ int32_t mi_paged_decode_qkv(
  * Replaces triton_paged_prefill + _paged_prefill_kernel
  * (microinfer/layer/triton_paged_attention.py:260-339, :134-233) and the
  * reference-path fallback of paged_attention_meta (paged_attention.py:277-293).
- * bf16/f16 with head_dim 128 run on the MFMA kernel; every other supported
- * shape (including f32) runs on the vector kernel. max_seqlen_q bounds the
- * query rows of any request (launch shape only).
+ * bf16/f16 with head_dim 128 and Hq/Hkv 1, 2 or 4 run on the MFMA kernel, f32
+ * with head_dim 128 (contiguous K/V or blocks of at least 16) on the float32
+ * MFMA unless the rows are few; every other supported shape runs on the vector
+ * kernel (Hq/Hkv up to 8). max_seqlen_q bounds the query rows of any request
+ * (launch shape only).
  *
  * block_tables == NULL selects contiguous varlen K/V instead of a paged cache:
  * key_cache/value_cache are [sum c_r, Hkv, D] arrays (token stride
