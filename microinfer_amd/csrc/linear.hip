@@ -60,9 +60,6 @@ struct LinMfma<F16> {
 
 constexpr int kLinMaxRows = 64;
 constexpr int kLinMaxFusedRows = 4096;  // mi_linear_fused without a norm
-// s_waitcnt immediate that waits for vmcnt <= n only (vmcnt bits 3:0 and
-// 15:14, the other counters at their maxima).
-constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kLinStep = 32;  // k per MFMA
 
 struct LinArgs {

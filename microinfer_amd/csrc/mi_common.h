@@ -132,6 +132,10 @@ __device__ __forceinline__ void lds_load16_sbase(const void* base, uint32_t byte
                : "memory", "m0");
 }
 
+// s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding: vmcnt
+// bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
+constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+
 template <typename R, int N>
 __device__ __forceinline__ Pack<R, N> zero_pack() {
   Pack<R, N> z;
@@ -193,6 +197,21 @@ __device__ __forceinline__ float xor_max(float v) {
 #pragma unroll
   for (int o = FROM; o < TO; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
   return v;
+}
+
+// The value held by lane ^ 16 / lane ^ 32, with v_permlane16/32_swap (VALU ops,
+// no LDS round trip). The instruction swaps the upper half of its first operand
+// (of 32 or 64 lanes) with the lower half of its second: lower lanes find their
+// partner in the second result, upper lanes in the first.
+__device__ __forceinline__ float lane_xor16(float v, int lane) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
+}
+__device__ __forceinline__ float lane_xor32(float v, int lane) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, lane < 32 ? r[1] : r[0]);
 }
 
 // DPP lane move within a 16-lane row (bound_ctrl off: every source used here

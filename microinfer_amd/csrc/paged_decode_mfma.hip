@@ -92,9 +92,6 @@ constexpr int kSlotBytes = 2 * kHalfBytes;        // K then V
 constexpr int kLoadsPerHalf = kHalfBytes / kLoadBytes;  // 4
 constexpr int kLoadsPerTile = 2 * kLoadsPerHalf;        // 8
 constexpr int kRescaleSlack = 15;
-// s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding: vmcnt
-// bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
-constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 static_assert(3 * kLoadsPerTile <= 63, "vmcnt immediate");
 
 // LDS tile rows are 256 bytes; the 16-byte chunk c of row r sits at chunk
@@ -103,18 +100,6 @@ static_assert(3 * kLoadsPerTile <= 63, "vmcnt immediate");
 // rows r..r+7, two adjacent chunks each) with swz_v(r) = 2 (r & 7).
 __device__ __forceinline__ int swz_k(int r) { return r & 15; }
 __device__ __forceinline__ int swz_v(int r) { return 2 * (r & 7); }
-
-// The value held by lane ^ 16 / lane ^ 32 (v_permlane16/32_swap).
-__device__ __forceinline__ float lane_xor16(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
-}
-__device__ __forceinline__ float lane_xor32(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, lane < 32 ? r[1] : r[0]);
-}
 
 // One step of the running split merge: fold partial (mb, lb, ob) into
 // (mx, ls, os) in the log2 domain; an empty partial (mb = -inf) weighs zero.

@@ -46,18 +46,6 @@ constexpr int kRows = 16;  // query rows per workgroup, keys per tile
 constexpr int kOutStride = kD + 4;  // LDS row of a wave's sums: 16 rows hit 16 bank groups
 constexpr float kSlack = 8.f;  // the running maximum may lag by 2^8
 
-// The value held by lane ^ 16 / lane ^ 32.
-__device__ __forceinline__ float swap16(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
-}
-__device__ __forceinline__ float swap32(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, lane < 32 ? r[1] : r[0]);
-}
-
 template <int NW, bool PAGED>
 __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(16))) float s_o[NW][kRows * kOutStride];
@@ -212,8 +200,8 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
       if (p0 + 4 * quad + i >= lim) s[i] = -INFINITY;
       tmax = fmaxf(tmax, s[i] * a.scale_log2);
     }
-    tmax = fmaxf(tmax, swap16(tmax, lane));
-    tmax = fmaxf(tmax, swap32(tmax, lane));
+    tmax = fmaxf(tmax, lane_xor16(tmax, lane));
+    tmax = fmaxf(tmax, lane_xor32(tmax, lane));
     if (__ballot(tmax > m + kSlack) != 0) {
       const float mnew = fmaxf(m, tmax);
       const float alpha = mnew == -INFINITY ? 1.f : fast_exp2(m - mnew);
@@ -310,8 +298,8 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_prefill_f32_kernel(const 
   }
 
   // Merge the waves. o[4 j + e][i] is dim 64 j + 16 quad + 4 i + e of row `col`.
-  l += swap16(l, lane);
-  l += swap32(l, lane);
+  l += lane_xor16(l, lane);
+  l += lane_xor32(l, lane);
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll

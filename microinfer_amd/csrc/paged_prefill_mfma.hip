@@ -48,16 +48,6 @@ __device__ __forceinline__ uint16_t to_raw(float x) {
   }
 }
 
-// The value held by lane ^ 32 (the other half of a query row's keys), with
-// v_permlane32_swap (a VALU op; no LDS round trip). The instruction swaps the
-// upper half of its first operand with the lower half of its second: lanes
-// 0-31 find their partner in the second result, lanes 32-63 in the first.
-__device__ __forceinline__ float partner32(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, lane < 32 ? r[1] : r[0]);
-}
-
 // Two packed 1.0 values of the element type (for row sums with dot2).
 template <typename E>
 constexpr uint32_t kOnes2 = std::is_same<E, BF16>::value ? 0x3F803F80u : 0x3C003C00u;
@@ -210,12 +200,6 @@ static_assert(kWaves * kRowSlot <= 2 * 3 * kTileElems * 2, "slots fit the tile r
 __device__ __forceinline__ int row_swz_k(int r) { return r & 15; }
 __device__ __forceinline__ int row_swz_v(int r) { return 2 * (r & 7); }
 
-__device__ __forceinline__ float lane_xor16(float v, int lane) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (lane & 16) ? r[0] : r[1]);
-}
-
 // Attention of request `req`'s single query row (row `q_row`) over its `ctx`
 // paged keys for KV head `head`, all G query heads, written to the output.
 // `slots`: kWaves x kRowSlot bytes of LDS; s_m / s_l: [kWaves][16] floats.
@@ -330,7 +314,7 @@ __device__ __forceinline__ void single_row_attention(const AttnArgs& a, int req,
       tmax = fmaxf(tmax, sc[i]);
     }
     tmax = fmaxf(tmax, lane_xor16(tmax, lane));
-    tmax = fmaxf(tmax, partner32(tmax, lane));
+    tmax = fmaxf(tmax, lane_xor32(tmax, lane));
     if (__ballot(col < G && tmax > m + kRescaleSlack) != 0) {
       const float mnew = fmaxf(m, tmax);
       const float alpha = (mnew == -INFINITY) ? 1.f : fast_exp2(m - mnew);
@@ -359,7 +343,7 @@ __device__ __forceinline__ void single_row_attention(const AttnArgs& a, int req,
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   // Per-head row sum over the four position groups.
   l += lane_xor16(l, lane);
-  l += partner32(l, lane);
+  l += lane_xor32(l, lane);
   // Wave states to LDS: acc[h][d] floats in the wave's own (drained) slot.
   float* my_acc = reinterpret_cast<float*>(slot);
   if (col < G) {
@@ -703,7 +687,7 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
     // exponents stay below 2^kRescaleSlack and the normalisation by l at the
     // end is unchanged.
     if (__ballot(smax > thr) != 0) {
-      const float rmax = fmaxf(smax, partner32(smax, lane)) * scale_log2;
+      const float rmax = fmaxf(smax, lane_xor32(smax, lane)) * scale_log2;
       const float mnew = fmaxf(m, rmax);
       const float alpha = (mnew == -INFINITY) ? 1.f : fast_exp2(m - mnew);
       l *= alpha;
@@ -950,7 +934,7 @@ __global__ __launch_bounds__(kThreads, 3) void paged_prefill_mfma_kernel(const A
   }
   // The row's sum: both halves add (lane l & 31) + (lane l | 32).
   {
-    const float other = partner32(l, lane);
+    const float other = lane_xor32(l, lane);
     l = lane < 32 ? l + other : other + l;
   }
   if (!row_ok) return;
