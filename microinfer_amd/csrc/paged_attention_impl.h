@@ -160,10 +160,10 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_attention_vector_kernel(c
   // request's row, or an unused one, may hold NaN).
   const int64_t head_off = head * a.c_hs + row0 * a.c_ts;
   int64_t safe_head_off = head * a.c_hs;
-  if (paged) {
+  if (paged && a.t_width > 0) {
     const int blk = trow[max(min(blk_begin, a.t_width - 1), 0)];
     if (blk > 0 && blk < a.num_blocks) safe_head_off += blk * a.c_bs;
-  } else if (row0 > 0 && row0 < a.num_blocks) {
+  } else if (!paged && row0 > 0 && row0 < a.num_blocks) {
     safe_head_off += row0 * a.c_ts;
   }
   const int lane_off = grp * static_cast<int>(a.c_ts) + d0;
