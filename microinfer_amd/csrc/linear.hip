@@ -103,7 +103,7 @@ __device__ __forceinline__ Pack<uint16_t, 8> norm8(const Pack<uint16_t, 8>& x, f
   Pack<uint16_t, 8> r;
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    r.v[i] = E::store(E::load(E::store(E::load(x.v[i]) * inv)) * E::load(w.v[i]));
+    r.v[i] = norm_round<E>(x.v[i], inv, w.v[i]);
   return r;
 }
 

@@ -74,6 +74,17 @@ __device__ __forceinline__ uint16_t silu_mul_round(uint16_t g, uint16_t u) {
   return E::store(act * E::load(u));
 }
 
+// round(round(x * inv) * w): the rounding steps of torch's rms_norm on 16-bit
+// inputs. The first product rounds to float32 on the way; the fused
+// multiply-convert that the compiler may form for float16 would not, and differs
+// once in some 10^4 elements, so it is kept from seeing the pair.
+template <typename E>
+__device__ __forceinline__ uint16_t norm_round(uint16_t x, float inv, uint16_t w) {
+  float n = E::load(x) * inv;
+  asm("" : "+v"(n));
+  return E::store(E::load(E::store(n)) * E::load(w));
+}
+
 // N consecutive raw elements moved with one load/store instruction.
 template <typename R, int N>
 struct alignas(sizeof(R) * N) Pack {

@@ -80,10 +80,7 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void rms_norm_residual_kerne
     if (c < chunks) {
       Pack<R, 8> o;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float n = E::load(E::store(E::load(s[i].v[j]) * inv));
-        o.v[j] = E::store(n * E::load(w[i].v[j]));
-      }
+      for (int j = 0; j < 8; ++j) o.v[j] = norm_round<E>(s[i].v[j], inv, w[i].v[j]);
       store_pack<R, 8>(out + c * 8, o);
     }
   }

@@ -269,6 +269,19 @@ def test_norm_inside_over_the_range_of_the_type(dtype, m, n, k):
                                hip_linear_swiglu(normed, w))
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 17])
+def test_norm_inside_rounds_as_its_launch(m):
+    """Enough elements (160 x 1024 a row) that one rounding less in the
+    normalised row would show."""
+    torch.manual_seed(m)
+    w = (0.05 * torch.randn(48, 1024, device=DEV)).half()
+    for scale in torch.logspace(-1, 1, 160).tolist():
+        x = (scale * torch.randn(m, 1024, device=DEV)).half()
+        g = (1 + 0.3 * torch.randn(1024, device=DEV)).half()
+        normed, _ = hip_rms_norm_residual(x, None, g, 1e-6)
+        assert torch.equal(hip_linear_fused(x, w, norm_weight=g, eps=1e-6), hip_linear(normed, w))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m", [65, 128, 200, 333, 641])
 @pytest.mark.parametrize("n,k", [(4096, 1024), (1024, 3072), (6144, 1024), (48, 64), (2080, 160)])
