@@ -266,12 +266,15 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
     return *reinterpret_cast<const Pack<R, 8>*>(tile + col * kRowBytes +
                                                 (((4 * step + quad) ^ swz(col)) * 16));
   };
+  auto issue_first = [&]() {
 #pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (c_begin + s < c_end) issue(s, c_begin + s);
+    for (int s = 0; s < S; ++s)
+      if (c_begin + s < c_end) issue(s, c_begin + s);
+  };
   const R* nrow = static_cast<const R*>(a.norm) + quad * 8;
   [[maybe_unused]] float inv[MT];
   if constexpr (kFirst) {
+    issue_first();
     constexpr int kRows = MT * 16 / NW;
     const R* row[kRows];
     float row_inv[kRows];
@@ -288,6 +291,7 @@ __global__ __launch_bounds__(NW* kWave) void linear_kernel(const LinArgs a) {
     for (int t = 0; t < MT; ++t) inv[t] = s_ss[0][16 * t + col];
   }
   if (c_begin < c_end) {
+    if constexpr (!kFirst) issue_first();
     for (int c = c_begin, slot = 0; c < c_end; ++c, slot = slot + 1 == S ? 0 : slot + 1) {
       Pack<R, 8> g[NORM ? kChunkSteps : 1];
       if constexpr (NORM) {

@@ -81,7 +81,7 @@ __device__ __forceinline__ uint16_t silu_mul_round(uint16_t g, uint16_t u) {
 template <typename E>
 __device__ __forceinline__ uint16_t norm_round(uint16_t x, float inv, uint16_t w) {
   float n = E::load(x) * inv;
-  asm("" : "+v"(n));
+  if constexpr (std::is_same<E, F16>::value) asm("" : "+v"(n));
   return E::store(E::load(E::store(n)) * E::load(w));
 }
 

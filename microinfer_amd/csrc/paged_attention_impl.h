@@ -161,7 +161,8 @@ __global__ __launch_bounds__(kWave * NW, 2) void paged_attention_vector_kernel(c
   const int64_t head_off = head * a.c_hs + row0 * a.c_ts;
   int64_t safe_head_off = head * a.c_hs;
   if (paged && a.t_width > 0) {
-    const int blk = trow[max(min(blk_begin, a.t_width - 1), 0)];
+    using ConstI32 = __attribute__((address_space(4))) const int32_t;
+    const int blk = ((ConstI32*)(trow))[max(min(blk_begin, a.t_width - 1), 0)];  // scalar load
     if (blk > 0 && blk < a.num_blocks) safe_head_off += blk * a.c_bs;
   } else if (!paged && row0 > 0 && row0 < a.num_blocks) {
     safe_head_off += row0 * a.c_ts;
